@@ -476,8 +476,9 @@ def main():
                     frac=achieved / PEAK_FP64_TFLOPS,
                     traffic=TRAFFIC_BYTES_PER_LAUNCH if args.variant in ("auto", "ws") else None,
                     traffic_source=TRAFFIC_SOURCE if args.variant in ("auto", "ws") else None,
-                    kernel={"lane": "sweep2_lane_kernel<LCAO2>",
-                            "quad": "sweep2_quad_kernel<LCAO2,2>"}.get(args.variant, "sweep2_ws_kernel<LCAO2,2,6>"),
+                    kernel={"lane": "sweep2_wide_kernel<LCAO2,2>",
+                            "quad": "sweep2_ws_kernel<LCAO2,2,4,2,0,4>"}.get(args.variant,
+                                                                            "sweep2_ws_kernel<LCAO2,2,2,2,1,4>"),
                     kernel_ms=1e3 * avg_kernel_s,
                     flop_per_launch=fl)
     cpu = None

@@ -520,14 +520,14 @@ mole_status mole_dmc_read_walkers(mole_ctx *ctx, uint32_t sys, double *weights, 
 
 /* ---- launch configuration ----------------------------------------------
  * No counterpart in the reference (rayon's fan-out, src/vmc/src/vmc.rs:63-76,
- * is the closest).  Selects the two-electron sweep kernel: AUTO picks
- * WAVESPEC where it applies (He, or LCAO with at most 2 nuclei); WAVESPEC
- * gives each 64 walkers a workgroup of four specialised waves (chain, two
- * draw producers, sampler); QUAD spreads each walker over four lanes of a
- * wave (same eligibility);
- * LANE runs one lane per walker with block_threads threads per workgroup
- * (0 keeps the current value).  Every variant produces bit-identical walker
- * trajectories. */
+ * is the closest).  Selects the two-electron sweep kernel.  WAVESPEC and QUAD
+ * (He, or LCAO with at most 2 nuclei) give the Metropolis chain, the draws and
+ * the sampling of a workgroup's walkers waves of their own, with two (WAVESPEC,
+ * 64 walkers per workgroup) or four (QUAD, 32) lanes per walker in the chain;
+ * LANE runs one lane per walker with block_threads threads per workgroup (0
+ * keeps the current value).  AUTO picks by walkers per compute unit: QUAD up
+ * to 32, WAVESPEC up to 128, LANE beyond and for more nuclei.  Every variant
+ * produces bit-identical walker trajectories. */
 #define MOLE_VARIANT_AUTO 0
 #define MOLE_VARIANT_LANE 1
 #define MOLE_VARIANT_WAVESPEC 2

@@ -83,6 +83,7 @@ DEBUG_COSPI = 8
 DEBUG_BOXMULLER0 = 9
 DEBUG_BOXMULLER1 = 10
 DEBUG_BF16 = 11
+DEBUG_SQRT_NORMAL = 12
 
 
 class MoleError(RuntimeError):

@@ -616,7 +616,7 @@ mole_status enqueue_sweeps(mole_ctx *ctx, uint32_t n, uint32_t sample_start, uin
         a.trace_sample0 = ctx->trace_samples;
         a.cap_sweeps = (st.d_trace_mask) ? ctx->run.record_sweeps : 0;
         a.cap_samples = (st.d_trace_e || st.d_samp_psi) ? ctx->run.record_sweeps : 0;
-        HIP_TRY(launch_sweep2(a, ctx->variant, ctx->block_threads, ctx->stream));
+        HIP_TRY(launch_sweep2(a, ctx->variant, ctx->block_threads, ctx->cu_count, ctx->stream));
         ++launches;
       }
     }

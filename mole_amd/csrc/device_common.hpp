@@ -22,6 +22,11 @@ struct u32x4 {
   uint32_t x, y, z, w;
 };
 
+// a ^ b ^ c in one instruction (v_bitop3_b32, truth table 0x96)
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+}
+
 __device__ __forceinline__ u32x4 philox4x32_10(u32x4 c, uint32_t k0,
                                                uint32_t k1) {
 #pragma unroll
@@ -33,9 +38,9 @@ __device__ __forceinline__ u32x4 philox4x32_10(u32x4 c, uint32_t k0,
     const uint64_t p0 = (uint64_t)kPhiloxM0 * c.x;
     const uint64_t p1 = (uint64_t)kPhiloxM1 * c.z;
     u32x4 n;
-    n.x = (uint32_t)(p1 >> 32) ^ c.y ^ k0;
+    n.x = xor3((uint32_t)(p1 >> 32), c.y, k0);
     n.y = (uint32_t)p1;
-    n.z = (uint32_t)(p0 >> 32) ^ c.w ^ k1;
+    n.z = xor3((uint32_t)(p0 >> 32), c.w, k1);
     n.w = (uint32_t)p0;
     c = n;
   }
@@ -87,42 +92,65 @@ __device__ __forceinline__ double u64_range(uint64_t x, double scale,
 }
 
 // exp(x): Cody-Waite reduction with the fdlibm split of ln2, degree-13
-// Taylor polynomial by Horner with fma, two exact power-of-two scalings.
-__device__ __forceinline__ double exp_m(double x) {
-  const double kLn2Hi = 6.93147180369123816490e-01;
-  const double kLn2Lo = 1.90821492927058770002e-10;
-  const double kInvLn2 = 1.44269504088896338700e+00;
-  const double kOvf = 709.782712893383973096;
-  const double kUnf = -745.133219101941108420;
-  const double xc = fmin(fmax(x, kUnf), kOvf);
-  const double kd = rint(xc * kInvLn2);
-  double r = fma(-kd, kLn2Hi, xc);
-  r = fma(-kd, kLn2Lo, r);
-  double p = 1.0 / 6227020800.0;
-  p = fma(p, r, 1.0 / 479001600.0);
-  p = fma(p, r, 1.0 / 39916800.0);
-  p = fma(p, r, 1.0 / 3628800.0);
-  p = fma(p, r, 1.0 / 362880.0);
-  p = fma(p, r, 1.0 / 40320.0);
-  p = fma(p, r, 1.0 / 5040.0);
-  p = fma(p, r, 1.0 / 720.0);
-  p = fma(p, r, 1.0 / 120.0);
-  p = fma(p, r, 1.0 / 24.0);
-  p = fma(p, r, 1.0 / 6.0);
+// Taylor polynomial by Horner with fma, scaled by 2^k in one v_ldexp_f64.
+// The scaling rounds once (a subnormal result) or not at all, saturates to
+// inf above ln of the largest double and rounds to 0 below -745.13, so no
+// range selects are needed; the clamp only keeps the reduction of huge
+// arguments finite, and NaN passes through.
+struct ExpConst {
+  double inv_ln2 = 1.44269504088896338700e+00;
+  double nln2_hi = -6.93147180369123816490e-01;
+  double nln2_lo = -1.90821492927058770002e-10;
+  // 1/13!, 1/12!, .., 1/3!
+  double c[11] = {1.0 / 6227020800.0, 1.0 / 479001600.0, 1.0 / 39916800.0, 1.0 / 3628800.0,
+                  1.0 / 362880.0,     1.0 / 40320.0,     1.0 / 5040.0,     1.0 / 720.0,
+                  1.0 / 120.0,        1.0 / 24.0,        1.0 / 6.0};
+  // Holds the constants in vector registers across a loop: as literals each
+  // evaluation re-creates them (a 64-bit literal is two moves, and a wave
+  // issues one instruction of any kind per 4 cycles).
+  __device__ __forceinline__ void pin() {
+    asm("" : "+v"(inv_ln2), "+v"(nln2_hi), "+v"(nln2_lo));
+#pragma unroll
+    for (int k = 0; k < 11; ++k) asm("" : "+v"(c[k]));
+  }
+};
+
+__device__ __forceinline__ double exp_k(double x, const ExpConst &K) {
+  const double xc = fmin(fmax(x, -1500.0), 1500.0);
+  const double kd = rint(xc * K.inv_ln2);
+  double r = fma(kd, K.nln2_hi, xc);
+  r = fma(kd, K.nln2_lo, r);
+  double p = K.c[0];
+#pragma unroll
+  for (int k = 1; k < 11; ++k) p = fma(p, r, K.c[k]);
   p = fma(p, r, 0.5);
   p = fma(p, r, 1.0);
   p = fma(p, r, 1.0);
-  const int k = (int)kd;
-  const int k1 = k >> 1;
-  const int k2 = k - k1;
-  const double s1 = __longlong_as_double((long long)(k1 + 1023) << 52);
-  const double s2 = __longlong_as_double((long long)(k2 + 1023) << 52);
-  double res = (p * s1) * s2;
-  // out-of-range and NaN inputs: +inf above, 0 below, NaN through
-  res = (x > kOvf) ? __longlong_as_double(0x7FF0000000000000ll) : res;
-  res = (x < kUnf) ? 0.0 : res;
-  res = (x != x) ? x : res;
-  return res;
+  const double res = __builtin_amdgcn_ldexp(p, (int)kd);
+  return (x != x) ? x : res;
+}
+__device__ __forceinline__ double exp_m(double x) { return exp_k(x, ExpConst{}); }
+
+// sqrt(x), correctly rounded, for 2^-767 <= x < 2^1000: Goldschmidt's
+// iteration from v_rsq_f64 (Markstein, "Software division and square root
+// using Goldschmidt's algorithms", 2004) with two residual corrections, and
+// none of sqrt's scaling and zero/infinity selects.  0, infinity and NaN give
+// NaN; smaller arguments are the caller's to exclude.
+__device__ __forceinline__ double sqrt_normal(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  return fma(fma(-g, g, x), h, g);
+}
+
+// x^2 + y^2 + z^2 as norm3 sums it
+__device__ __forceinline__ double sumsq3(double x, double y, double z) {
+  double s = x * x;
+  s = s + y * y;
+  return s + z * z;
 }
 
 // |v| as sqrt((x*x + y*y) + z*z), two roundings per term.

@@ -69,7 +69,8 @@ struct Eval2Args {
   double *value, *grad, *lap, *e_local, *pgrad;
 };
 
-// variant: 0 auto, 1 one lane per walker, 2 wave-specialised (when eligible)
+// One electron-nucleus distance (helium) or at most two orbital centres: the
+// wave-specialised and unrolled one-lane kernels apply.
 bool sweep2_wavespec_eligible(const Sys2 &sp);
 
 // One optimizer step on the device from the reduced accumulator columns
@@ -82,8 +83,8 @@ hipError_t launch_block_records(const double *trace_e, int W, size_t cap, size_t
                                 double *out, hipStream_t stream);
 hipError_t launch_vmc_step(const double *red, double n_samples, double *params, mole_optimizer *opt, double *log,
                            hipStream_t stream);
-hipError_t launch_sweep2(const Sweep2Args &a, int variant, int block_threads,
-                         hipStream_t stream);
+// variant MOLE_VARIANT_*; cus: compute units of the device
+hipError_t launch_sweep2(const Sweep2Args &a, int variant, int block_threads, int cus, hipStream_t stream);
 hipError_t launch_init2(double *pos, int W, uint64_t seed, uint32_t sys,
                         uint32_t epoch, hipStream_t stream);
 hipError_t launch_eval2(const Eval2Args &a, hipStream_t stream);

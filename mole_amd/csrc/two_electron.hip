@@ -1,11 +1,10 @@
 // Two-electron walker kernels (He singlet with Pade e-e factor; LCAO
 // sigma_g^2 with Pade e-e factor).
 //
-// One lane owns one walker for the whole launch: positions, the cached
-// psi and the distances it was built from, and every accumulator live in
-// VGPRs across all sweeps of the launch; HBM is touched once at entry and
-// once at exit (positions as [6][W] and accumulators as [column][W], both
-// coalesced).  Each move does what MetropolisBox::move_state does
+// A walker's positions, the cached psi and the distances it was built from,
+// and every accumulator live in VGPRs across all sweeps of the launch; HBM is
+// touched once at entry and once at exit (positions as [6][W] and accumulators
+// as [column][W], both coalesced).  Each move does what MetropolisBox::move_state does
 // (src/metropolis/src/metrop.rs:60-96): three Range draws, one Standard
 // draw, psi at the proposal, min(psi'^2/psi^2, 1) > u.  psi at the
 // current configuration is the cached value of the same expression, so
@@ -19,6 +18,7 @@
 #include "device_common.hpp"
 #include "internal.hpp"
 #include "sr_math.hpp"
+#include <type_traits>
 
 namespace mole {
 
@@ -142,10 +142,8 @@ struct SampleAcc {
     for (int k = 0; k < kAccColumns2; ++k)
       if (k != kAccAccepted) a.acc[(size_t)k * a.W + w] = acc[k];
   }
-  // write: this lane records the sample's trace and compat entries (the
-  // sums are kept either way)
   __device__ __forceinline__ void add(const Sweep2Args &a, int w, double E,
-                                      const double *dlog, double psi, double inv_block, bool write = true) {
+                                      const double *dlog, double psi, double inv_block) {
     acc[kAccSumE] += E;
     acc[kAccSumE2] = fma(E, E, acc[kAccSumE2]);
     acc[kAccBlockSum] += E;
@@ -159,7 +157,10 @@ struct SampleAcc {
     double O[kNParam2];
     if (a.o_conv == MOLE_O_REFERENCE) {
       // G = psi ./ (psi * dpsi), dpsi = psi dlog; O = G / psi_s with
-      // psi_s = (psi*psi)/psi the "Wavefunction value" sample
+      // psi_s = (psi*psi)/psi the "Wavefunction value" sample.  The empty asm
+      // keeps these seven divisions behind the branch: without it they are
+      // computed for every sample and selected away.
+      asm volatile("");
       const double psi_s = (psi * psi) / psi;
 #pragma unroll
       for (int k = 0; k < kNParam2; ++k) O[k] = (psi / (psi * (psi * dlog[k]))) / psi_s;
@@ -176,7 +177,7 @@ struct SampleAcc {
       for (int l = k; l < kNParam2; ++l, ++t)
         acc[kAccSumOO + t] = fma(O[k], O[l], acc[kAccSumOO + t]);
     }
-    if (write && sample_idx < a.cap_samples) {
+    if (sample_idx < a.cap_samples) {
       const size_t si = (size_t)w * a.cap_samples + sample_idx;
       const double psi_s = (psi * psi) / psi;
       if (a.trace_e) a.trace_e[si] = E;
@@ -332,234 +333,18 @@ __device__ __forceinline__ void local2_cached(const Sys2 &sp, const double *x,
   dlog[2] = -b * r12 * r12 * iden * iden;
 }
 
-// Wave-specialised sweep: a workgroup of four waves owns 64 walkers.
-//   wave 0      the Metropolis chain (proposal, psi', accept, state update);
-//   waves 1, 2  Philox draws of chunk c+1 (electron 0 / electron 1) into LDS;
-//   wave 3      local energy, d ln psi/dp and accumulators of chunk c-1,
-//               from state snapshots the chain leaves in LDS.
-// Chunks are T sweeps; every buffer is double-buffered and the four roles
-// meet at one barrier per chunk, so the chain -- the only serial part --
-// runs alone on its SIMD and its arithmetic is exactly that of the
-// one-wave kernel.
-template <int KIND, int NNUC, int T>
-__global__ void __launch_bounds__(256) sweep2_ws_kernel(Sweep2Args a) {
-  constexpr int SNAP = 6 + 4 * NNUC + 2;  // x, r[e][I], e[e][I], r12, psi
-  // one block with the draws first: their LDS addresses then start at 0, so
-  // the eight draws of a sweep are one base register plus immediate offsets
-  struct Lds {
-    double rng[2][T][2][4][64];
-    double snap[2][T][SNAP][64];
-  };
-  __shared__ Lds lds;
-  auto &rng_lds = lds.rng;
-  auto &snap_lds = lds.snap;
-  const int lane = threadIdx.x & 63;
-  const int role = threadIdx.x >> 6;
-  const int w = blockIdx.x * 64 + lane;
-  const bool live = w < a.W;
-  const int W = a.W;
-  Sys2 sp = a.sp;
-  if (a.dparams) {  // parameters updated on the device between launches
-    sp.zeta = a.dparams[0];
-    sp.b = a.dparams[1];
-    sp.c = a.dparams[2];
-  }
-  const uint32_t nchunks = (a.n_sweeps + T - 1) / T;
-  const double inv_block = 1.0 / (double)a.block_size;
-
-  // chain state
-  double x[6];
-  double r[2][NNUC], ee[2][NNUC], phi[2];
-  double r12 = 0.0, psi = 1.0, accepted = 0.0;
-  // producer state
-  Stream rng;
-  // sampler state
-  SampleAcc sa;
-
-  if (role == 0) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) x[k] = live ? a.pos[(size_t)k * W + w] : 0.0;
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      phi[e] = 0.0;
-#pragma unroll
-      for (int I = 0; I < NNUC; ++I) {
-        r[e][I] = norm3(x[3 * e] - sp.nuc[I][0], x[3 * e + 1] - sp.nuc[I][1],
-                        x[3 * e + 2] - sp.nuc[I][2]);
-        ee[e][I] = (KIND == MOLE_WF_HELIUM_PADE) ? 1.0 : exp_m(-sp.zeta * r[e][I]);
-        phi[e] = (I == 0) ? ee[e][I] : phi[e] + ee[e][I];
-      }
-    }
-    r12 = norm3(x[0] - x[3], x[1] - x[4], x[2] - x[5]);
-    if (KIND == MOLE_WF_HELIUM_PADE) {
-      psi = exp_m(-sp.zeta * (r[0][0] + r[1][0]) + pade(sp.b, sp.c, r12));
-    } else {
-      psi = (phi[0] * phi[1]) * exp_m(pade(sp.b, sp.c, r12));
-    }
-    accepted = (live && !a.fresh) ? a.acc[(size_t)kAccAccepted * W + w] : 0.0;
-  } else if (role == 3) {
-    if (live) sa.load(a, w);
-  } else {
-    rng.init(a.seed, a.sys, (uint32_t)w, a.epoch);
-  }
-
-  // producers: draws of chunk cc for electron e = role - 1
-  auto produce = [&](uint32_t cc) {
-    const int e = role - 1;
-    const int buf = cc & 1;
-    const uint32_t s0 = cc * T;
-    for (int t = 0; t < T; ++t) {
-      if (s0 + t >= a.n_sweeps) break;
-      const uint64_t p = a.draw0 + ((uint64_t)(s0 + t) * 2 + e) * 4;
-      rng_lds[buf][t][e][0][lane] = u64_range(rng.draw(p), a.scale, a.offset);
-      rng_lds[buf][t][e][1][lane] = u64_range(rng.draw(p + 1), a.scale, a.offset);
-      rng_lds[buf][t][e][2][lane] = u64_range(rng.draw(p + 2), a.scale, a.offset);
-      rng_lds[buf][t][e][3][lane] = u64_standard(rng.draw(p + 3));
-    }
-  };
-
-  if (role == 1 || role == 2) {
-    if (nchunks > 0) produce(0);
-  }
-  __syncthreads();
-
-  for (uint32_t c = 0; c <= nchunks; ++c) {
-    const int buf = c & 1;
-    const uint32_t s0 = c * T;
-    if (role == 0 && c < nchunks) {
-      for (int t = 0; t < T; ++t) {
-        const uint32_t s = s0 + t;
-        if (s >= a.n_sweeps) break;
-        // the sweep's eight draws read from LDS together, ahead of the arithmetic
-        double dr[2][4];
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) dr[e][k] = rng_lds[buf][t][e][k][lane];
-        uint64_t mask = 0;
-        // electron-local parts of both moves first (trial position, distances to
-        // the nuclei, orbital values: none depends on the other electron's
-        // decision), then each move's coupled part (r12, Jastrow, ratio) in
-        // order; the updates are selects.  Every value is computed by the same
-        // operations from the same operands as move-by-move code, so the chain
-        // is bit-identical while its two halves overlap in the pipeline.
-        double nx[2][3], nr[2][NNUC], ne[2][NNUC], nphi[2], uu[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          nx[e][0] = x[3 * e] + dr[e][0];
-          nx[e][1] = x[3 * e + 1] + dr[e][1];
-          nx[e][2] = x[3 * e + 2] + dr[e][2];
-          uu[e] = dr[e][3];
-          nphi[e] = 0.0;
-#pragma unroll
-          for (int I = 0; I < NNUC; ++I) {
-            nr[e][I] = norm3(nx[e][0] - sp.nuc[I][0], nx[e][1] - sp.nuc[I][1], nx[e][2] - sp.nuc[I][2]);
-            ne[e][I] = (KIND == MOLE_WF_HELIUM_PADE) ? 1.0 : exp_m(-sp.zeta * nr[e][I]);
-            nphi[e] = (I == 0) ? ne[e][I] : nphi[e] + ne[e][I];
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const double n12 = (e == 0) ? norm3(nx[0][0] - x[3], nx[0][1] - x[4], nx[0][2] - x[5])
-                                      : norm3(x[0] - nx[1][0], x[1] - nx[1][1], x[2] - nx[1][2]);
-          double psin;
-          if (KIND == MOLE_WF_HELIUM_PADE) {
-            const double s12 = (e == 0) ? (nr[0][0] + r[1][0]) : (r[0][0] + nr[1][0]);
-            psin = exp_m(-sp.zeta * s12 + pade(sp.b, sp.c, n12));
-          } else {
-            const double jas = exp_m(pade(sp.b, sp.c, n12));
-            psin = ((e == 0) ? (nphi[0] * phi[1]) : (phi[0] * nphi[1])) * jas;
-          }
-          const double ratio = min_one((psin * psin) / (psi * psi));
-          const bool acc = ratio > uu[e];
-          x[3 * e] = sel(acc, nx[e][0], x[3 * e]);
-          x[3 * e + 1] = sel(acc, nx[e][1], x[3 * e + 1]);
-          x[3 * e + 2] = sel(acc, nx[e][2], x[3 * e + 2]);
-#pragma unroll
-          for (int I = 0; I < NNUC; ++I) {
-            r[e][I] = sel(acc, nr[e][I], r[e][I]);
-            ee[e][I] = sel(acc, ne[e][I], ee[e][I]);
-          }
-          phi[e] = sel(acc, nphi[e], phi[e]);
-          r12 = sel(acc, n12, r12);
-          psi = sel(acc, psin, psi);
-          accepted += acc ? 1.0 : 0.0;
-          mask |= acc ? ((uint64_t)1 << e) : 0;
-        }
-        if (live && a.trace_mask && a.trace_sweep0 + s < a.cap_sweeps)
-          a.trace_mask[(size_t)w * a.cap_sweeps + a.trace_sweep0 + s] = mask;
-        double *sn = &snap_lds[buf][t][0][0];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) sn[k * 64 + lane] = x[k];
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-#pragma unroll
-          for (int I = 0; I < NNUC; ++I) {
-            sn[(6 + e * NNUC + I) * 64 + lane] = r[e][I];
-            sn[(6 + 2 * NNUC + e * NNUC + I) * 64 + lane] = ee[e][I];
-          }
-        sn[(6 + 4 * NNUC) * 64 + lane] = r12;
-        sn[(7 + 4 * NNUC) * 64 + lane] = psi;
-      }
-    } else if ((role == 1 || role == 2) && c + 1 < nchunks) {
-      produce(c + 1);
-    } else if (role == 3 && c >= 1) {
-      const int pb = (c - 1) & 1;
-      const uint32_t p0 = (c - 1) * T;
-      for (int t = 0; t < T; ++t) {
-        const uint32_t s = p0 + t;
-        if (s >= a.n_sweeps) break;
-        if (s < a.sample_start) continue;
-        const double *sn = &snap_lds[pb][t][0][0];
-        double xs[6], rs[2][NNUC], es[2][NNUC];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) xs[k] = sn[k * 64 + lane];
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-#pragma unroll
-          for (int I = 0; I < NNUC; ++I) {
-            rs[e][I] = sn[(6 + e * NNUC + I) * 64 + lane];
-            es[e][I] = sn[(6 + 2 * NNUC + e * NNUC + I) * 64 + lane];
-          }
-        const double r12s = sn[(6 + 4 * NNUC) * 64 + lane];
-        double E, dlog[kNParam2];
-        local2_cached<KIND, NNUC>(sp, xs, rs, es, r12s, E, dlog);
-        const double psis = sn[(7 + 4 * NNUC) * 64 + lane];
-        if (live) sa.add(a, w, E, dlog, psis, inv_block);
-      }
-    }
-    __syncthreads();
-  }
-
-  if (role == 0 && live) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) a.pos[(size_t)k * W + w] = x[k];
-    a.acc[(size_t)kAccAccepted * W + w] = accepted;
-  } else if (role == 3 && live) {
-    sa.store(a, w);
-  }
+// Metropolis decision min(a / b, 1) > u (a = psi'^2, b = psi^2) without the
+// division where its outcome is beyond rounding: t = a - u b is formed with
+// one rounding, and with |t| > 2^-50 b the quotient differs from u by more
+// than two units in u's last place (u < 1), so its rounding lies on the same
+// side of u.  Close calls, NaN, infinities and b < 2^-900 are not `sure`: the
+// caller then divides (accept_div), so every decision is the division's.
+__device__ __forceinline__ bool accept_fast(double a, double b, double u, bool &sure) {
+  const double t = fma(-u, b, a);
+  sure = sure && fabs(t) > b * 0x1p-50 && b > 0x1p-900;
+  return t > 0.0;
 }
-
-// ---- four lanes per walker ---------------------------------------------------
-//
-// A quad of lanes owns one walker; every lane holds the walker's state.  Per
-// sweep, lane q
-//   - draws u64s p+2q and p+2q+1 (one Philox block when p is even): lanes 0-1
-//     hold electron 0's (dx, dy | dz, u), lanes 2-3 electron 1's;
-//   - forms electron q/2's trial position and its distance and orbital
-//     exponential to nucleus q%2 (the electron-local part of the moves);
-//   - forms one coupled part: lane 0 electron 0's (r12', Jastrow / psi'),
-//     lane 1 electron 1's if electron 0's move is rejected, lanes 2-3 if it
-//     is accepted;
-// and the lanes exchange these by DPP quad permutations (register moves, no
-// LDS, no barrier).  The remaining chain -- two ratios and the selects of
-// the state update -- runs on all four lanes alike.  Every value is the
-// same operation on the same operands as in the one-lane chain, so the
-// trajectories are bit for bit the other kernels'.  After a sampled sweep
-// the local energy is split the same way: lane q divides by r_{q/2, q%2},
-// then by phi_0 (lane 0), r12 (lane 1), phi_1 (lane 2), 1 + c r12 (lane 3),
-// with local2_cached's operations in its order.  With 4 lanes per walker,
-// 16,384 walkers occupy all 1,024 SIMDs of the chip.
+__device__ __forceinline__ bool accept_div(double a, double b, double u) { return min_one(a / b) > u; }
 
 constexpr int kQuadXor1 = 0xB1;  // quad_perm [1, 0, 3, 2]
 constexpr int kQuadXor2 = 0x4E;  // quad_perm [2, 3, 0, 1]
@@ -574,16 +359,46 @@ __device__ __forceinline__ double quad_mov(double v) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// coordinate k of electron 1 (e1) or electron 0
-__device__ __forceinline__ double xe_sel(bool e1, const double *x, int k) { return e1 ? x[3 + k] : x[k]; }
+// Wave-specialised sweep.  A workgroup of G + 2 waves owns NW = 64 G / L
+// walkers:
+//   waves 0 .. G-1  the Metropolis chain, L lanes (2 or 4) per walker;
+//   wave G          local energy, d ln psi/dp and accumulators of chunk c-1
+//                   from snapshots the chain leaves, one lane per walker;
+//   wave G + 1      Philox draws of chunk c+1 into LDS (S of every 4 draw
+//                   pairs by the sampler wave, to even the two out).
+// Chunks are T sweeps, double-buffered, one barrier per chunk.
+//
+// The chain is a serial sequence of FP64 operations; a wave issues one
+// instruction per 4 cycles whatever its kind, so the chain's instruction
+// count bounds every walker count that fits the chip at once, and it is
+// spread over the lanes.  L = 4: lane q forms the trial position's distance
+// and orbital exponential for electron q/2 and nucleus q%2, then one coupled
+// part (r12', Jastrow, psi'): lane 0 electron 0's, lane 1 electron 1's if
+// electron 0's move is rejected, lanes 2-3 if it is accepted.  L = 2: lane h
+// forms electron h's local part for all nuclei, then electron 0's (lane 0) or
+// the rejected electron 1's (lane 1) coupled part, and both lanes the accepted
+// one.  DPP permutations exchange the results; the decisions and the selects
+// of the state update run on all lanes alike.  Every value is the same
+// operation on the same operands as in the one-lane kernel, so trajectories
+// agree bit for bit.
+constexpr int kPairEven = 0xA0;  // quad_perm [0, 0, 2, 2]
+constexpr int kPairOdd = 0xF5;   // quad_perm [1, 1, 3, 3]
 
-template <int KIND, int NNUC>
-__global__ void __launch_bounds__(64) sweep2_quad_kernel(Sweep2Args a) {
-  static_assert(NNUC == 1 || NNUC == 2, "one lane per (electron, nucleus) pair");
-  const int q = threadIdx.x & 3;
-  const int w = (int)((blockIdx.x * 64u + threadIdx.x) >> 2);
-  const bool live = w < a.W;
-  const bool lead = live && q == 0;  // writes the walker's results
+template <int KIND, int NNUC, int L, int G, int S, int T>
+__global__ void __launch_bounds__(64 * (G + 2)) sweep2_ws_kernel(Sweep2Args a) {
+  constexpr bool HE = KIND == MOLE_WF_HELIUM_PADE;
+  constexpr int NW = 64 * G / L;
+  static_assert(NW <= 64, "one sampler lane per walker");
+  constexpr int NE = HE ? 0 : 2 * NNUC;        // orbital exponentials kept
+  constexpr int SNAP = 6 + 2 * NNUC + NE + 1;  // x, r[e][I], ee[e][I], psi
+  struct Lds {
+    double rng[2][T][8][NW];
+    double snap[2][T][SNAP][NW];
+  };
+  __shared__ Lds lds;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int w0 = blockIdx.x * NW;
   const int W = a.W;
   Sys2 sp = a.sp;
   if (a.dparams) {  // parameters updated on the device between launches
@@ -591,241 +406,360 @@ __global__ void __launch_bounds__(64) sweep2_quad_kernel(Sweep2Args a) {
     sp.b = a.dparams[1];
     sp.c = a.dparams[2];
   }
-  const bool me = (q >> 1) != 0;                 // this lane's electron is 1
-  const bool mi = NNUC == 2 && (q & 1) != 0;     // this lane's nucleus is 1
-  const double *Rq = mi ? sp.nuc[NNUC - 1] : sp.nuc[0];
-  const double inv_block = 1.0 / (double)a.block_size;
+  const uint32_t nchunks = (a.n_sweeps + T - 1) / T;
 
-  // the walker's state, on every lane of the quad
-  double x[6];
+  if (wave >= G) {
+    // draws p .. p+7 of a sweep as (dx, dy, dz, u) per electron, in pairs (one
+    // Philox block each when p is even); pairs [b0, b1) of every 4 here
+    const uint32_t k0 = (uint32_t)a.seed, k1 = (uint32_t)(a.seed >> 32) ^ a.sys;
+    const bool odd = (a.draw0 & 1) != 0;
+    auto produce = [&](uint32_t cc, int b0, int nb) {
+      const int nt = (int)min((uint32_t)T, a.n_sweeps - cc * T);
+      for (int it = lane; it < nt * nb * NW; it += 64) {
+        const int wl = it % NW, tb = it / NW;
+        const int t = tb / nb, b = b0 + tb % nb;
+        const uint64_t blk = ((a.draw0 + 8 * (uint64_t)(cc * T + t)) >> 1) + b;
+        const uint32_t wg = (uint32_t)(w0 + wl);
+        u32x4 o = philox4x32_10({(uint32_t)blk, (uint32_t)(blk >> 32), wg, a.epoch}, k0, k1);
+        if (odd) {  // the pair straddles two blocks
+          const u32x4 o2 = philox4x32_10({(uint32_t)(blk + 1), (uint32_t)((blk + 1) >> 32), wg, a.epoch}, k0, k1);
+          o = {o.z, o.w, o2.x, o2.y};
+        }
+        const uint64_t v0 = (uint64_t)o.x | ((uint64_t)o.y << 32), v1 = (uint64_t)o.z | ((uint64_t)o.w << 32);
+        double *d = &lds.rng[cc & 1][t][2 * b][wl];
+        d[0] = u64_range(v0, a.scale, a.offset);
+        d[NW] = (b & 1) ? u64_standard(v1) : u64_range(v1, a.scale, a.offset);
+      }
+    };
+    if (wave > G) {
+      if (nchunks > 0) produce(0, S, 4 - S);
+      __syncthreads();
+      for (uint32_t c = 0; c <= nchunks; ++c) {
+        if (c + 1 < nchunks) produce(c + 1, S, 4 - S);
+        __syncthreads();
+      }
+      return;
+    }
+    const int w = w0 + lane;
+    const bool live = lane < NW && w < W;
+    const int wl = lane < NW ? lane : 0;
+    const double inv_block = 1.0 / (double)a.block_size;
+    SampleAcc sa;
+    if (live) sa.load(a, w);
+    if constexpr (S > 0)
+      if (nchunks > 0) produce(0, 0, S);
+    __syncthreads();
+    for (uint32_t c = 0; c <= nchunks; ++c) {
+      if constexpr (S > 0)
+        if (c + 1 < nchunks) produce(c + 1, 0, S);
+      if (c >= 1) {
+        const uint32_t p0 = (c - 1) * T;
+        const int nt = (int)min((uint32_t)T, a.n_sweeps - p0);
+#pragma unroll 1
+        for (int t = a.sample_start > p0 ? (int)min((uint32_t)T, a.sample_start - p0) : 0; t < nt; ++t) {
+          const double *sn = &lds.snap[(c - 1) & 1][t][0][wl];
+          double xs[6], rs[2][NNUC], es[2][NNUC];
+#pragma unroll
+          for (int k = 0; k < 6; ++k) xs[k] = sn[k * NW];
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int I = 0; I < NNUC; ++I) {
+              rs[e][I] = sn[(6 + e * NNUC + I) * NW];
+              es[e][I] = HE ? 1.0 : sn[(6 + 2 * NNUC + e * NNUC + I) * NW];
+            }
+          const double psis = sn[(SNAP - 1) * NW];
+          const double r12 = norm3(xs[0] - xs[3], xs[1] - xs[4], xs[2] - xs[5]);
+          double E, dlog[kNParam2];
+          local2_cached<KIND, NNUC>(sp, xs, rs, es, r12, E, dlog);
+          if (live) sa.add(a, w, E, dlog, psis, inv_block);
+        }
+      }
+      __syncthreads();
+    }
+    if (live) sa.store(a, w);
+    return;
+  }
+
+  // ---- chain ----
+  const int q = lane & (L - 1);
+  const int wl = wave * (64 / L) + lane / L;
+  const int w = w0 + wl;
+  const bool live = w < W;
+  const bool lead = q == 0;
+  const bool me = L == 4 ? (q >> 1) != 0 : q != 0;      // this lane's electron is 1
+  const bool c0 = q == 0, c1 = q == 1;
+  constexpr int NL = L == 4 ? 1 : NNUC;                 // nuclei of this lane's local part
+  const int I0 = (L == 4 && NNUC == 2) ? (q & 1) : 0;   // the first of them
+  double R[NL][3];
+#pragma unroll
+  for (int I = 0; I < NL; ++I)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) R[I][k] = (L == 4 && NNUC == 2 && I0) ? sp.nuc[NNUC - 1][k] : sp.nuc[I][k];
+  ExpConst K;
+  K.pin();
+  const double nzeta = -sp.zeta;
+  // the orbital value (LCAO) or nuclear distance (helium) of both electrons
+  // from each lane's local parts
+  auto exchange = [&](const double *rl, const double *el, double &f0, double &f1) {
+    double fe = HE ? rl[0] : el[0];
+    if constexpr (!HE && NNUC == 2) fe = fe + (L == 4 ? quad_mov<kQuadXor1>(el[0]) : el[NL - 1]);
+    f0 = quad_mov<L == 4 ? kQuadLane0 : kPairEven>(fe);
+    f1 = quad_mov<L == 4 ? kQuadLane2 : kPairOdd>(fe);
+  };
+  double x[6], rl[NL], el[NL], f[2];
 #pragma unroll
   for (int k = 0; k < 6; ++k) x[k] = live ? a.pos[(size_t)k * W + w] : 0.0;
-  double r[2][NNUC], ee[2][NNUC], phi[2];
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    phi[e] = 0.0;
+  for (int I = 0; I < NL; ++I) {
+    rl[I] = norm3((me ? x[3] : x[0]) - R[I][0], (me ? x[4] : x[1]) - R[I][1], (me ? x[5] : x[2]) - R[I][2]);
+    el[I] = HE ? 1.0 : exp_k(nzeta * rl[I], K);
+  }
+  exchange(rl, el, f[0], f[1]);
+  double psi;
+  {
+    const double r12 = norm3(x[0] - x[3], x[1] - x[4], x[2] - x[5]);
+    psi = HE ? exp_k(nzeta * (f[0] + f[1]) + pade(sp.b, sp.c, r12), K)
+             : (f[0] * f[1]) * exp_k(pade(sp.b, sp.c, r12), K);
+  }
+  double psi2 = psi * psi;
+  uint32_t n_acc = 0;
+  __syncthreads();
+
+  for (uint32_t c = 0; c <= nchunks; ++c) {
+    const uint32_t s0 = c * T;
+    const int nt = c < nchunks ? (int)min((uint32_t)T, a.n_sweeps - s0) : 0;
+#pragma unroll 1
+    for (int t = 0; t < nt; ++t) {
+      // the sweep's eight draws together, ahead of the arithmetic
+      double d[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) d[k] = lds.rng[c & 1][t][k][wl];
+      double n[6];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        n[k] = x[k] + d[k];
+        n[3 + k] = x[3 + k] + d[4 + k];
+      }
+      double nr[NL], ne[NL], nf0, nf1;
+      double p0, pr, pa;  // psi' of electron 0's move, and of electron 1's after its rejection / acceptance
+      double smin;        // the smallest square root argument
+      // FAST leaves out sqrt's range handling; its results stand if every
+      // argument is in sqrt_normal's range and every decision is sure (an
+      // infinity, zero or NaN under a root makes psi' NaN, which is not)
+      auto evaluate = [&](auto fast) {
+        constexpr bool FAST = decltype(fast)::value;
+        auto root = [&](double v0, double v1, double v2) {
+          const double ss = sumsq3(v0, v1, v2);
+          if constexpr (FAST) {
+            smin = fmin(smin, ss);
+            return sqrt_normal(ss);
+          } else {
+            return sqrt(ss);
+          }
+        };
+        smin = 1.0;
+#pragma unroll
+        for (int I = 0; I < NL; ++I) {
+          nr[I] = root(sel(me, n[3], n[0]) - R[I][0], sel(me, n[4], n[1]) - R[I][1], sel(me, n[5], n[2]) - R[I][2]);
+          ne[I] = HE ? 1.0 : exp_k(nzeta * nr[I], K);
+        }
+        exchange(nr, ne, nf0, nf1);
+        auto coupled = [&](const double *A, const double *B, double fa, double fb) {
+          const double J = pade(sp.b, sp.c, root(A[0] - B[0], A[1] - B[1], A[2] - B[2]));
+          if constexpr (HE) return exp_k(nzeta * (fa + fb) + J, K);
+          else return (fa * fb) * exp_k(J, K);
+        };
+        const bool ko = L == 4 ? c1 : me, kn = L == 4 ? c0 : !me;  // electron 0 / 1 stays put
+        double A[3], B[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          A[k] = sel(ko, x[k], n[k]);
+          B[k] = sel(kn, x[3 + k], n[3 + k]);
+        }
+        const double pc = coupled(A, B, sel(ko, f[0], nf0), sel(kn, f[1], nf1));
+        if constexpr (L == 4) {
+          p0 = quad_mov<kQuadLane0>(pc);
+          pr = quad_mov<kQuadLane1>(pc);
+          pa = quad_mov<kQuadLane2>(pc);
+        } else {
+          p0 = quad_mov<kPairEven>(pc);
+          pr = quad_mov<kPairOdd>(pc);
+          pa = coupled(n, n + 3, nf0, nf1);
+        }
+      };
+      evaluate(std::true_type{});
+      double p02 = p0 * p0, pr2 = pr * pr, pa2 = pa * pa;
+      bool sure = smin >= 0x1p-767;
+      bool acc0 = accept_fast(p02, psi2, d[3], sure);
+      bool acc1r = accept_fast(pr2, psi2, d[7], sure);
+      bool acc1a = accept_fast(pa2, p02, d[7], sure);
+      if (__builtin_expect(__any(!sure), 0)) {
+        evaluate(std::false_type{});
+        p02 = p0 * p0;
+        pr2 = pr * pr;
+        pa2 = pa * pa;
+        acc0 = accept_div(p02, psi2, d[3]);
+        acc1r = accept_div(pr2, psi2, d[7]);
+        acc1a = accept_div(pa2, p02, d[7]);
+      }
+      const bool acc1 = acc0 ? acc1a : acc1r;
+      const bool mine = me ? acc1 : acc0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        x[k] = sel(acc0, n[k], x[k]);
+        x[3 + k] = sel(acc1, n[3 + k], x[3 + k]);
+      }
+      f[0] = sel(acc0, nf0, f[0]);
+      f[1] = sel(acc1, nf1, f[1]);
+#pragma unroll
+      for (int I = 0; I < NL; ++I) {
+        rl[I] = sel(mine, nr[I], rl[I]);
+        if constexpr (!HE) el[I] = sel(mine, ne[I], el[I]);
+      }
+      psi = sel(acc1, sel(acc0, pa, pr), sel(acc0, p0, psi));
+      psi2 = psi * psi;
+      n_acc += (acc0 ? 1u : 0u) + (acc1 ? 1u : 0u);
+      if (a.trace_mask) {
+        const uint32_t s = s0 + t;
+        if (live && lead && a.trace_sweep0 + s < a.cap_sweeps)
+          a.trace_mask[(size_t)w * a.cap_sweeps + a.trace_sweep0 + s] = (acc0 ? 1ull : 0ull) | (acc1 ? 2ull : 0ull);
+      }
+      double *sn = &lds.snap[c & 1][t][0][wl];
+      if (lead) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) sn[k * NW] = x[k];
+        sn[(SNAP - 1) * NW] = psi;
+      }
+      // (with one nucleus both lanes of a quad's pair write the same value)
+      const int ri = (me ? NNUC : 0) + I0;
+#pragma unroll
+      for (int I = 0; I < NL; ++I) {
+        sn[(6 + ri + I) * NW] = rl[I];
+        if constexpr (!HE) sn[(6 + 2 * NNUC + ri + I) * NW] = el[I];
+      }
+    }
+    __syncthreads();
+  }
+  if (live && lead) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) a.pos[(size_t)k * W + w] = x[k];
+    a.acc[(size_t)kAccAccepted * W + w] = (a.fresh ? 0.0 : a.acc[(size_t)kAccAccepted * W + w]) + (double)n_acc;
+  }
+}
+
+// One lane per walker, every stage in the same wave, the distances and
+// orbital exponentials of the walker kept in registers: for walker counts
+// that fill every SIMD with walkers of its own, where the total of issued
+// instructions bounds the sweep and the pair's duplicated ones cost more than
+// its shorter chain gains.  262,144 walkers of H2: 19.6 -> 6.23 us per sweep
+// (the wave-specialised kernel's LDS let one workgroup on a CU).
+template <int KIND, int NNUC>
+__global__ void __launch_bounds__(256, 2) sweep2_wide_kernel(Sweep2Args a) {
+  constexpr bool HE = KIND == MOLE_WF_HELIUM_PADE;
+  const int w = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool live = w < a.W;
+  if (!live) return;
+  Sys2 sp = a.sp;
+  if (a.dparams) {  // parameters updated on the device between launches
+    sp.zeta = a.dparams[0];
+    sp.b = a.dparams[1];
+    sp.c = a.dparams[2];
+  }
+  const int W = a.W;
+  double x[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) x[k] = a.pos[(size_t)k * W + w];
+  double r[2][NNUC], ee[2][NNUC], f[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
 #pragma unroll
     for (int I = 0; I < NNUC; ++I) {
       r[e][I] = norm3(x[3 * e] - sp.nuc[I][0], x[3 * e + 1] - sp.nuc[I][1], x[3 * e + 2] - sp.nuc[I][2]);
-      ee[e][I] = (KIND == MOLE_WF_HELIUM_PADE) ? 1.0 : exp_m(-sp.zeta * r[e][I]);
-      phi[e] = (I == 0) ? ee[e][I] : phi[e] + ee[e][I];
+      ee[e][I] = HE ? 1.0 : exp_m(-sp.zeta * r[e][I]);
+      const double fI = HE ? r[e][I] : ee[e][I];
+      f[e] = (I == 0) ? fI : f[e] + fI;
     }
-  }
   double r12 = norm3(x[0] - x[3], x[1] - x[4], x[2] - x[5]);
-  double psi = (KIND == MOLE_WF_HELIUM_PADE) ? exp_m(-sp.zeta * (r[0][0] + r[1][0]) + pade(sp.b, sp.c, r12))
-                                             : (phi[0] * phi[1]) * exp_m(pade(sp.b, sp.c, r12));
-  double accepted = (live && !a.fresh) ? a.acc[(size_t)kAccAccepted * W + w] : 0.0;
+  double psi = HE ? exp_m(-sp.zeta * (f[0] + f[1]) + pade(sp.b, sp.c, r12)) : (f[0] * f[1]) * exp_m(pade(sp.b, sp.c, r12));
+  ExpConst K;
+  K.pin();
   SampleAcc sa;
-  if (live) {
-    sa.load(a, w);
-  } else {
-#pragma unroll
-    for (int k = 0; k < kAccColumns2; ++k) sa.acc[k] = 0.0;
-    sa.fill = a.block_fill;
-    sa.sample_idx = a.trace_sample0;
-  }
+  sa.load(a, w);
+  uint32_t n_acc = 0;
   Stream rng;
   rng.init(a.seed, a.sys, (uint32_t)w, a.epoch);
   uint64_t p = a.draw0;
-
+  const double inv_block = 1.0 / (double)a.block_size;
   for (uint32_t s = 0; s < a.n_sweeps; ++s) {
-    // ---- draws: electron q/2's (dx, dy) on its even lane, (dz, u) on its odd one
-    const uint64_t da = rng.draw(p + 2 * (uint64_t)q), db = rng.draw(p + 2 * (uint64_t)q + 1);
-    p += 8;
-    const bool odd = (q & 1) != 0;
-    const double va = u64_range(da, a.scale, a.offset);
-    const double vb = odd ? u64_standard(db) : u64_range(db, a.scale, a.offset);
-    const double pa = quad_mov<kQuadXor1>(va), pb = quad_mov<kQuadXor1>(vb);
-    const double dxe = odd ? pa : va, dye = odd ? pb : vb, dze = odd ? va : pa, ue = odd ? vb : pb;
-    // ---- electron-local part of this lane's (electron, nucleus)
-    const double xe0 = me ? x[3] : x[0], xe1 = me ? x[4] : x[1], xe2 = me ? x[5] : x[2];
-    const double nxe0 = xe0 + dxe, nxe1 = xe1 + dye, nxe2 = xe2 + dze;
-    const double nrq = norm3(nxe0 - Rq[0], nxe1 - Rq[1], nxe2 - Rq[2]);
-    const double neq = (KIND == MOLE_WF_HELIUM_PADE) ? 1.0 : exp_m(-sp.zeta * nrq);
-    // this electron's nuclei (the partner lane holds the other nucleus)
-    double nre[NNUC], nee[NNUC];
-    if constexpr (NNUC == 2) {
-      const double nrp = quad_mov<kQuadXor1>(nrq), nep = quad_mov<kQuadXor1>(neq);
-      nre[0] = mi ? nrp : nrq;
-      nre[1] = mi ? nrq : nrp;
-      nee[0] = mi ? nep : neq;
-      nee[1] = mi ? neq : nep;
-    } else {
-      nre[0] = nrq;
-      nee[0] = neq;
-    }
-    double nphie = nee[0];
-    if constexpr (NNUC == 2) nphie = nphie + nee[1];
-    // the other electron's, from the lane pair (q ^ 2)
-    double nx[2][3], nr[2][NNUC], ne[2][NNUC], nphi[2], uu[2];
-    {
-      const double o0 = quad_mov<kQuadXor2>(nxe0), o1 = quad_mov<kQuadXor2>(nxe1), o2 = quad_mov<kQuadXor2>(nxe2);
-      const double ou = quad_mov<kQuadXor2>(ue), ophi = quad_mov<kQuadXor2>(nphie);
-      nx[0][0] = me ? o0 : nxe0;
-      nx[0][1] = me ? o1 : nxe1;
-      nx[0][2] = me ? o2 : nxe2;
-      nx[1][0] = me ? nxe0 : o0;
-      nx[1][1] = me ? nxe1 : o1;
-      nx[1][2] = me ? nxe2 : o2;
-      uu[0] = me ? ou : ue;
-      uu[1] = me ? ue : ou;
-      nphi[0] = me ? ophi : nphie;
-      nphi[1] = me ? nphie : ophi;
-#pragma unroll
-      for (int I = 0; I < NNUC; ++I) {
-        const double orr = quad_mov<kQuadXor2>(nre[I]), oee = quad_mov<kQuadXor2>(nee[I]);
-        nr[0][I] = me ? orr : nre[I];
-        nr[1][I] = me ? nre[I] : orr;
-        ne[0][I] = me ? oee : nee[I];
-        ne[1][I] = me ? nee[I] : oee;
-      }
-    }
-    // ---- coupled parts: lane 0 electron 0's move; lane 1 electron 1's after
-    // a rejected, lanes 2-3 after an accepted move of electron 0
-    const bool c0 = q == 0, c1 = q == 1;
-    const double A0 = c1 ? x[0] : nx[0][0], A1 = c1 ? x[1] : nx[0][1], A2 = c1 ? x[2] : nx[0][2];
-    const double B0 = c0 ? x[3] : nx[1][0], B1 = c0 ? x[4] : nx[1][1], B2 = c0 ? x[5] : nx[1][2];
-    const double n12c = norm3(A0 - B0, A1 - B1, A2 - B2);
-    double valc;
-    if constexpr (KIND == MOLE_WF_HELIUM_PADE) {
-      const double s12 = c0 ? (nr[0][0] + r[1][0]) : (c1 ? (r[0][0] + nr[1][0]) : (nr[0][0] + nr[1][0]));
-      valc = exp_m(-sp.zeta * s12 + pade(sp.b, sp.c, n12c));
-    } else {
-      valc = exp_m(pade(sp.b, sp.c, n12c));
-    }
-    const double n12_0 = quad_mov<kQuadLane0>(n12c), n12_r = quad_mov<kQuadLane1>(n12c),
-                 n12_a = quad_mov<kQuadLane2>(n12c);
-    const double v_0 = quad_mov<kQuadLane0>(valc), v_r = quad_mov<kQuadLane1>(valc), v_a = quad_mov<kQuadLane2>(valc);
-    // ---- the chain: electron 0, then electron 1 (every lane)
     uint64_t mask = 0;
-    {
-      const double psin = (KIND == MOLE_WF_HELIUM_PADE) ? v_0 : (nphi[0] * phi[1]) * v_0;
-      const double ratio = min_one((psin * psin) / (psi * psi));
-      const bool acc = ratio > uu[0];
-      x[0] = sel(acc, nx[0][0], x[0]);
-      x[1] = sel(acc, nx[0][1], x[1]);
-      x[2] = sel(acc, nx[0][2], x[2]);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      double n[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) n[k] = x[3 * e + k] + u64_range(rng.draw(p + k), a.scale, a.offset);
+      const double u = u64_standard(rng.draw(p + 3));
+      p += 4;
+      double nr[NNUC], ne[NNUC], nf, n12, psin, smin;
+      auto evaluate = [&](auto fast) {  // as in sweep2_ws_kernel
+        constexpr bool FAST = decltype(fast)::value;
+        smin = 1.0;
+        auto root = [&](double v0, double v1, double v2) {
+          const double ss = sumsq3(v0, v1, v2);
+          if constexpr (FAST) {
+            smin = fmin(smin, ss);
+            return sqrt_normal(ss);
+          } else {
+            return sqrt(ss);
+          }
+        };
+#pragma unroll
+        for (int I = 0; I < NNUC; ++I) {
+          nr[I] = root(n[0] - sp.nuc[I][0], n[1] - sp.nuc[I][1], n[2] - sp.nuc[I][2]);
+          ne[I] = HE ? 1.0 : exp_k(-sp.zeta * nr[I], K);
+          const double fI = HE ? nr[I] : ne[I];
+          nf = (I == 0) ? fI : nf + fI;
+        }
+        n12 = (e == 0) ? root(n[0] - x[3], n[1] - x[4], n[2] - x[5]) : root(x[0] - n[0], x[1] - n[1], x[2] - n[2]);
+        const double fa = e == 0 ? nf : f[0], fb = e == 0 ? f[1] : nf;
+        const double J = pade(sp.b, sp.c, n12);
+        psin = HE ? exp_k(-sp.zeta * (fa + fb) + J, K) : (fa * fb) * exp_k(J, K);
+      };
+      evaluate(std::true_type{});
+      double pn2 = psin * psin;
+      const double ps2 = psi * psi;
+      bool sure = smin >= 0x1p-767;
+      bool acc = accept_fast(pn2, ps2, u, sure);
+      if (__builtin_expect(__any(!sure), 0)) {
+        evaluate(std::false_type{});
+        pn2 = psin * psin;
+        acc = accept_div(pn2, ps2, u);
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[3 * e + k] = sel(acc, n[k], x[3 * e + k]);
 #pragma unroll
       for (int I = 0; I < NNUC; ++I) {
-        r[0][I] = sel(acc, nr[0][I], r[0][I]);
-        ee[0][I] = sel(acc, ne[0][I], ee[0][I]);
+        r[e][I] = sel(acc, nr[I], r[e][I]);
+        if constexpr (!HE) ee[e][I] = sel(acc, ne[I], ee[e][I]);
       }
-      phi[0] = sel(acc, nphi[0], phi[0]);
-      r12 = sel(acc, n12_0, r12);
+      f[e] = sel(acc, nf, f[e]);
+      r12 = sel(acc, n12, r12);
       psi = sel(acc, psin, psi);
-      accepted += acc ? 1.0 : 0.0;
-      mask |= acc ? 1ull : 0ull;
-      // electron 1's coupled part for this outcome
-      const double n12_1 = acc ? n12_a : n12_r;
-      const double v_1 = acc ? v_a : v_r;
-      const double psin1 = (KIND == MOLE_WF_HELIUM_PADE) ? v_1 : (phi[0] * nphi[1]) * v_1;
-      const double ratio1 = min_one((psin1 * psin1) / (psi * psi));
-      const bool acc1 = ratio1 > uu[1];
-      x[3] = sel(acc1, nx[1][0], x[3]);
-      x[4] = sel(acc1, nx[1][1], x[4]);
-      x[5] = sel(acc1, nx[1][2], x[5]);
-#pragma unroll
-      for (int I = 0; I < NNUC; ++I) {
-        r[1][I] = sel(acc1, nr[1][I], r[1][I]);
-        ee[1][I] = sel(acc1, ne[1][I], ee[1][I]);
-      }
-      phi[1] = sel(acc1, nphi[1], phi[1]);
-      r12 = sel(acc1, n12_1, r12);
-      psi = sel(acc1, psin1, psi);
-      accepted += acc1 ? 1.0 : 0.0;
-      mask |= acc1 ? 2ull : 0ull;
+      n_acc += acc ? 1u : 0u;
+      mask |= acc ? ((uint64_t)1 << e) : 0;
     }
-    if (lead && a.trace_mask && a.trace_sweep0 + s < a.cap_sweeps)
+    if (a.trace_mask && a.trace_sweep0 + s < a.cap_sweeps)
       a.trace_mask[(size_t)w * a.cap_sweeps + a.trace_sweep0 + s] = mask;
-    if (s < a.sample_start) continue;
-    // ---- local energy and d ln psi/dp (local2_cached's operations, split over the quad)
-    const double zeta = sp.zeta, b = sp.b, c = sp.c;
-    double inv[2][NNUC];
-    {
-      const double rq = me ? (mi ? r[1][NNUC - 1] : r[1][0]) : (mi ? r[0][NNUC - 1] : r[0][0]);
-      const double iq = 1.0 / rq;
-      double ie[NNUC];
-      if constexpr (NNUC == 2) {
-        const double ip_ = quad_mov<kQuadXor1>(iq);
-        ie[0] = mi ? ip_ : iq;
-        ie[1] = mi ? iq : ip_;
-      } else {
-        ie[0] = iq;
-      }
-#pragma unroll
-      for (int I = 0; I < NNUC; ++I) {
-        const double oi = quad_mov<kQuadXor2>(ie[I]);
-        inv[0][I] = me ? oi : ie[I];
-        inv[1][I] = me ? ie[I] : oi;
-      }
+    if (s >= a.sample_start) {
+      double E, dlog[kNParam2];
+      local2_cached<KIND, NNUC>(sp, x, r, ee, r12, E, dlog);
+      sa.add(a, w, E, dlog, psi, inv_block);
     }
-    // this lane's electron: the sums over nuclei
-    double phis = 0.0, gs0 = 0.0, gs1 = 0.0, gs2 = 0.0, ls = 0.0, zs = 0.0;
-#pragma unroll
-    for (int I = 0; I < NNUC; ++I) {
-      const double d0 = xe_sel(me, x, 0) - sp.nuc[I][0], d1 = xe_sel(me, x, 1) - sp.nuc[I][1],
-                   d2 = xe_sel(me, x, 2) - sp.nuc[I][2];
-      const double iv = me ? inv[1][I] : inv[0][I];
-      const double eI = (KIND == MOLE_WF_HELIUM_PADE) ? 1.0 : (me ? ee[1][I] : ee[0][I]);
-      phis += eI;
-      const double f = -zeta * eI * iv;
-      gs0 = fma(f, d0, gs0);
-      gs1 = fma(f, d1, gs1);
-      gs2 = fma(f, d2, gs2);
-      ls = fma(eI, zeta * zeta - 2.0 * zeta * iv, ls);
-      zs = fma(-(me ? r[1][I] : r[0][I]), eI, zs);
-    }
-    // one division per lane: 1/phi_0, 1/r12, 1/phi_1, 1/(1 + c r12)
-    const double dv = (q & 1) ? ((q == 1) ? r12 : (1.0 + c * r12)) : phis;
-    const double qv = 1.0 / dv;
-    const double ip0 = quad_mov<kQuadLane0>(qv), i12 = quad_mov<kQuadLane1>(qv), ip1 = quad_mov<kQuadLane2>(qv),
-                 iden = quad_mov<kQuadLane3>(qv);
-    const double ogs0 = quad_mov<kQuadXor2>(gs0), ogs1 = quad_mov<kQuadXor2>(gs1), ogs2 = quad_mov<kQuadXor2>(gs2);
-    const double ols = quad_mov<kQuadXor2>(ls), ozs = quad_mov<kQuadXor2>(zs);
-    double E, dlog[kNParam2];
-    {
-      double V = sp.v_nn;
-#pragma unroll
-      for (int e = 0; e < 2; ++e)
-#pragma unroll
-        for (int I = 0; I < NNUC; ++I) V = V - sp.charge[I] * inv[e][I];
-      double gi[2][3], li[2], dz = 0.0;
-      const double g0[3] = {me ? ogs0 : gs0, me ? ogs1 : gs1, me ? ogs2 : gs2};
-      const double g1[3] = {me ? gs0 : ogs0, me ? gs1 : ogs1, me ? gs2 : ogs2};
-      const double ls0 = me ? ols : ls, ls1 = me ? ls : ols, zs0 = me ? ozs : zs, zs1 = me ? zs : ozs;
-      gi[0][0] = g0[0] * ip0;
-      gi[0][1] = g0[1] * ip0;
-      gi[0][2] = g0[2] * ip0;
-      li[0] = ls0 * ip0;
-      dz += zs0 * ip0;
-      gi[1][0] = g1[0] * ip1;
-      gi[1][1] = g1[1] * ip1;
-      gi[1][2] = g1[2] * ip1;
-      li[1] = ls1 * ip1;
-      dz += zs1 * ip1;
-      const double d0 = x[0] - x[3], d1 = x[1] - x[4], d2 = x[2] - x[5];
-      const double up = b * iden * iden;
-      const double upp = -2.0 * b * c * iden * iden * iden;
-      const double J = upp + 2.0 * up * i12 + up * up;
-      const double h0 = d0 * i12, h1 = d1 * i12, h2 = d2 * i12;
-      const double gd1 = gi[0][0] * h0 + gi[0][1] * h1 + gi[0][2] * h2;
-      const double gd2 = gi[1][0] * h0 + gi[1][1] * h1 + gi[1][2] * h2;
-      const double k1 = li[0] + J + 2.0 * up * gd1;
-      const double k2 = li[1] + J - 2.0 * up * gd2;
-      if (sp.hamiltonian == MOLE_H_ELECTRONIC) V = V + i12;
-      E = -0.5 * (k1 + k2) + V;
-      dlog[0] = dz;
-      dlog[1] = r12 * iden;
-      dlog[2] = -b * r12 * r12 * iden * iden;
-    }
-    sa.add(a, w, E, dlog, psi, inv_block, lead);
   }
-  if (lead) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) a.pos[(size_t)k * W + w] = x[k];
-    sa.store(a, w);
-    a.acc[(size_t)kAccAccepted * W + w] = accepted;
-  }
+  for (int k = 0; k < 6; ++k) a.pos[(size_t)k * W + w] = x[k];
+  sa.store(a, w);
+  a.acc[(size_t)kAccAccepted * W + w] = (a.fresh ? 0.0 : a.acc[(size_t)kAccAccepted * W + w]) + (double)n_acc;
 }
 
 __global__ void init2_kernel(double *pos, int W, uint64_t seed, uint32_t sys,
@@ -927,33 +861,52 @@ bool sweep2_wavespec_eligible(const Sys2 &sp) {
   return (sp.kind == MOLE_WF_HELIUM_PADE) ? sp.n_nuc == 1 : sp.n_nuc <= 2;
 }
 
-hipError_t launch_sweep2(const Sweep2Args &a, int variant, int block_threads, hipStream_t stream) {
+namespace {
+template <int KIND, int NNUC, int L, int G, int S, int T>
+void launch_ws(const Sweep2Args &a, hipStream_t stream) {
+  constexpr int NW = 64 * G / L;
+  hipLaunchKernelGGL((sweep2_ws_kernel<KIND, NNUC, L, G, S, T>), dim3((unsigned)((a.W + NW - 1) / NW)),
+                     dim3(64 * (G + 2)), 0, stream, a);
+}
+
+template <int KIND, int NNUC>
+void launch_spec(const Sweep2Args &a, int variant, int bt, int cus, hipStream_t stream) {
+  // us per sweep on 256 CUs, helium / H2 (start: four waves per 64 walkers,
+  // one lane per walker in the chain wave):
+  //   W         quad, 32/wg   pair, 64/wg   pair, T = 2   wide          start
+  //   8,192     0.60 / 0.70   0.69 / 0.85   0.75 / 0.87   1.37 / 1.87   0.80 / 1.24
+  //   16,384    0.89 / 1.11   0.71 / 0.86   0.77 / 0.87   1.38 / 1.90   0.83 / 1.26
+  //   32,768    1.43 / 2.02   1.08 / 1.71   1.12 / 1.40   1.39 / 1.90   1.59 / 2.45
+  //   49,152    2.08 / 2.92   1.62 / 2.61   1.55 / 2.02   1.37 / 1.86   -
+  //   262,144   10.1 / 14.5   7.86 / 13.8   6.90 / 9.42   4.40 / 6.23   12.6 / 19.6
+  // Up to 32 walkers per CU the quad's shorter chain wins; up to 64 the pair
+  // keeps one wave on each SIMD; up to 128 two pair workgroups share a CU if
+  // their LDS is small (T = 2); beyond that every SIMD has walkers of its own
+  // and the fewest instructions per walker win.
+  const int64_t per_cu = ((int64_t)a.W + cus - 1) / cus;
+  if (variant == MOLE_VARIANT_LANE || (variant == MOLE_VARIANT_AUTO && per_cu > 128))
+    hipLaunchKernelGGL((sweep2_wide_kernel<KIND, NNUC>), dim3((a.W + bt - 1) / bt), dim3(bt), 0, stream, a);
+  else if (variant == MOLE_VARIANT_QUAD || (variant == MOLE_VARIANT_AUTO && per_cu <= 32))
+    launch_ws<KIND, NNUC, 4, 2, 0, 4>(a, stream);
+  else if (variant == MOLE_VARIANT_WAVESPEC || per_cu <= 64)
+    launch_ws<KIND, NNUC, 2, 2, 1, 4>(a, stream);
+  else
+    launch_ws<KIND, NNUC, 2, 2, 1, 2>(a, stream);
+}
+}  // namespace
+
+hipError_t launch_sweep2(const Sweep2Args &a, int variant, int block_threads, int cus, hipStream_t stream) {
   const bool he = a.sp.kind == MOLE_WF_HELIUM_PADE;
-  const int nn = a.sp.n_nuc;
-  if (variant == MOLE_VARIANT_QUAD && sweep2_wavespec_eligible(a.sp)) {
-    // four lanes per walker, 16 walkers per one-wave workgroup
-    const dim3 grid((unsigned)((4 * (size_t)a.W + 63) / 64)), blk(64);
-    if (he)
-      hipLaunchKernelGGL((sweep2_quad_kernel<MOLE_WF_HELIUM_PADE, 1>), grid, blk, 0, stream, a);
-    else if (nn == 1)
-      hipLaunchKernelGGL((sweep2_quad_kernel<MOLE_WF_LCAO2_PADE, 1>), grid, blk, 0, stream, a);
-    else
-      hipLaunchKernelGGL((sweep2_quad_kernel<MOLE_WF_LCAO2_PADE, 2>), grid, blk, 0, stream, a);
-    return hipGetLastError();
-  }
-  if (variant != MOLE_VARIANT_LANE && sweep2_wavespec_eligible(a.sp)) {
-    // wave-specialised path: 64 walkers per 256-thread workgroup
-    const dim3 grid((a.W + 63) / 64), blk(256);
-    constexpr int T = 6;
-    if (he)
-      hipLaunchKernelGGL((sweep2_ws_kernel<MOLE_WF_HELIUM_PADE, 1, T>), grid, blk, 0, stream, a);
-    else if (nn == 1)
-      hipLaunchKernelGGL((sweep2_ws_kernel<MOLE_WF_LCAO2_PADE, 1, T>), grid, blk, 0, stream, a);
-    else
-      hipLaunchKernelGGL((sweep2_ws_kernel<MOLE_WF_LCAO2_PADE, 2, T>), grid, blk, 0, stream, a);
-    return hipGetLastError();
-  }
   const int bt = block_threads ? block_threads : 64;
+  if (sweep2_wavespec_eligible(a.sp)) {
+    if (he)
+      launch_spec<MOLE_WF_HELIUM_PADE, 1>(a, variant, bt, cus, stream);
+    else if (a.sp.n_nuc == 1)
+      launch_spec<MOLE_WF_LCAO2_PADE, 1>(a, variant, bt, cus, stream);
+    else
+      launch_spec<MOLE_WF_LCAO2_PADE, 2>(a, variant, bt, cus, stream);
+    return hipGetLastError();
+  }
   const dim3 grid((a.W + bt - 1) / bt);
   if (he)
     hipLaunchKernelGGL((sweep2_lane_kernel<MOLE_WF_HELIUM_PADE>), grid, dim3(bt), 0, stream, a);

@@ -52,6 +52,17 @@ def test_device_sqrt_and_division_are_correctly_rounded():
     assert np.array_equal(bits(M.debug_math(M.DEBUG_DIV, a, b)), bits(a / b))
 
 
+def test_chain_root_is_correctly_rounded_in_its_range():
+    rng = np.random.default_rng(4)
+    m = rng.uniform(1, 2, 200000)
+    sq = rng.integers(1, 1 << 26, 50000).astype(np.float64)
+    a = np.concatenate([rng.uniform(0, 400, 400000), m * 2.0 ** rng.integers(-767, 1000, m.size), sq * sq,
+                        np.nextafter(sq * sq, np.inf), np.nextafter(sq * sq, 0.0), [2.0 ** -767, 1.0, 4.0]])
+    assert np.array_equal(bits(M.debug_math(M.DEBUG_SQRT_NORMAL, a)), bits(np.sqrt(a)))
+    # outside it the caller's range test sees NaN or a small argument
+    assert np.all(np.isnan(M.debug_math(M.DEBUG_SQRT_NORMAL, np.array([0.0, np.inf, np.nan]))))
+
+
 def test_device_u64_maps_match_oracle():
     L = O.lib()
     rng = np.random.default_rng(2)
@@ -160,6 +171,51 @@ def test_variants_agree_on_split_sweeps(make):
             assert s0[k] == s1[k], k
         for k in ("sum_o", "sum_oe", "sum_oo"):
             assert np.array_equal(r0[k], r1[k]), k
+
+
+@pytest.mark.parametrize("W,position", [(8191, 6), (8193, 7), (16385, 6), (32769, 9)])
+@pytest.mark.parametrize("make", [M.h2, M.helium], ids=["h2", "he"])
+def test_dispatch_edges_agree_with_the_one_lane_kernel(make, W, position):
+    # walker counts on both sides of each automatic choice (32, 64 and 128
+    # walkers per CU on 256 CUs), last workgroups nearly empty, draws that
+    # start inside a Philox block
+    res = []
+    for variant in (M.VARIANT_LANE, M.VARIANT_AUTO):
+        with M.Context([make(W)], seed=21, step=0.5, block_size=4) as ctx:
+            ctx.set_launch_config(variant)
+            ctx.init_walkers()
+            ctx.set_stream(2, position)
+            ctx.sweep(3)
+            ctx.sweep(6, sample=True)
+            res.append((ctx.get_configs(), ctx.stats(), ctx.sr_sums()))
+    (c0, s0, r0), (c1, s1, r1) = res
+    assert np.array_equal(bits(c0), bits(c1)) and s0 == s1
+    assert all(np.array_equal(r0[k], r1[k]) for k in r0)
+
+
+@pytest.mark.parametrize("variant", [M.VARIANT_LANE, M.VARIANT_WAVESPEC, M.VARIANT_QUAD])
+@pytest.mark.parametrize("kind,zeta,side", [("he", 1.6875, 1e-200), ("he", 1.6875, 1e-130), ("he", 1.6875, 1e-100),
+                                            ("h2", 1.0, 1e-200), ("he", 300.0, 0.5), ("h2", 500.0, 0.5)])
+def test_moves_outside_the_fast_paths_match_oracle(kind, zeta, side, variant):
+    # distances that underflow to zero or to tiny squares, and psi^2 that
+    # underflows: the moves are evaluated by the full roots and divisions
+    W, steps, B = 40, 12, 4
+    gsys, owf = _systems(kind, W, (zeta, 0.5, 0.3))
+    cfg = np.zeros((W, 6))
+    if kind == "h2":
+        cfg[:, 2], cfg[:, 5] = 0.7, -0.7  # an electron on each nucleus
+    if side == 0.5:
+        cfg += np.random.default_rng(1).uniform(-1, 1, cfg.shape)
+    with M.Context([gsys], seed=3, step=side, block_size=B, flags=M.FLAG_TRACE, record_sweeps=steps) as ctx:
+        ctx.set_launch_config(variant)
+        ctx.set_configs(cfg)
+        ctx.set_stream(0, 6)
+        ctx.run(steps)
+        masks, _ = ctx.trace(steps, steps - B)
+        got = ctx.get_configs()
+    ref = O.run_box(owf, seed=3, walkers=W, steps=steps, block_size=B, box_side=side, cfg=cfg, pos0=6)
+    assert np.array_equal(masks, ref["accept_mask"])
+    assert np.array_equal(bits(got), bits(ref["cfg"]))
 
 
 @pytest.mark.parametrize("conv", [M.O_LOGDERIV, M.O_REFERENCE])
