@@ -5,12 +5,15 @@
 //   f_i = 0 from the first negative rho on, var with n - 1 (statfor.rs:86-88),
 // so effective sample counts need no copy of the series to the host.
 //
-// One 256-thread workgroup per walker.  The series is staged in LDS; the
-// mean and the variance are sums in sample order on thread 0; thread i - 1
-// forms rho_i as one sum in sample order (a lag per thread, every sum the
-// reference's sequential fold), and thread 0 then adds them in lag order.
-// Compiled with -ffp-contract=off, the result equals the CPU fold bit for
-// bit.
+// tau_tile_kernel (series that fit a workgroup's LDS, from 2,048 walkers on): a
+// workgroup takes 16 walkers, their series side by side in LDS; a lane takes
+// one walker and 8 neighbouring lags, whose partners it slides through
+// registers (two LDS reads for 8 products), and the lags are taken in passes
+// of 8 per lane group, ending when every walker's sum has met its first
+// negative rho.  Every sum is the reference's sequential fold on one lane.
+// tau_corr_kernel (the rest): one 256-thread workgroup per walker, a lag
+// per thread, all lags.  Compiled with -ffp-contract=off, both results equal
+// the CPU fold bit for bit.
 #include <hip/hip_runtime.h>
 
 #include "../../include/mole_gpu.h"
@@ -23,6 +26,149 @@ namespace {
 constexpr int kTauThreads = 256;
 constexpr int kTauMaxLag = 200;
 constexpr int kTauLdsSamples = 8192;  // series up to this length are staged in LDS
+constexpr int kTauTileMinWalkers = 2048;
+constexpr int kTauTileSamples = 1000;  // 16 of them, and a pass's lags, within a CU's 160 KiB
+
+// Bound: the serial mean and variance of a workgroup (one lane per walker),
+// then FP64 issue, a multiply and an add per product.  The sum stops at the
+// first negative rho, so lags past the last walker's cut are not formed: with
+// all 200 lags, a thread each and two LDS reads per product, 65,536 walkers x
+// 400 samples took 1,610 us a call (LDS-bound); this kernel takes 420 with 32
+// groups of 4 lags (565 with 8 of 8, 455 with 16 of 8, 526 with 64 of 2: the
+// fewer lags per lane, the shorter the fold that a workgroup waits for, the
+// more LDS reads per product).  16 walkers per workgroup: few enough that one
+// slow walker does not hold many others' lanes, and series up to 1,000 samples
+// fit the LDS.
+constexpr int kTileWalkers = 16, kTileStride = 17, kTilePad = 8;
+
+__host__ __device__ constexpr size_t tau_tile_lds(int n, int lags_per_pass) {
+  return sizeof(double) * ((size_t)(n + kTilePad) * kTileStride + (size_t)(lags_per_pass + 1) * kTileWalkers);
+}
+
+template <int GROUPS, int LAGS>
+__global__ void __launch_bounds__(GROUPS * kTileWalkers) tau_tile_kernel(const double *trace_e, int W, size_t cap,
+                                                                         size_t first, int n, double *tau_out) {
+  extern __shared__ double lds[];
+  double *y = lds;                                            // [n + pad][stride]
+  double *corr = y + (size_t)(n + kTilePad) * kTileStride;    // [lags of a pass][walker]
+  double *stat = corr + GROUPS * LAGS * kTileWalkers;    // mean, then 0 / 1: the walker's sum is complete
+  constexpr int kThreads = GROUPS * kTileWalkers, kPass = GROUPS * LAGS;
+  const int tid = threadIdx.x, wl = tid % kTileWalkers, g = tid / kTileWalkers;
+  const int w0 = blockIdx.x * kTileWalkers;
+  const int nw = min(kTileWalkers, W - w0);
+  // GROUPS consecutive samples of a walker per lane group, eight loads of a
+  // lane in flight; absent walkers of the last workgroup repeat the first
+  {
+    const int r = tid / GROUPS, t0 = tid % GROUPS;
+    const double *src = trace_e + (size_t)(w0 + (r < nw ? r : 0)) * cap + first;
+    double *o = y + r;
+    int t = t0;
+    for (; t + 7 * GROUPS < n; t += 8 * GROUPS) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = src[t + u * GROUPS];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) o[(t + u * GROUPS) * kTileStride] = v[u];
+    }
+    for (; t < n; t += GROUPS) o[t * kTileStride] = src[t];
+  }
+  for (int e = tid; e < kTilePad * kTileStride; e += kThreads) y[n * kTileStride + e] = 0.0;
+  __syncthreads();
+  // mean and variance: one sequential sum per walker, the next batch's reads
+  // ahead of this batch's additions
+  auto fold = [&](auto term) {
+    const double *yt = y + tid;
+    double sum = 0.0, v[8], nv[8];
+    int t = 0;
+    if (n >= 8) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = yt[u * kTileStride];
+      for (; t + 8 <= n; t += 8) {
+        // rows past n + pad - 1 are not read: the last batch's prefetch stays
+        // within the padding
+        const int tn = t + 16 <= n + kTilePad ? t + 8 : t;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) nv[u] = yt[(tn + u) * kTileStride];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum += term(v[u]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = nv[u];
+      }
+    }
+    for (; t < n; ++t) sum += term(yt[t * kTileStride]);
+    return sum;
+  };
+  if (tid < kTileWalkers) stat[tid] = fold([](double x) { return x; }) / (double)n;
+  __syncthreads();
+  {
+    const double mean = stat[wl];
+    for (int t = g; t < n; t += GROUPS) y[t * kTileStride + wl] = y[t * kTileStride + wl] - mean;
+  }
+  __syncthreads();
+  if (tid < kTileWalkers) stat[tid] = fold([](double d) { return d * d; }) / (double)(n - 1);
+  __syncthreads();
+  const double var = stat[wl];
+  const int max_i = kTauMaxLag < n - 1 ? kTauMaxLag : n - 1;
+  const double *yw = y + wl;
+  double tau = 1.0;     // threads 0..15: the walker's sum
+  bool done = tid >= kTileWalkers;
+  for (int i0 = 0; i0 < max_i; i0 += kPass) {
+    // lags b + 1 .. b + LAGS of this lane; rows past n are never used
+    const int b = i0 + g * LAGS;
+    double c[LAGS], v[LAGS];
+#pragma unroll
+    for (int j = 0; j < LAGS; ++j) c[j] = 0.0;
+    const int full = n - (b + LAGS);  // t below it: all LAGS products
+    int t = 0;
+    if (full >= 8) {
+#pragma unroll
+      for (int j = 0; j < LAGS; ++j) v[j] = yw[(b + 1 + j) * kTileStride];
+      for (; t + 8 <= full; t += 8) {
+        double a[8], nv[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          a[u] = yw[(t + u) * kTileStride];
+          nv[u] = yw[(t + u + b + 1 + LAGS) * kTileStride];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+#pragma unroll
+          for (int j = 0; j < LAGS; ++j) {
+            const double yj = u + j < LAGS ? v[u + j < LAGS ? u + j : 0] : nv[u + j < LAGS ? 0 : u + j - LAGS];
+            c[j] += a[u] * yj;
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < LAGS; ++j) v[j] = nv[8 - LAGS + j];
+      }
+    }
+    for (; t < n - (b + 1); ++t) {
+      const double a = yw[t * kTileStride];
+#pragma unroll
+      for (int j = 0; j < LAGS; ++j)
+        if (t + b + 1 + j < n) c[j] += a * yw[(t + b + 1 + j) * kTileStride];
+    }
+#pragma unroll
+    for (int j = 0; j < LAGS; ++j)
+      if (b + 1 + j <= max_i) corr[(g * LAGS + j) * kTileWalkers + wl] = c[j] / (var * (double)(n - (b + 1 + j)));
+    __syncthreads();
+    if (!done) {
+      // the terms in lag order up to the first negative one (its factor f
+      // and all later ones are 0; a NaN is not negative and is added)
+      const int k1 = min(kPass, max_i - i0);
+      for (int k = 0; k < k1; ++k) {
+        const double r = corr[k * kTileWalkers + tid];
+        if (r < 0.0) {
+          done = true;
+          break;
+        }
+        tau += 2.0 * r;
+      }
+    }
+    if (__syncthreads_and(done)) break;
+  }
+  if (tid < nw) tau_out[w0 + tid] = tau > 1.0 ? tau : 1.0;
+}
 
 template <bool LDS>
 __global__ void __launch_bounds__(kTauThreads) tau_corr_kernel(const double *trace_e, size_t cap, size_t first, int n,
@@ -82,11 +228,31 @@ __global__ void __launch_bounds__(kTauThreads) tau_corr_kernel(const double *tra
   }
 }
 
+template <int GROUPS, int LAGS>
+hipError_t launch_tile(const double *trace_e, int W, size_t cap, size_t first, int n, double *tau_out,
+                       hipStream_t stream) {
+  const size_t bytes = tau_tile_lds(n, GROUPS * LAGS);
+  if (bytes > 65536) {
+    // more than the default 64 KiB of dynamic LDS needs an opt-in per kernel
+    const hipError_t e = hipFuncSetAttribute((const void *)(tau_tile_kernel<GROUPS, LAGS>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((tau_tile_kernel<GROUPS, LAGS>), dim3((unsigned)((W + kTileWalkers - 1) / kTileWalkers)),
+                     dim3(GROUPS * kTileWalkers), bytes, stream, trace_e, W, cap, first, n, tau_out);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t launch_tau_corr(const double *trace_e, int W, size_t cap, size_t first, int n, double *tau_out,
                            hipStream_t stream) {
   if (W <= 0) return hipSuccess;
+  // Below 2,048 walkers a workgroup per walker has the chip to itself and its
+  // lag-parallel fold is the shorter one (500 walkers x 400 samples: 52 against
+  // 60 us a call; 4,096: 149 against 89).
+  if (W >= kTauTileMinWalkers && n <= kTauTileSamples)
+    return launch_tile<32, 4>(trace_e, W, cap, first, n, tau_out, stream);
   if (n <= kTauLdsSamples)
     hipLaunchKernelGGL(tau_corr_kernel<true>, dim3(W), dim3(kTauThreads), sizeof(double) * n, stream, trace_e, cap,
                        first, n, tau_out);

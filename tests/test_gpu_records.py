@@ -118,3 +118,24 @@ def test_tau_int_on_device_matches_oracle_fold():
 
 def bits(a):
     return np.asarray(a, dtype=np.float64).view(np.uint64)
+
+
+@pytest.mark.parametrize("W", [2047, 2049])
+def test_tau_int_tiles_match_oracle_fold(W):
+    # both sides of the walker rule, a last tile of one walker, series lengths
+    # at the edges of the unrolled folds, of a pass of lags (128) and of the
+    # LDS rule (1,000), and slowly mixing walkers that need a second pass
+    from oracle import oracle_ffi as O
+
+    cap = 1001
+    with M.Context([M.helium(W)], seed=6, step=0.15, block_size=10, flags=M.FLAG_TRACE, record_sweeps=cap) as ctx:
+        ctx.init_walkers()
+        ctx.sweep(cap, sample=True)
+        _, el = ctx.trace(cap, cap)
+        L = O.lib()
+        picks = sorted({0, 1, 15, 16, 17, W - 17, W - 2, W - 1})
+        for first, n in [(0, 2), (5, 3), (0, 8), (3, 9), (0, 16), (1, 17), (0, 129), (2, 130), (0, 137), (7, 400),
+                         (1, 1000), (0, 1001)]:
+            tau = ctx.tau_int(n, first=first)
+            want = [L.orc_tau_corr(O.dptr(np.ascontiguousarray(el[w, first:first + n])), n) for w in picks]
+            assert np.array_equal(bits(tau[picks]), bits(want)), (first, n)
