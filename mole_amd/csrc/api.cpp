@@ -300,8 +300,6 @@ void fill_sys2(SysState &st, const mole_system_desc &d) {
   sp.c = d.params[2];
 }
 
-int default_lanes(int N) { return N <= 4 ? 4 : N <= 10 ? 8 : N <= 20 ? 16 : 32; }
-
 mole_status check_ctx(mole_ctx *ctx, uint32_t sys) {
   if (!ctx) return fail(MOLE_ERR_INVALID_ARGUMENT, "null context");
   if (sys >= ctx->sys.size()) return fail(MOLE_ERR_INVALID_ARGUMENT, "system index %u out of range", sys);
@@ -344,6 +342,18 @@ int sj_prop(const mole_ctx *ctx) {
                                                       : kSJPropBox;
 }
 
+// LDS bytes of a workgroup of system s at L lanes per walker.
+size_t sj_footprint(const mole_ctx *ctx, const SysState &s, int L, int tsize) {
+  return sj_lds_per_group(s.n_nuc) +
+         (size_t)(64 / L) * sj_lds_per_walker((int)s.N, (int)s.n_up, (int)s.n_down, s.n_nuc, s.n_basis, tsize,
+                                              (int)s.params.size(), sj_prop(ctx));
+}
+
+int sj_default_lanes(const mole_ctx *ctx, const SysState &s) {
+  if (ctx->run.proposal == MOLE_PROPOSAL_LEARNED) return 4;
+  return s.N <= 4 ? 4 : s.N <= 10 ? 8 : s.N <= 20 ? 16 : 32;
+}
+
 // Tiles of 64/L walkers grouped by LDS footprint class (4 KiB steps, the
 // largest class first), most expensive first within a group
 // (longest-processing-time order, so the tail of each launch is short
@@ -355,13 +365,13 @@ mole_status sj_build_tiles(mole_ctx *ctx) {
   for (size_t s = 0; s < ctx->sys.size(); ++s) {
     SysState &st = ctx->sys[s];
     st.lds_walker = sj_lds_per_walker((int)st.N, (int)st.n_up, (int)st.n_down, st.n_nuc, st.n_basis,
-                                      sj_tsize(ctx), (int)st.params.size());
+                                      sj_tsize(ctx), (int)st.params.size(), sj_prop(ctx));
     const int wpt = 64 / st.L;
-    lds = std::max(lds, (size_t)wpt * st.lds_walker);
+    const size_t fp = sj_footprint(ctx, st, st.L, sj_tsize(ctx));
+    lds = std::max(lds, fp);
     const int nmax = (int)std::max(st.n_up, st.n_down);
     const double per_walker = (double)st.N * (st.N + st.n_nuc + st.n_basis + (double)nmax * st.n_basis +
                                                (double)nmax * nmax);
-    const size_t fp = (size_t)wpt * st.lds_walker;
     for (int w0 = 0; w0 < st.W; w0 += wpt)
       tiles.push_back({{(int)s, w0, std::min(wpt, st.W - w0)}, per_walker / st.L, fp});
   }
@@ -778,7 +788,6 @@ mole_status mole_ctx_create(const mole_system_desc *sys, uint32_t n_sys, const m
       S.n_basis = (int)d.n_basis;
       S.n_orb = (int)d.n_orbitals;
       S.v_nn = nuclear_repulsion(d.nuclei_xyz, d.nuclei_charge, d.n_nuclei);
-      S.L = run->proposal == MOLE_PROPOSAL_LEARNED ? 4 : default_lanes((int)S.N);
       S.n_cols = sj_columns((int)d.n_params);
     }
   }
@@ -843,6 +852,7 @@ mole_status mole_ctx_create(const mole_system_desc *sys, uint32_t n_sys, const m
         tab.push_back(d.n_params == (uint32_t)kSJNParam ? d.params[5] * d.basis_exponent[m] : d.basis_exponent[m]);
       for (uint32_t m = 0; m < d.n_basis; ++m)
         for (uint32_t k = 0; k < d.n_orbitals; ++k) tab.push_back(d.orbital_coeff[(size_t)k * d.n_basis + m]);
+      tab.insert(tab.end(), kSJCoefPad, 0.0);
       // centres, then the basis kinds (MOLE_BASIS_*)
       std::vector<int> cen(d.basis_center, d.basis_center + d.n_basis);
       for (uint32_t m = 0; m < d.n_basis; ++m) cen.push_back(d.basis_kind ? (int)d.basis_kind[m] : MOLE_BASIS_STO);
@@ -865,6 +875,7 @@ mole_status mole_ctx_create(const mole_system_desc *sys, uint32_t n_sys, const m
     CTX_TRY(hipMalloc(&ctx->d_sysdev, sizeof(SJSysDev) * n_sys));
     CTX_TRY(hipMalloc(&ctx->d_state, sizeof(SJLaunchState)));
     if (sj_push_state(ctx) != MOLE_OK) return bail(MOLE_ERR_DEVICE);
+    for (SysState &S : ctx->sys) S.L = sj_default_lanes(ctx, S);
     mole_status ts = sj_build_tiles(ctx);
     if (ts != MOLE_OK) return bail(ts);
   }
@@ -1287,10 +1298,12 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
   if (n > ((size_t)1 << 28)) return fail(MOLE_ERR_SHAPE, "mole_eval: at most 2^28 configurations per call");
   // evaluated in FP64 whatever the context's precision (Function::value and
   // its derivatives at given configurations, no update chain to save)
-  const size_t lds_walker = sj_lds_per_walker((int)s.N, (int)s.n_up, (int)s.n_down, s.n_nuc, s.n_basis, 8, (int)np);
-  if ((size_t)wpt * lds_walker > ctx->lds_limit)
+  const size_t lds_walker =
+      sj_lds_per_walker((int)s.N, (int)s.n_up, (int)s.n_down, s.n_nuc, s.n_basis, 8, (int)np, kSJPropBox);
+  const size_t lds = sj_lds_per_group(s.n_nuc) + (size_t)wpt * lds_walker;
+  if (lds > ctx->lds_limit)
     return fail(MOLE_ERR_UNSUPPORTED, "mole_eval: %zu B of LDS per workgroup at %d lanes per walker (limit %zu)",
-                (size_t)wpt * lds_walker, s.L, ctx->lds_limit);
+                lds, s.L, ctx->lds_limit);
   const size_t n_tiles = (n + wpt - 1) / wpt;
   // one allocation of doubles: positions, inverses (8 bytes per element for
   // either precision), accumulators, determinants, then the outputs
@@ -1351,7 +1364,7 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
       a.ext = 1;
       a.one_wave = 0;
       a.cap_sweeps = a.cap_samples = 0;
-      e = launch_sj(a, (int)n_tiles, 0, kSJPropBox, (size_t)wpt * lds_walker, ctx->stream);
+      e = launch_sj(a, (int)n_tiles, 0, kSJPropBox, lds, ctx->stream);
     }
     auto back = [&](double *host, size_t off, size_t cnt) {
       if (e == hipSuccess && host)
@@ -1495,7 +1508,7 @@ mole_status mole_set_walker_lanes(mole_ctx *ctx, uint32_t sys, uint32_t lanes) {
     return fail(MOLE_ERR_UNSUPPORTED, "the learned proposal runs 16 walkers of 4 lanes per wave");
   SysState &s = ctx->sys[sys];
   const int old = s.L;
-  s.L = lanes ? (int)lanes : (ctx->run.proposal == MOLE_PROPOSAL_LEARNED ? 4 : default_lanes((int)s.N));
+  s.L = lanes ? (int)lanes : sj_default_lanes(ctx, s);
   HIP_TRY(hipSetDevice(ctx->device));
   HIP_TRY(hipStreamSynchronize(ctx->stream));
   st = sj_build_tiles(ctx);

@@ -33,22 +33,10 @@ __device__ __forceinline__ double basis_value(int kind, double z, double d0, dou
   return e;
 }
 
-// Value v, gradient (g0, g1, g2) and laplacian l.
-template <bool GTO>
-__device__ __forceinline__ void basis_vgl(int kind, double z, double d0, double d1, double d2, double r, double &v,
-                                          double &g0, double &g1, double &g2, double &l) {
-  if (GTO && kind == MOLE_BASIS_GTO) {
-    const double r2 = r * r;
-    v = exp_m(-z * r2);
-    const double gf = -2.0 * z * v;
-    g0 = gf * d0;
-    g1 = gf * d1;
-    g2 = gf * d2;
-    l = v * (4.0 * z * z * r2 - 6.0 * z);
-    return;
-  }
-  const double e = exp_m(-z * r);
-  const double ir = 1.0 / r;  // one division
+// The same of an STO from e = exp(-z r) and ir = 1/r, which the functions of
+// one shell share.
+__device__ __forceinline__ void basis_vgl_sto(int kind, double z, double d0, double d1, double d2, double e, double ir,
+                                              double &v, double &g0, double &g1, double &g2, double &l) {
   const double gf = (-z * e) * ir;
   if (kind >= MOLE_BASIS_STO_PX) {
     const int q = kind - MOLE_BASIS_STO_PX;
@@ -70,6 +58,25 @@ __device__ __forceinline__ void basis_vgl(int kind, double z, double d0, double 
   }
 }
 
+// Value v, gradient (g0, g1, g2) and laplacian l.
+template <bool GTO>
+__device__ __forceinline__ void basis_vgl(int kind, double z, double d0, double d1, double d2, double r, double &v,
+                                          double &g0, double &g1, double &g2, double &l) {
+  if (GTO && kind == MOLE_BASIS_GTO) {
+    const double r2 = r * r;
+    v = exp_m(-z * r2);
+    const double gf = -2.0 * z * v;
+    g0 = gf * d0;
+    g1 = gf * d1;
+    g2 = gf * d2;
+    l = v * (4.0 * z * z * r2 - 6.0 * z);
+    return;
+  }
+  const double e = exp_m(-z * r);
+  const double ir = 1.0 / r;  // one division
+  basis_vgl_sto(kind, z, d0, d1, d2, e, ir, v, g0, g1, g2, l);
+}
+
 // Gradient only (the drift): as basis_vgl's gradient.
 template <bool GTO>
 __device__ __forceinline__ void basis_grad(int kind, double z, double d0, double d1, double d2, double r, double &g0,
@@ -82,7 +89,9 @@ __device__ __forceinline__ void basis_grad(int kind, double z, double d0, double
 // [1/2, 1) in magnitude by frexp after every product (exact), so products of
 // many ratios neither overflow nor underflow.  log|det| = log|mant| + ex ln 2
 // with ln 2 split as in log_m; a zero mantissa (a singular block) gives -inf.
-__device__ __forceinline__ double logdet_value(double mant, double ex) {
+// Out of line: inlined, the sweep kernels hold log's constants in registers
+// (3 % on the atoms).
+static __device__ __noinline__ double logdet_value(double mant, double ex) {
   if (mant == 0.0) return -__builtin_inf();
   const double kLn2Hi = 6.93147180369123816490e-01;
   const double kLn2Lo = 1.90821492927058770002e-10;

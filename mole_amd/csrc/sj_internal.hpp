@@ -146,7 +146,12 @@ struct SJArgs {
   int n_tiles;             // persistent launch: tiles in `tiles`
 };
 
-size_t sj_lds_per_walker(int N, int nu, int nd, int nn, int K, int tsize, int np);
+// LDS bytes of one walker (prop: SJProposal) and of what a workgroup shares.
+size_t sj_lds_per_walker(int N, int nu, int nd, int nn, int K, int tsize, int np, int prop);
+size_t sj_lds_per_group(int nn);
+// Doubles read past the end of the coefficient table (register chunks of the
+// local energy): the host pads it.
+constexpr int kSJCoefPad = 8;
 
 // Draws start at draw_base + D N sweeps_done (D draws per move of the
 // proposal) and moves at move_base + N sweeps_done for every system; sample

@@ -3,13 +3,20 @@
 // re-inversion in FP64, and the local energy after sampled sweeps.
 //
 // A workgroup is one wave.  It owns 64/L walkers of one system (a tile);
-// the L lanes of a walker split every stage of a move -- distances and
-// Jastrow terms over electrons and nuclei, basis functions, orbitals,
-// Sherman-Morrison columns and matrix elements -- and the walker's state
-// (positions, inverse Slater matrices, scratch) lives in LDS for the whole
-// launch, read from and written to HBM once.  Every sum is formed by the
-// walker's sub-lane 0 in a fixed sequential order, so results do not depend
-// on L and equal those of a sequential evaluation bit for bit.
+// the L lanes of a walker split the parallel stages of a move -- Jastrow terms
+// over electrons and nuclei, basis functions, orbitals, Sherman-Morrison
+// columns and rows -- and a walker's positions, inverse Slater matrices and
+// stage arrays live in LDS for the whole launch, read from and written to HBM
+// once.  Every sum is formed in a fixed sequential order, so results do not
+// depend on L and equal those of a sequential evaluation bit for bit.
+//
+// What bounds the kernel is the number of instructions a wave issues: a stage
+// costs the same whether one or all of a walker's lanes take part.  So the
+// serial parts (sums, decision) run on all lanes alike, which needs no
+// broadcast; stages that need no exchange share a phase; and the LDS a walker
+// holds is kept small (stage arrays, re-inversion and local-energy scratch
+// overlap; counters and determinants in registers; sample sums in HBM), so
+// that few lanes per walker still leave two waves per SIMD.
 //
 // Math (per move of electron i of spin s, column c; B = A_s^-1 with
 // A_s[c][k] = phi_k(r_c)):
@@ -27,94 +34,91 @@
 
 namespace mole {
 
-// LDS layout of one walker (bytes); identical on host and device.
+// LDS layout (bytes); identical on host and device.  Per walker:
+//   pos | B | draws of the sweep | scratch
+// scratch: the stage arrays of a move, or a Gauss-Jordan re-inversion; the
+// local energy's per-electron results take the draws and the scratch together
+// (no draw is pending after a sweep).  Per workgroup, ahead of the walkers:
+// the nuclei (x, y, z, -a Z) and the factor pairs of the sample sums.
 struct SJLayout {
-  uint32_t pos, B, rng, rn, chi, phin, jn, jo, f, scr, flag, mv, acc, ld, bytes;
-  __host__ __device__ SJLayout(int N, int nu, int nd, int nn, int K, int tsize, int np) {
-    const int nmax = nu > nd ? nu : nd;
-    uint32_t o = 0;
-    auto take = [&](uint32_t n_bytes) {
-      const uint32_t at = o;
-      o += (n_bytes + 7u) & ~7u;
-      return at;
-    };
-    pos = take(24u * N);
-    B = take((uint32_t)tsize * (nu * nu + nd * nd));
-    rng = take(32u * N);
-    rn = take(8u * (nn > 0 ? nn : 1));
-    chi = take(8u * K);
-    phin = take(8u * nmax);
-    jn = take(8u * (N + nn));
-    jo = take(8u * (N + nn));
-    f = take(8u * nmax);
-    // scratch: Gauss-Jordan (2 n^2 + n), per-electron local-energy results
-    // ((3 + np) N), drift pieces (3K + 3n + 3(N + n_nuc))
-    const uint32_t lu = 8u * (2u * nmax * nmax + nmax);
-    const uint32_t el = 8u * ((3u + (uint32_t)np) * N);
-    const uint32_t dr = 8u * (3u * K + 3u * nmax + 3u * (N + nn));
-    const uint32_t sc = lu > el ? lu : el;
-    scr = take(sc > dr ? sc : dr);
-    flag = take(16u);
-    mv = take(64u);  // proposed position and drift (Gaussian proposals)
-    acc = take(8u * sj_columns(np));
-    ld = take(8u * kSJLdColumns);  // directly after acc: addressed as acc + sj_columns(np)
+  uint32_t pos, B, rng, scr, mv, chi, phin, jn, jo, dots, gch, og, jg, le, bytes;
+  __host__ __device__ SJLayout(int N, int nu, int nd, int nn, int K, int tsize, int np, int prop) {
+    const uint32_t n = nu > nd ? nu : nd, M = N + nn;
+    auto up = [](uint32_t x) { return (x + 7u) & ~7u; };
+    pos = 0;
+    B = pos + 24u * N;
+    rng = B + up((uint32_t)tsize * (nu * nu + nd * nd));
+    scr = rng + 32u * N;
+    // a move's stages
+    mv = scr;  // proposed position and drift (Gaussian proposals)
+    chi = mv + (prop == kSJPropBox ? 0u : 64u);
+    phin = chi + 8u * K;
+    jn = phin + up(tsize * n);
+    jo = jn + up(tsize * M);
+    dots = jo + up(tsize * M);
+    gch = dots + up(tsize * n);
+    og = gch + (prop == kSJPropDiffuse ? 24u * K : 0u);
+    jg = og + (prop == kSJPropDiffuse ? 24u * n : 0u);
+    uint32_t end = jg + (prop == kSJPropDiffuse ? 24u * M : 0u);
+    // Gauss-Jordan: A, then I and the pivot column (the basis values while A is built)
+    const uint32_t second = n * n + n > (uint32_t)K ? n * n + n : (uint32_t)K;
+    const uint32_t lu = scr + 8u * (n * n + second);
+    end = end > lu ? end : lu;
+    // per-electron local-energy results, then (1, E, d ln psi/dp)
+    le = rng;
+    const uint32_t el = le + 8u * ((3u + (uint32_t)np) * N + 8u);
+    end = end > el ? end : el;
     // the walkers of a tile sit bytes apart; an odd number of 8-byte words
     // puts the same field of consecutive walkers in different LDS banks
     // (an even count maps many walkers of a wave onto one bank)
-    bytes = ((o / 8u) % 2u == 0u) ? o + 8u : o;
+    bytes = ((end / 8u) % 2u == 0u) ? end + 8u : end;
   }
 };
 
-__host__ size_t sj_lds_per_walker(int N, int nu, int nd, int nn, int K, int tsize, int np) {
-  return SJLayout(N, nu, nd, nn, K, tsize, np).bytes;
+// (a, b) of sample sum q, packed a | b << 4: the sum gains v[a] v[b] with v =
+// (1, E, O_0 .. O_np-1); q = 0, 1 are columns kSJSumE, kSJSumE2, the rest
+// follow from kSJSumO on (O, O E, upper triangle of O O^T).
+__host__ __device__ constexpr int sj_sample_sums(int np) { return 2 + 2 * np + np * (np + 1) / 2; }
+constexpr uint32_t kSJPairBytes = (sj_sample_sums(kSJNParam) + 7) / 8 * 8;
+__host__ __device__ constexpr uint32_t sj_lds_shared(int nn) { return kSJPairBytes + 32u * (uint32_t)nn; }
+
+__host__ size_t sj_lds_per_walker(int N, int nu, int nd, int nn, int K, int tsize, int np, int prop) {
+  return SJLayout(N, nu, nd, nn, K, tsize, np, prop).bytes;
 }
+__host__ size_t sj_lds_per_group(int nn) { return sj_lds_shared(nn); }
 
 namespace {
 
+// Orders LDS accesses of a one-wave workgroup: the wave's LDS operations
+// execute in program order, so only the compiler has to keep it.
+__device__ __forceinline__ void sync_wave() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <typename T>
 struct SJWalker {
-  double *pos, *rng, *rn, *chi, *scr, *flag, *mv;
-  T *Bup, *Bdn, *phin, *jn, *jo, *f;
+  double *pos, *rng, *scr, *chi, *mv, *le;
+  T *Bup, *Bdn, *phin, *jn, *jo, *dots;
 };
 
-__device__ __forceinline__ double pade_pair(double b, double c, double r) {
-  return (b * r) / (1.0 + c * r);
-}
-
-// e-e term between electron i at r and electron j at x (T precision)
+// Jastrow term num r/(1 + c r) of the points x and q, r = |x - q| (T
+// precision): electron pairs with num = b, nuclei with num = -a Z, c = d.
 template <typename T>
-__device__ __forceinline__ T pair_term(double b, double c, const double *r, const double *x);
+__device__ __forceinline__ T jastrow_term(T num, T c, const double *x, const double *q);
 template <>
-__device__ __forceinline__ double pair_term<double>(double b, double c, const double *r, const double *x) {
-  const double rij = norm3(r[0] - x[0], r[1] - x[1], r[2] - x[2]);
-  return pade_pair(b, c, rij);
+__device__ __forceinline__ double jastrow_term<double>(double num, double c, const double *x, const double *q) {
+  const double r = norm3(x[0] - q[0], x[1] - q[1], x[2] - q[2]);
+  return (num * r) / (1.0 + c * r);
 }
 template <>
-__device__ __forceinline__ float pair_term<float>(double b, double c, const double *r, const double *x) {
-  const float d0 = (float)(r[0] - x[0]), d1 = (float)(r[1] - x[1]), d2 = (float)(r[2] - x[2]);
-  float q = d0 * d0;
-  q = q + d1 * d1;
-  q = q + d2 * d2;
-  const float rij = sqrtf(q);
-  return ((float)b * rij) / (1.0f + (float)c * rij);
-}
-
-// e-n term of an electron at r and nucleus R with aZ = a Z_I (T precision)
-template <typename T>
-__device__ __forceinline__ T en_term(double aZ, double d, const double *r, const double *R);
-template <>
-__device__ __forceinline__ double en_term<double>(double aZ, double d, const double *r, const double *R) {
-  const double rI = norm3(r[0] - R[0], r[1] - R[1], r[2] - R[2]);
-  return -(aZ * rI) / (1.0 + d * rI);
-}
-template <>
-__device__ __forceinline__ float en_term<float>(double aZ, double d, const double *r, const double *R) {
-  const float d0 = (float)(r[0] - R[0]), d1 = (float)(r[1] - R[1]), d2 = (float)(r[2] - R[2]);
-  float q = d0 * d0;
-  q = q + d1 * d1;
-  q = q + d2 * d2;
-  const float rI = sqrtf(q);
-  return -((float)aZ * rI) / (1.0f + (float)d * rI);
+__device__ __forceinline__ float jastrow_term<float>(float num, float c, const double *x, const double *q) {
+  const float d0 = (float)(x[0] - q[0]), d1 = (float)(x[1] - q[1]), d2 = (float)(x[2] - q[2]);
+  float s = d0 * d0;
+  s = s + d1 * d1;
+  s = s + d2 * d2;
+  const float r = sqrtf(s);
+  return (num * r) / (1.0f + c * r);
 }
 
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return fma(a, b, c); }
@@ -124,26 +128,43 @@ __device__ __forceinline__ float fma_t(float a, float b, float c) { return fmaf(
 // lies at least 1/(2n) from an integer, far beyond the rounding error.
 __device__ __forceinline__ int small_div(int e, float inv_n) { return (int)(((float)e + 0.5f) * inv_n); }
 
-// Basis values chi[m] of the point r into LDS (lanes over nuclei, then over
-// basis functions).  gto/pk: Gaussians / p-type STOs may occur (otherwise
-// every function is an s-type STO and the kinds are not read).  Ends with a
-// barrier.
-__device__ __forceinline__ void basis_to_lds(const SJSysDev &S, const double *r, double *rn, double *chi,
-                                             int t, int L, bool gto, bool pk) {
-  for (int I = t; I < S.n_nuc; I += L)
-    rn[I] = norm3(r[0] - S.nuc[3 * I], r[1] - S.nuc[3 * I + 1], r[2] - S.nuc[3 * I + 2]);
-  __syncthreads();
-  for (int m = t; m < S.n_basis; m += L) {
+// The first basis function a lane evaluates (m = t), kept in registers: with
+// as many lanes as functions the sweep reads no basis table.  (Eight orbital
+// coefficients kept the same way cost 2-3 % in spills.)
+struct SJLaneBasis {
+  double zeta, R[3];
+  int kind;
+  __device__ __forceinline__ void load(const SJSysDev &S, int t) {
+    const int m = t < S.n_basis ? t : 0;
+    zeta = S.zeta[m];
+    kind = S.kind[m];
     const int I = S.center[m];
-    const double rr = rn[I];
-    if (gto || pk) {
-      const double *R = S.nuc + 3 * I;
-      chi[m] = basis_value<true>(S.kind[m], S.zeta[m], r[0] - R[0], r[1] - R[1], r[2] - R[2], rr);
-    } else {
-      chi[m] = exp_m(-S.zeta[m] * rr);
-    }
+    for (int q = 0; q < 3; ++q) R[q] = S.nuc[3 * I + q];
   }
-  __syncthreads();
+};
+
+// Basis values chi[m] of the point r into LDS (lanes over basis functions, each
+// with its own centre's distance).  gto/pk: Gaussians / p-type STOs may occur
+// (otherwise every function is an s-type STO).  rn (optional): the distances
+// by function.  No barrier.
+__device__ __forceinline__ void basis_to_lds(const SJSysDev &S, const SJLaneBasis &lb, const double *r, double *chi,
+                                             int t, int L, bool gto, bool pk) {
+  double z = lb.zeta, R0 = lb.R[0], R1 = lb.R[1], R2 = lb.R[2];
+  int kd = lb.kind;
+  for (int m = t;;) {
+    if (m >= S.n_basis) break;
+    const double d0 = r[0] - R0, d1 = r[1] - R1, d2 = r[2] - R2;
+    const double rr = norm3(d0, d1, d2);
+    chi[m] = (gto || pk) ? basis_value<true>(kd, z, d0, d1, d2, rr) : exp_m(-z * rr);
+    m += L;
+    if (m >= S.n_basis) break;
+    const int I = S.center[m];
+    z = S.zeta[m];
+    kd = S.kind[m];
+    R0 = S.nuc[3 * I];
+    R1 = S.nuc[3 * I + 1];
+    R2 = S.nuc[3 * I + 2];
+  }
 }
 
 // Sequential sums whose loads are issued U at a time ahead of the
@@ -204,7 +225,31 @@ __device__ __forceinline__ double orbital_value(const SJSysDev &S, int k, const 
   return phi;
 }
 
-// What a re-inversion of one spin block found (valid on sub-lane 0).
+// The draws of one Gaussian move at stream position q.  Out of line: inlined,
+// the constants of log, sin and cos are kept in registers across the sweeps
+// and push the moves' own state into scratch memory.
+struct SJGauss {
+  double z0, z1, z2, u;
+};
+__device__ __noinline__ SJGauss gauss_draws(uint64_t q, uint32_t k0, uint32_t k1, uint32_t walker, uint32_t epoch) {
+  Stream st;
+  st.init((uint64_t)k0 | ((uint64_t)k1 << 32), 0, walker, epoch);
+  const uint64_t d0 = st.draw(q), d1 = st.draw(q + 1), d2 = st.draw(q + 2), d3 = st.draw(q + 3), d4 = st.draw(q + 4);
+  SJGauss g;
+  double z3;
+  box_muller(d0, d1, &g.z0, &g.z1);
+  box_muller(d2, d3, &g.z2, &z3);
+  g.u = u64_standard(d4);
+  return g;
+}
+
+// A walker's counters and determinants, the same on all its lanes.
+struct SJBooks {
+  double ld[4];     // (mantissa, exponent) of det A_up, det A_dn
+  double cond, drift, singular;
+};
+
+// What a re-inversion of one spin block found (on every lane).
 struct SJRefresh {
   double cond;      // ||A||_1 ||A^-1||_1
   double mant, ex;  // det A = mant 2^ex (mant = 0: singular)
@@ -216,69 +261,64 @@ struct SJRefresh {
 // pivots (the row swaps' signs times their product, carried as mant 2^ex).
 // A pivot |p| <= n 2^-52 ||A||_1 (or NaN) marks the block singular: its
 // division is skipped (the row is zeroed), so the inverse stays finite and
-// the determinant reads 0.  All lanes of the workgroup must call it.
+// the determinant reads 0.  All lanes of the workgroup must call it; the
+// norms and the pivot search run on every lane alike.
 template <typename T>
-__device__ SJRefresh refresh_spin(const SJSysDev &S, SJWalker<T> &wk, int s, int t, int L, bool gto, bool pk,
-                                  bool write_B) {
+__device__ __forceinline__ SJRefresh refresh_spin(const SJSysDev &S, const SJLaneBasis &lb, SJWalker<T> &wk, int s,
+                                                  int t, int L, bool gto, bool pk, bool write_B) {
   SJRefresh res{1.0, 1.0, 0.0, false};
   const int n = s == 0 ? S.n_up : S.n_dn;
   if (n == 0) return res;
   const int first = s == 0 ? 0 : S.n_up;
   T *B = s == 0 ? wk.Bup : wk.Bdn;
-  double *M = wk.scr, *I = wk.scr + n * n, *colp = wk.scr + 2 * n * n;
+  double *M = wk.scr, *I = wk.scr + n * n, *colp = wk.scr + 2 * n * n, *chi = I;
+  sync_wave();
   for (int c = 0; c < n; ++c) {
-    basis_to_lds(S, wk.pos + 3 * (first + c), wk.rn, wk.chi, t, L, gto, pk);
-    for (int k = t; k < n; k += L) M[c * n + k] = orbital_value(S, k, wk.chi);
-    __syncthreads();
+    basis_to_lds(S, lb, wk.pos + 3 * (first + c), chi, t, L, gto, pk);
+    sync_wave();
+    for (int k = t; k < n; k += L) M[c * n + k] = orbital_value(S, k, chi);
+    sync_wave();
   }
   double anorm = 0.0;
-  if (t == 0)
-    for (int k = 0; k < n; ++k) {
-      double cs = 0.0;
-      for (int c = 0; c < n; ++c) cs += fabs(M[c * n + k]);
-      anorm = cs > anorm ? cs : anorm;
-    }
+  for (int k = 0; k < n; ++k) {
+    double cs = 0.0;
+    for (int c = 0; c < n; ++c) cs += fabs(M[c * n + k]);
+    anorm = cs > anorm ? cs : anorm;
+  }
   const double thresh = anorm * ((double)n * 0x1p-52);
   const float inv_n = 1.0f / (float)n;
   for (int e = t; e < n * n; e += L) I[e] = (e == small_div(e, inv_n) * (n + 1)) ? 1.0 : 0.0;
-  __syncthreads();
+  sync_wave();
   for (int p = 0; p < n; ++p) {
-    if (t == 0) {
-      int piv = p;
-      for (int r = p + 1; r < n; ++r)
-        if (fabs(M[r * n + p]) > fabs(M[piv * n + p])) piv = r;
-      const double pv = M[piv * n + p];
-      const bool bad = !(fabs(pv) > thresh);
-      if (bad) {
-        res.singular = true;
-      } else {
-        if (piv != p) res.mant = -res.mant;
-        logdet_mul(res.mant, res.ex, pv);
+    int piv = p;
+    double pv = M[p * n + p];
+    for (int r = p + 1; r < n; ++r) {
+      const double v = M[r * n + p];
+      if (fabs(v) > fabs(pv)) {
+        piv = r;
+        pv = v;
       }
-      wk.flag[0] = (double)piv;
-      wk.flag[1] = bad ? 1.0 : 0.0;
     }
-    __syncthreads();
-    const int piv = (int)wk.flag[0];
-    const bool bad = wk.flag[1] != 0.0;
-    if (piv != p)
-      for (int j = t; j < n; j += L) {
-        double tm = M[p * n + j];
-        M[p * n + j] = M[piv * n + j];
-        M[piv * n + j] = tm;
-        tm = I[p * n + j];
-        I[p * n + j] = I[piv * n + j];
-        I[piv * n + j] = tm;
-      }
-    __syncthreads();
-    const double ip = bad ? 0.0 : 1.0 / M[p * n + p];
-    __syncthreads();
+    const bool bad = !(fabs(pv) > thresh);
+    if (bad) {
+      res.singular = true;
+    } else {
+      if (piv != p) res.mant = -res.mant;
+      logdet_mul(res.mant, res.ex, pv);
+    }
+    sync_wave();
+    const double ip = bad ? 0.0 : 1.0 / pv;
+    // rows p and piv swapped, row p scaled
     for (int j = t; j < n; j += L) {
-      M[p * n + j] = M[p * n + j] * ip;
-      I[p * n + j] = I[p * n + j] * ip;
+      const double mp = M[p * n + j], mv = M[piv * n + j], ap = I[p * n + j], av = I[piv * n + j];
+      M[piv * n + j] = mp;
+      I[piv * n + j] = ap;
+      M[p * n + j] = mv * ip;
+      I[p * n + j] = av * ip;
     }
+    sync_wave();
     for (int r = t; r < n; r += L) colp[r] = M[r * n + p];
-    __syncthreads();
+    sync_wave();
     // row p's own column entry was just scaled; colp[p] is unused
     for (int e = t; e < n * n; e += L) {
       const int r = small_div(e, inv_n), j = e - r * n;
@@ -286,18 +326,17 @@ __device__ SJRefresh refresh_spin(const SJSysDev &S, SJWalker<T> &wk, int s, int
       M[e] = fma(-colp[r], M[p * n + j], M[e]);
       I[e] = fma(-colp[r], I[p * n + j], I[e]);
     }
-    __syncthreads();
+    sync_wave();
   }
   if (write_B)
     for (int e = t; e < n * n; e += L) B[e] = (T)I[e];
   double bnorm = 0.0;
-  if (t == 0)
-    for (int c = 0; c < n; ++c) {
-      double cs = 0.0;
-      for (int k = 0; k < n; ++k) cs += fabs(I[k * n + c]);
-      bnorm = cs > bnorm ? cs : bnorm;
-    }
-  __syncthreads();
+  for (int c = 0; c < n; ++c) {
+    double cs = 0.0;
+    for (int k = 0; k < n; ++k) cs += fabs(I[k * n + c]);
+    bnorm = cs > bnorm ? cs : bnorm;
+  }
+  sync_wave();
   res.cond = anorm * bnorm;
   if (res.singular) {
     res.mant = 0.0;
@@ -306,30 +345,29 @@ __device__ SJRefresh refresh_spin(const SJSysDev &S, SJWalker<T> &wk, int s, int
   return res;
 }
 
-// Re-inverts both spin blocks and keeps the books on sub-lane 0: with count,
-// the condition maximum and the singular blocks; the log-determinant state
-// when ld_mode is 1 (taken from the re-inversion) or 2 (the same, after
-// recording how far the value the updates carried drifted from it).
+// Re-inverts both spin blocks and keeps the books: with count, the condition
+// maximum and the singular blocks; the log-determinant state when ld_mode is 1
+// (taken from the re-inversion) or 2 (the same, after recording how far the
+// value the updates carried drifted from it).
 template <typename T>
-__device__ void refresh_walker(const SJSysDev &S, SJWalker<T> &wk, double *acc, int t, int L, bool gto, bool pk,
-                               bool write_B, bool count, int ld_mode) {
-  double *ld = acc + sj_columns(5 + S.opt_exp);
+__device__ __forceinline__ void refresh_walker(const SJSysDev &S, const SJLaneBasis &lb, SJWalker<T> &wk, SJBooks &bk,
+                                               int t, int L, bool gto, bool pk, bool write_B, bool count,
+                                               int ld_mode) {
 #pragma unroll 1
   for (int q = 0; q < 2; ++q) {
-    const SJRefresh r = refresh_spin<T>(S, wk, q, t, L, gto, pk, write_B);
-    if (t == 0) {
-      if (count) {
-        acc[kSJCondMax] = fmax(acc[kSJCondMax], r.cond);
-        if (r.singular) acc[kSJSingular] += 1.0;
-      }
-      if (ld_mode == 2 && !r.singular && ld[2 * q] != 0.0) {
-        const double carried = logdet_value(ld[2 * q], ld[2 * q + 1]);
-        acc[kSJLdDrift] = fmax(acc[kSJLdDrift], fabs(carried - logdet_value(r.mant, r.ex)));
-      }
-      if (ld_mode) {
-        ld[2 * q] = r.mant;
-        ld[2 * q + 1] = r.ex;
-      }
+    const SJRefresh r = refresh_spin<T>(S, lb, wk, q, t, L, gto, pk, write_B);
+    if (count) {
+      bk.cond = fmax(bk.cond, r.cond);
+      if (r.singular) bk.singular += 1.0;
+    }
+    const double m = q ? bk.ld[2] : bk.ld[0], e = q ? bk.ld[3] : bk.ld[1];
+    if (ld_mode == 2 && !r.singular && m != 0.0)
+      bk.drift = fmax(bk.drift, fabs(logdet_value(m, e) - logdet_value(r.mant, r.ex)));
+    if (ld_mode) {
+      bk.ld[0] = q ? bk.ld[0] : r.mant;
+      bk.ld[1] = q ? bk.ld[1] : r.ex;
+      bk.ld[2] = q ? r.mant : bk.ld[2];
+      bk.ld[3] = q ? r.ex : bk.ld[3];
     }
   }
 }
@@ -339,9 +377,9 @@ __device__ void refresh_walker(const SJSysDev &S, SJWalker<T> &wk, double *acc, 
 // and forms each electron's kinetic term (orbital gradients and laplacians
 // as fma chains over the basis, contracted with the inverse column; Jastrow
 // gradient and laplacian over partners, electrons then nuclei), potential and
-// parameter derivatives in registers; sub-lane 0 adds the electrons' results
-// in electron order.  Every sum has a fixed order, so the result does not
-// depend on L.  One barrier per call; returns on sub-lane 0.
+// parameter derivatives in registers; the electrons' results are then added in
+// electron order.  Every sum has a fixed order, so the result does not depend
+// on L.
 constexpr int kSJLanesNMax = 8;  // orbitals per register chunk
 
 // The pieces of the local energy the operator terms need (sub-lane 0).
@@ -352,7 +390,7 @@ struct SJParts {
 };
 
 // sum_k coef_k term_k of one operator (terms as the C ABI defines them).
-__device__ double operator_value(const mole_operator &op, const SJParts &P, const SJSysDev &S, const double *pos) {
+__device__ __noinline__ double operator_value(const mole_operator &op, SJParts P, const SJSysDev &S, const double *pos) {
   const int N = S.N;
   double v = 0.0;
   for (uint32_t k = 0; k < op.n_terms; ++k) {
@@ -452,52 +490,78 @@ __device__ __noinline__ void sj_compat_sample(const SJSysDev &S, const double *l
 }
 
 // g_out (extended kernel, optional): grad_i ln psi of every electron, written
-// by the lane that takes the electron as g_out[3 i + q].
+// by the lane that takes the electron as g_out[3 i + q].  Returns the energy
+// on every lane and leaves (1, E, d ln psi/dp) at the end of wk.le, whose
+// address is *vec.
 template <typename T, bool EXT>
-__device__ double local_energy(const SJSysDev &S, SJWalker<T> &wk, int t, int L, double *dl,
-                               SJParts *parts = nullptr, double *g_out = nullptr) {
+__device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &wk, int t, int L, double **vec,
+                                               SJParts &parts, double *g_out) {
   const int N = S.N, K = S.n_basis, nn = S.n_nuc, no = S.n_orb;
   const double bA = S.p[0], bP = S.p[1], c = S.p[2], a = S.p[3], d = S.p[4];
   // [N][RS]: kinetic term, potential, five Jastrow derivatives, e-e potential
   // (EXT), exponent-scale derivative (with the scale); RS = 3 + np
-  double *res = wk.scr;
+  double *res = wk.le;
   const int RS = 8 + S.opt_exp;
-  SJParts own;
+  const bool kinds = (EXT && S.any_gto) || S.any_p;
+  sync_wave();
   for (int i = t; i < N; i += L) {
     const int s = i < S.n_up ? 0 : 1;
     const int cc = s == 0 ? i : i - S.n_up;
     const int n = s == 0 ? S.n_up : S.n_dn;
     const T *B = s == 0 ? wk.Bup : wk.Bdn;
-    const double *xi = wk.pos + 3 * i;
+    const double xi[3] = {wk.pos[3 * i], wk.pos[3 * i + 1], wk.pos[3 * i + 2]};
     // orbitals in register chunks of kCh; the basis values are recomputed
     // per chunk (bit-identical each time), and the chunks add in orbital
     // order, so the width does not change the sums.  The extended
     // instantiations (DMC, operators, Gaussians) carry more live state and
-    // take 6, which keeps their spills down (scratch 240 -> 176 bytes per
-    // lane in the mixed-precision DMC step).
+    // take 6, which keeps their spills down.  Coefficients past the last
+    // orbital are read (the table is padded) and their chains not used.
     constexpr int kCh = EXT ? 6 : kSJLanesNMax;
     double Dg0 = 0.0, Dg1 = 0.0, Dg2 = 0.0, Dl = 0.0;
+#pragma unroll 1
     for (int k0 = 0; k0 < n; k0 += kCh) {
       double og[kCh][4];
 #pragma unroll
       for (int k = 0; k < kCh; ++k) og[k][0] = og[k][1] = og[k][2] = og[k][3] = 0.0;
+      // consecutive functions of one centre share its displacement, distance
+      // and 1/r, and those of one shell the exponential (a p shell's three)
+      int Ip = -1;
+      double zp = 0.0, d0 = 0.0, d1 = 0.0, d2 = 0.0, r = 0.0, ir = 0.0, e = 0.0;
+      bool have_e = false;
+#pragma unroll 1
       for (int m = 0; m < K; ++m) {
         const int I = S.center[m];
-        const double d0 = xi[0] - S.nuc[3 * I], d1 = xi[1] - S.nuc[3 * I + 1], d2 = xi[2] - S.nuc[3 * I + 2];
-        const double r = norm3(d0, d1, d2);
-        const int kd = ((EXT && S.any_gto) || S.any_p) ? S.kind[m] : MOLE_BASIS_STO;
+        const double z = S.zeta[m];
+        const int kd = kinds ? S.kind[m] : MOLE_BASIS_STO;
+        if (I != Ip) {
+          d0 = xi[0] - S.nuc[3 * I];
+          d1 = xi[1] - S.nuc[3 * I + 1];
+          d2 = xi[2] - S.nuc[3 * I + 2];
+          r = norm3(d0, d1, d2);
+          ir = 1.0 / r;
+          Ip = I;
+          have_e = false;
+        }
         double ch, g0, g1, g2, lc;
-        basis_vgl<EXT>(kd, S.zeta[m], d0, d1, d2, r, ch, g0, g1, g2, lc);
+        if (EXT && kd == MOLE_BASIS_GTO) {
+          basis_vgl<true>(kd, z, d0, d1, d2, r, ch, g0, g1, g2, lc);
+        } else {
+          if (!have_e || z != zp) {
+            e = exp_m(-z * r);
+            zp = z;
+            have_e = true;
+          }
+          basis_vgl_sto(kd, z, d0, d1, d2, e, ir, ch, g0, g1, g2, lc);
+        }
         const double *cm = S.coef_t + (size_t)m * no + k0;
 #pragma unroll
-        for (int k = 0; k < kCh; ++k)
-          if (k0 + k < n) {
-            const double cv = cm[k];
-            og[k][0] = fma(cv, g0, og[k][0]);
-            og[k][1] = fma(cv, g1, og[k][1]);
-            og[k][2] = fma(cv, g2, og[k][2]);
-            og[k][3] = fma(cv, lc, og[k][3]);
-          }
+        for (int k = 0; k < kCh; ++k) {
+          const double cv = cm[k];
+          og[k][0] = fma(cv, g0, og[k][0]);
+          og[k][1] = fma(cv, g1, og[k][1]);
+          og[k][2] = fma(cv, g2, og[k][2]);
+          og[k][3] = fma(cv, lc, og[k][3]);
+        }
       }
 #pragma unroll
       for (int k = 0; k < kCh; ++k)
@@ -510,9 +574,10 @@ __device__ double local_energy(const SJSysDev &S, SJWalker<T> &wk, int t, int L,
         }
     }
     // exponent scale s: sum_m zeta_m d ln psi / d zeta_m of electron i's row
-    const double ez = S.opt_exp ? exponent_scale_term<T, EXT>(S, B, n, cc, xi) : 0.0;
+    const double ez = S.opt_exp ? exponent_scale_term<T, EXT>(S, B, n, cc, wk.pos + 3 * i) : 0.0;
     double gJ0 = 0.0, gJ1 = 0.0, gJ2 = 0.0, lJ = 0.0;
     double Vi = 0.0, Vee = 0.0, e0 = 0.0, e1 = 0.0, e2 = 0.0, e3 = 0.0, e4 = 0.0;
+#pragma unroll 1
     for (int j = 0; j < N; ++j) {
       if (j == i) continue;
       const double *xj = wk.pos + 3 * j;
@@ -541,6 +606,7 @@ __device__ double local_energy(const SJSysDev &S, SJWalker<T> &wk, int t, int L,
         e2 += (-b * r * r) * iden2;
       }
     }
+#pragma unroll 1
     for (int I = 0; I < nn; ++I) {
       const double d0 = xi[0] - S.nuc[3 * I], d1 = xi[1] - S.nuc[3 * I + 1], d2 = xi[2] - S.nuc[3 * I + 2];
       const double r = norm3(d0, d1, d2);
@@ -578,68 +644,83 @@ __device__ double local_energy(const SJSysDev &S, SJWalker<T> &wk, int t, int L,
     if constexpr (EXT) o[7] = Vee;
     if (S.opt_exp) o[8] = ez;
   }
-  __syncthreads();
-  double kin = 0.0, V = 0.0;
-  for (int q = 0; q < kSJNParam; ++q) dl[q] = 0.0;
-  if (t == 0) {
-    for (int i = 0; i < N; ++i) {
-      const double *o = res + RS * i;
-      kin += o[0];
-      V += o[1];
-      for (int q = 0; q < 5; ++q) dl[q] += o[2 + q];
-      if (S.opt_exp) dl[5] += o[8];
+  sync_wave();
+  // sums over electrons, in electron order: lane q forms component q into
+  // electron 0's slot (kinetic, potential, derivatives)
+  for (int q = t; q < RS; q += L) {
+    if (!EXT && q == 7) continue;
+    double sum = 0.0;
+    int i = 0;
+    for (; i + 4 <= N; i += 4) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = res[RS * (i + u) + q];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sum += v[u];
     }
-    // d ln psi / d s = (1/s) sum_m zeta_m d ln psi / d zeta_m
-    if (S.opt_exp) dl[5] = dl[5] / S.p[5];
-    if (S.hamiltonian != MOLE_H_ELECTRONIC) {
-      V = 0.0;
-      for (int i = 0; i < N; ++i)
-        for (int I = 0; I < nn; ++I) {
-          const double *xi = wk.pos + 3 * i;
-          V += -S.charge[I] / norm3(xi[0] - S.nuc[3 * I], xi[1] - S.nuc[3 * I + 1], xi[2] - S.nuc[3 * I + 2]);
-        }
-    }
-    if (EXT && parts) parts->kin = kin;
-    if (EXT && (S.custom_h || S.n_obs)) {
-      if (!parts) parts = &own;
-      parts->kin = kin;
-      double vee = 0.0, ven = 0.0;
-      for (int i = 0; i < N; ++i) vee += res[RS * i + 7];
-      // IonicPotential::value's order: ions outer, electrons inner
-      for (int I = 0; I < nn; ++I)
-        for (int i = 0; i < N; ++i) {
-          const double *xi = wk.pos + 3 * i;
-          ven -= S.charge[I] / norm3(xi[0] - S.nuc[3 * I], xi[1] - S.nuc[3 * I + 1], xi[2] - S.nuc[3 * I + 2]);
-        }
-      parts->vee = vee;
-      parts->ven = ven;
-    }
+    for (; i < N; ++i) sum += res[RS * i + q];
+    res[q] = sum;
   }
-  __syncthreads();
-  if (EXT && t == 0 && S.custom_h) return operator_value(S.ops[0], *parts, S, wk.pos);
-  return -0.5 * kin + V + S.v_nn;
+  sync_wave();
+  const double kin = res[0];
+  double V = res[1];
+  double *v = res + RS * N;  // (1, E, O)
+  double *dl = v + 2;
+  if (t == 0) {
+    v[0] = 1.0;
+    for (int q = 0; q < 5; ++q) dl[q] = res[2 + q];
+    // d ln psi / d s = (1/s) sum_m zeta_m d ln psi / d zeta_m
+    if (S.opt_exp) dl[5] = res[8] / S.p[5];
+  }
+  if (S.hamiltonian != MOLE_H_ELECTRONIC) {
+    V = 0.0;
+    for (int i = 0; i < N; ++i)
+      for (int I = 0; I < nn; ++I) {
+        const double *xi = wk.pos + 3 * i;
+        V += -S.charge[I] / norm3(xi[0] - S.nuc[3 * I], xi[1] - S.nuc[3 * I + 1], xi[2] - S.nuc[3 * I + 2]);
+      }
+  }
+  parts.kin = kin;
+  double E = -0.5 * kin + V + S.v_nn;
+  if (EXT && (S.custom_h || S.n_obs)) {
+    double ven = 0.0;
+    // IonicPotential::value's order: ions outer, electrons inner
+    for (int I = 0; I < nn; ++I)
+      for (int i = 0; i < N; ++i) {
+        const double *xi = wk.pos + 3 * i;
+        ven -= S.charge[I] / norm3(xi[0] - S.nuc[3 * I], xi[1] - S.nuc[3 * I + 1], xi[2] - S.nuc[3 * I + 2]);
+      }
+    parts.vee = res[7];
+    parts.ven = ven;
+    if (S.custom_h) E = operator_value(S.ops[0], parts, S, wk.pos);
+  }
+  if (t == 0) v[1] = E;
+  *vec = v;
+  sync_wave();
+  return E;
 }
 
 // Pieces of grad_i ln psi at r for the drift-diffusion proposal, FP64
 // (metrop.rs:153-155).  Basis gradients into gch[3m + q] (lanes over basis
-// functions; chi and rn of r must be in LDS) and the Jastrow gradient terms
+// functions; chi of r by the same lane) and the Jastrow gradient terms
 // of electron i at r into jg[3j + q] (lanes over partners, i's slot zero).
 // No barrier.
 __device__ __forceinline__ void drift_terms(const SJSysDev &S, const double *pos, int i, const double *r,
-                                            const double *rn, const double *chi, double *gch, double *jg,
-                                            int t, int L, bool gto, bool pk) {
+                                            const double *chi, double *gch, double *jg, int t, int L, bool gto,
+                                            bool pk) {
   for (int m = t; m < S.n_basis; m += L) {
     const int I = S.center[m];
     const double d0 = r[0] - S.nuc[3 * I], d1 = r[1] - S.nuc[3 * I + 1], d2 = r[2] - S.nuc[3 * I + 2];
+    const double rr = norm3(d0, d1, d2);
     const int kd = (gto || pk) ? S.kind[m] : MOLE_BASIS_STO;
     if (kd == MOLE_BASIS_STO) {
       // chi[m] = exp(-z r) is in LDS; basis_vgl's operations
-      const double gf = (-S.zeta[m] * chi[m]) * (1.0 / rn[I]);
+      const double gf = (-S.zeta[m] * chi[m]) * (1.0 / rr);
       gch[3 * m] = gf * d0;
       gch[3 * m + 1] = gf * d1;
       gch[3 * m + 2] = gf * d2;
     } else {
-      basis_grad<true>(kd, S.zeta[m], d0, d1, d2, rn[I], gch[3 * m], gch[3 * m + 1], gch[3 * m + 2]);
+      basis_grad<true>(kd, S.zeta[m], d0, d1, d2, rr, gch[3 * m], gch[3 * m + 1], gch[3 * m + 2]);
     }
   }
   const int N = S.N, si = i < S.n_up ? 0 : 1;
@@ -692,8 +773,8 @@ __device__ __forceinline__ void orbital_gradients(const SJSysDev &S, int n, cons
   }
 }
 
-// Sub-lane 0: g = sum_k og_k B[k][c] (chains in k order) + sum_j jg_j (in j
-// order), each as in the CPU restatement.
+// g = sum_k og_k B[k][c] (chains in k order) + sum_j jg_j (in j order), each as
+// in the CPU restatement, on every lane.
 template <typename T>
 __device__ __forceinline__ void drift_sum(const double *og, const T *B, int n, int c, const double *jg, int M,
                                           double det_scale, double g[3]) {
@@ -735,7 +816,7 @@ template <typename T, int PROP, bool EXT>
 __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsigned char *lds) {
   constexpr int DPM = sj_draws_per_move(PROP);
   const SJSysDev &S = a.systems[tile.sys];
-  const int N = S.N, nu = S.n_up, nd = S.n_dn, L = S.L, W = S.W;
+  const int N = S.N, nu = S.n_up, nd = S.n_dn, L = S.L, W = S.W, nn = S.n_nuc;
   const int lane = threadIdx.x;
   // learned proposal: 16 walkers of 4 lanes, walker s on lanes s, s+16,
   // s+32, s+48 (the sample columns of the MFMA tiles); otherwise L
@@ -746,56 +827,87 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
   const int lg_slots = __ffs(nslots) - 1;  // nslots is a power of two
   const bool live = slot < tile.nw;
   const int w = tile.w0 + slot;
-  const int np = 5 + S.opt_exp, ncol = sj_columns(np);
-  const SJLayout lay(N, nu, nd, S.n_nuc, S.n_basis, (int)sizeof(T), np);
-  unsigned char *base = lds + (size_t)slot * lay.bytes;
+  const int np = 5 + S.opt_exp;
+  const SJLayout lay(N, nu, nd, nn, S.n_basis, (int)sizeof(T), np, PROP);
+  // shared by the workgroup: the sample sums' factor pairs, the nuclei
+  uint8_t *pairs = lds;
+  double *nuc = (double *)(lds + kSJPairBytes);
+  unsigned char *walkers = lds + sj_lds_shared(nn);
+  unsigned char *base = walkers + (size_t)slot * lay.bytes;
   SJWalker<T> wk;
   wk.pos = (double *)(base + lay.pos);
   wk.Bup = (T *)(base + lay.B);
   wk.Bdn = wk.Bup + nu * nu;
   wk.rng = (double *)(base + lay.rng);
-  wk.rn = (double *)(base + lay.rn);
+  wk.scr = (double *)(base + lay.scr);
+  wk.mv = (double *)(base + lay.mv);
   wk.chi = (double *)(base + lay.chi);
   wk.phin = (T *)(base + lay.phin);
   wk.jn = (T *)(base + lay.jn);
   wk.jo = (T *)(base + lay.jo);
-  wk.f = (T *)(base + lay.f);
-  wk.scr = (double *)(base + lay.scr);
-  wk.flag = (double *)(base + lay.flag);
-  wk.mv = (double *)(base + lay.mv);
-  const int nB = nu * nu + nd * nd;
+  wk.dots = (T *)(base + lay.dots);
+  wk.le = (double *)(base + lay.le);
+  const int nB = nu * nu + nd * nd, M = N + nn;
   const bool gto = EXT && S.any_gto;
   const bool pk = S.any_p != 0;
   // DMC steps move walkers the branching gathered: the log-determinant state
   // is not carried there (mole_dmc_diffuse recomputes it at its end)
-  const bool track_ld = !(EXT && a.dmc == kSJDmcStep);
+  const bool dmc_step = EXT && a.dmc == kSJDmcStep;
+  const bool track_ld = !dmc_step;
 
   // ---- state in (a DMC step reads the walkers the branching gathered) ----
-  const bool dmc_in = EXT && a.dmc == kSJDmcStep;
-  const double *pin = dmc_in ? S.dmc_pos_in : S.pos;
-  const T *Bg = (const T *)(dmc_in ? S.dmc_B_in : S.B);
+  const double *pin = dmc_step ? S.dmc_pos_in : S.pos;
+  const T *Bg = (const T *)(dmc_step ? S.dmc_B_in : S.B);
   for (int e = lane; e < 3 * N * nslots; e += 64) {
     const int k = e >> lg_slots, sl = e & (nslots - 1);
-    double *pp = (double *)(lds + (size_t)sl * lay.bytes + lay.pos);
+    double *pp = (double *)(walkers + (size_t)sl * lay.bytes + lay.pos);
     pp[k] = (sl < tile.nw) ? pin[(size_t)k * W + tile.w0 + sl] : 0.0;
   }
   for (int e = lane; e < nB * nslots; e += 64) {
     const int k = e >> lg_slots, sl = e & (nslots - 1);
-    T *bb = (T *)(lds + (size_t)sl * lay.bytes + lay.B);
+    T *bb = (T *)(walkers + (size_t)sl * lay.bytes + lay.B);
     bb[k] = (sl < tile.nw) ? Bg[(size_t)k * W + tile.w0 + sl] : (T)0;
   }
-  // accumulators: LDS, touched by sub-lane 0 only
-  double *acc = (double *)(base + lay.acc);
-  if (t == 0) {
-    // DMC steps touch only the accepted-move count and the condition maximum
-    const bool dmc_step = EXT && a.dmc == kSJDmcStep;
-    for (int k = 0; k < ncol; ++k)
-      if (!dmc_step || k == kSJAccepted || k == kSJCondMax || k == kSJSingular)
-        acc[k] = live ? S.acc[(size_t)k * W + w] : 0.0;
-    if (track_ld)
-      for (int k = 0; k < kSJLdColumns; ++k) acc[ncol + k] = live ? S.ld[(size_t)k * W + w] : 1.0;
+  for (int I = lane; I < nn; I += 64) {
+    nuc[4 * I] = S.nuc[3 * I];
+    nuc[4 * I + 1] = S.nuc[3 * I + 1];
+    nuc[4 * I + 2] = S.nuc[3 * I + 2];
+    nuc[4 * I + 3] = -(S.p[3] * S.charge[I]);
   }
-  __syncthreads();
+  const int nsum = sj_sample_sums(np);
+  if (lane < nsum) {
+    // q = 0, 1: E, E^2; then O_k, O_k E, and the triangle O_k O_l row by row
+    int fa = lane == 0 ? 0 : 1, fb = 1;
+    if (lane >= 2 + 2 * np) {
+      int k = 0, e = lane - 2 - 2 * np;
+      while (e >= np - k) e -= np - k++;
+      fa = 2 + k;
+      fb = 2 + k + e;
+    } else if (lane >= 2) {
+      fa = lane < 2 + np ? 0 : 1;
+      fb = 2 + (lane - 2) % np;
+    }
+    pairs[lane] = (uint8_t)(fa | fb << 4);
+  }
+  SJLaneBasis lb;
+  lb.load(S, t);
+  SJBooks bk{{1.0, 0.0, 1.0, 0.0}, 0.0, 0.0, 0.0};
+  double block_sum = 0.0, acc_in = 0.0;
+  [[maybe_unused]] double dmc_el = 0.0, dmc_w = 0.0, dmc_eref = 0.0;
+  if (live) {
+    acc_in = S.acc[(size_t)kSJAccepted * W + w];
+    if (dmc_step) {
+      dmc_el = S.dmc_el_in[w];
+      dmc_w = S.dmc_w_in[w];
+      dmc_eref = *S.dmc_eref;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) bk.ld[k] = S.ld[(size_t)k * W + w];
+      block_sum = S.acc[(size_t)kSJBlockSum * W + w];
+    }
+  }
+  uint32_t n_acc = 0;
+  sync_wave();
 
   const uint32_t k0 = (uint32_t)a.seed, k1 = (uint32_t)(a.seed >> 32) ^ S.sys_index;
   if (a.init) {
@@ -807,313 +919,311 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
       wk.pos[2 * b] = u64_range(v0, 2.0, -3.0);
       if (2 * b + 1 < 3 * N) wk.pos[2 * b + 1] = u64_range(v1, 2.0, -3.0);
     }
-    __syncthreads();
-  }
-  if (a.init || a.refresh) {
-    // new configurations: the determinants are taken from the re-inversion
-    // (nothing accumulated to compare with); refresh 2 keeps the inverses
-    const bool wb = a.init || a.refresh == 1;
-    refresh_walker<T>(S, wk, acc, t, L, gto, pk, wb, wb, track_ld ? 1 : 0);
-  }
-  if (EXT && a.dmc == kSJDmcInit) {
-    // DmcRunner::new: weight 1; the local energy of the starting configuration
-    double dlg[kSJNParam];
-    const double E = local_energy<T, EXT>(S, wk, t, L, dlg);
-    if (t == 0 && live) {
-      S.dmc[w] = 1.0;
-      S.dmc[(size_t)W + w] = E;
-    }
-  }
-  if (EXT && a.dmc == kSJEval) {
-    // mole_eval: psi = sign exp(log|det up| + log|det dn| + J) from the
-    // re-inversion's determinants, d psi = psi grad ln psi, lap psi = psi
-    // sum_i lap_i psi/psi, E_L and d psi/dp = psi d ln psi/dp
-    double dlg[kSJNParam];
-    SJParts parts;
-    double *gw = (live && S.ev_grad) ? S.ev_grad + (size_t)w * 3 * N : nullptr;
-    const double E = local_energy<T, EXT>(S, wk, t, L, dlg, &parts, gw);
-    if (t == 0 && live) {
-      const double psi = sj_psi(S, acc + ncol, dlg);
-      if (S.ev_value) S.ev_value[w] = psi;
-      if (S.ev_lap) S.ev_lap[w] = psi * parts.kin;
-      if (S.ev_el) S.ev_el[w] = E;
-      if (S.ev_pgrad)
-        for (int k = 0; k < np; ++k) S.ev_pgrad[(size_t)w * np + k] = psi * dlg[k];
-      // the lanes' gradient stores precede local_energy's closing barrier
-      if (gw)
-        for (int k = 0; k < 3 * N; ++k) gw[k] = psi * gw[k];
-    }
+    sync_wave();
   }
   const uint32_t lu_period = a.lu_period;
-
   const SJLaunchState ls = *a.state;
   uint64_t p = S.draw_base + DPM * (uint64_t)N * ls.sweeps_done;
-  uint64_t m = S.move_base + (uint64_t)N * ls.sweeps_done;
+  const uint64_t m0 = S.move_base + (uint64_t)N * ls.sweeps_done;
+  // moves until the next re-inversion
+  uint32_t lu_left = lu_period ? lu_period - (uint32_t)(m0 % lu_period) : 0;
   uint32_t fill = ls.block_fill;
   uint32_t sidx = ls.trace_samples;
   const double inv_block = 1.0 / (double)a.block_size;
+  const T bA = (T)S.p[0], bP = (T)S.p[1], cee = (T)S.p[2], cen = (T)S.p[4];
+  // the pass before the first sweep re-inverts where the launch asks for it
+  // and takes the local energy of the configurations as they are (DMC's start,
+  // mole_eval); one copy of each stage serves it and the sweeps
+  const bool entry_refresh = a.init || a.refresh;
+  const bool entry_energy = EXT && (a.dmc == kSJDmcInit || a.dmc == kSJEval);
 
-  for (uint32_t sw = 0; sw < a.n_sweeps; ++sw) {
-    if constexpr (PROP == kSJPropBox) {
-      // ---- the sweep's draws: [p, p + 4N), lanes over Philox blocks ----
-      const uint64_t b0 = p >> 1, b1 = (p + 4 * (uint64_t)N - 1) >> 1;
-      for (uint64_t b = b0 + t; b <= b1; b += L) {
-        const u32x4 o = philox4x32_10({(uint32_t)b, (uint32_t)(b >> 32), (uint32_t)w, a.epoch}, k0, k1);
-        const uint64_t v[2] = {(uint64_t)o.x | ((uint64_t)o.y << 32), (uint64_t)o.z | ((uint64_t)o.w << 32)};
-        for (int h = 0; h < 2; ++h) {
-          const uint64_t q = 2 * b + h;
-          if (q < p || q >= p + 4 * (uint64_t)N) continue;
-          const int r = (int)(q - p);
-          wk.rng[r] = ((r & 3) == 3) ? u64_standard(v[h]) : u64_range(v[h], a.scale, a.offset);
-        }
-      }
-    } else {
-      // ---- Gaussian proposals: 6 draws per move, lanes over moves; Box-Muller
-      // of draws (0,1) and (2,3) -> z0, z1, z2; draw 4 -> the accept uniform
-      Stream st;
-      st.init(a.seed, S.sys_index, (uint32_t)w, a.epoch);
-      for (int i = t; i < N; i += L) {
-        const uint64_t q = p + 6 * (uint64_t)i;
-        const uint64_t d0 = st.draw(q), d1 = st.draw(q + 1), d2 = st.draw(q + 2), d3 = st.draw(q + 3);
-        const uint64_t d4 = st.draw(q + 4);
-        double z0, z1, z2, z3;
-        box_muller(d0, d1, &z0, &z1);
-        box_muller(d2, d3, &z2, &z3);
-        wk.rng[4 * i] = z0;
-        wk.rng[4 * i + 1] = z1;
-        wk.rng[4 * i + 2] = z2;
-        wk.rng[4 * i + 3] = u64_standard(d4);
-      }
-    }
-    __syncthreads();
-    uint64_t mask = 0;
-    for (int i = 0; i < N; ++i) {
-      const int s = i < nu ? 0 : 1;
-      const int c = s == 0 ? i : i - nu;
-      const int n = s == 0 ? nu : nd;
-      T *B = s == 0 ? wk.Bup : wk.Bdn;
-      const double *xi = wk.pos + 3 * i;
-      double xn[3];
-      double *gch = wk.scr, *og = wk.scr + 3 * S.n_basis, *jg = og + 3 * (nu > nd ? nu : nd);
+  for (uint32_t pass = entry_refresh || entry_energy ? 0u : 1u; pass <= a.n_sweeps; ++pass) {
+    const bool sweep = pass > 0;
+    const uint32_t sw = pass - 1;
+    if (sweep) {
       if constexpr (PROP == kSJPropBox) {
-        xn[0] = xi[0] + wk.rng[4 * i];
-        xn[1] = xi[1] + wk.rng[4 * i + 1];
-        xn[2] = xi[2] + wk.rng[4 * i + 2];
-      } else if constexpr (PROP == kSJPropLearned) {
-        // learned proposal: pass 0, the network at x -> (mu, ln sigma), x' =
-        // (x_i + mu) + sigma z; pass 1, the network at x' for the reverse
-        // density (all lanes run the MFMA passes).  One loop body keeps a
-        // single copy of the features and the network in the kernel's code.
-#pragma unroll 1
-        for (int pass = 0; pass < 2; ++pass) {
-          float fv[4];
-          mlp_features(wk.pos, N, S.nuc, S.n_nuc, i, pass == 0 ? xi : wk.mv, t, fv);
-          const f32x4 o = mlp_forward(a.net, features_bf16(fv), nullptr);
-          if (t == 0) {
-            const double ls = mlp_log_sigma((double)o[3]);
-            const double sg = exp_m(ls);
-            if (pass == 0) {
-              double z2 = 0.0;
-              for (int q = 0; q < 3; ++q) {
-                const double z = wk.rng[4 * i + q];
-                wk.mv[q] = (xi[q] + (double)o[q]) + sg * z;
-                z2 += z * z;
-              }
-              wk.mv[3] = -3.0 * ls - 0.5 * z2;  // log q(x'|x) + const
-            } else {
-              double e2 = 0.0;
-              for (int q = 0; q < 3; ++q) {
-                const double e = (xi[q] - wk.mv[q]) - (double)o[q];
-                e2 += e * e;
-              }
-              wk.mv[4] = (-3.0 * ls - e2 / (2.0 * sg * sg)) - wk.mv[3];  // log q(x|x') - log q(x'|x)
-            }
-          }
-          __syncthreads();
+        // ---- the sweep's draws: [p, p + 4N), lanes over Philox blocks ----
+        const uint64_t b0 = p >> 1;
+        const int odd = (int)(p & 1), n4 = 4 * N;
+        for (int b = t; 2 * b - odd < n4; b += L) {
+          const uint64_t bb = b0 + (uint64_t)b;
+          const u32x4 o = philox4x32_10({(uint32_t)bb, (uint32_t)(bb >> 32), (uint32_t)w, a.epoch}, k0, k1);
+          const uint64_t v0 = (uint64_t)o.x | ((uint64_t)o.y << 32), v1 = (uint64_t)o.z | ((uint64_t)o.w << 32);
+          const int r = 2 * b - odd;  // the first of the block's two draws
+          // (dx, dy, dz, u) per move: with an even start only second draws are u
+          const double d0 = odd && (r & 3) == 3 ? u64_standard(v0) : u64_range(v0, a.scale, a.offset);
+          const double d1 = !odd && (r & 3) == 2 ? u64_standard(v1) : u64_range(v1, a.scale, a.offset);
+          if (r >= 0) wk.rng[r] = d0;
+          if (r + 1 < n4) wk.rng[r + 1] = d1;
         }
-        xn[0] = wk.mv[0];
-        xn[1] = wk.mv[1];
-        xn[2] = wk.mv[2];
       } else {
-        // drift at x (metrop.rs:150-163): x' = (x_i + tau v) + sqrt(tau) z
-        basis_to_lds(S, xi, wk.rn, wk.chi, t, L, gto, pk);
-        drift_terms(S, wk.pos, i, xi, wk.rn, wk.chi, gch, jg, t, L, gto, pk);
-        __syncthreads();
-        orbital_gradients(S, n, gch, og, t, L);
-        __syncthreads();
-        if (t == 0) {
-          double v[3];
-          drift_sum<T>(og, B, n, c, jg, N + S.n_nuc, 1.0, v);
-          for (int q = 0; q < 3; ++q) {
-            wk.mv[3 + q] = v[q];
-            wk.mv[q] = (xi[q] + v[q] * a.tau) + a.sqrt_tau * wk.rng[4 * i + q];
-          }
+        // ---- Gaussian proposals: 6 draws per move, lanes over moves; Box-Muller
+        // of draws (0,1) and (2,3) -> z0, z1, z2; draw 4 -> the accept uniform
+        for (int i = t; i < N; i += L) {
+          const SJGauss g = gauss_draws(p + 6 * (uint64_t)i, k0, k1, (uint32_t)w, a.epoch);
+          wk.rng[4 * i] = g.z0;
+          wk.rng[4 * i + 1] = g.z1;
+          wk.rng[4 * i + 2] = g.z2;
+          wk.rng[4 * i + 3] = g.u;
         }
-        __syncthreads();
-        xn[0] = wk.mv[0];
-        xn[1] = wk.mv[1];
-        xn[2] = wk.mv[2];
       }
-      // Jastrow terms of electron i at r' and at r_i (lanes over partners)
-      for (int j = t; j < N + S.n_nuc; j += L) {
-        if (j < N) {
-          if (j == i) {  // zero: the sums below start at +0, so it adds nothing
-            wk.jn[j] = (T)0;
-            wk.jo[j] = (T)0;
-            continue;
+      p += DPM * (uint64_t)N;
+    }
+    sync_wave();
+    uint64_t mask = 0;
+#pragma unroll 1
+    for (int i = sweep ? 0 : N - 1; i < N; ++i) {
+      if (sweep) {
+        const int s = i < nu ? 0 : 1;
+        const int c = s == 0 ? i : i - nu;
+        const int n = s == 0 ? nu : nd;
+        T *B = s == 0 ? wk.Bup : wk.Bdn;
+        const double xi[3] = {wk.pos[3 * i], wk.pos[3 * i + 1], wk.pos[3 * i + 2]};
+        const double u = wk.rng[4 * i + 3];
+        double xn[3], v[3];
+        [[maybe_unused]] double *gch = (double *)(base + lay.gch), *og = (double *)(base + lay.og),
+                                *jg = (double *)(base + lay.jg);
+        if constexpr (PROP == kSJPropBox) {
+          xn[0] = xi[0] + wk.rng[4 * i];
+          xn[1] = xi[1] + wk.rng[4 * i + 1];
+          xn[2] = xi[2] + wk.rng[4 * i + 2];
+        } else if constexpr (PROP == kSJPropLearned) {
+          // learned proposal: pass 0, the network at x -> (mu, ln sigma), x' =
+          // (x_i + mu) + sigma z; pass 1, the network at x' for the reverse
+          // density (all lanes run the MFMA passes).  One loop body keeps a
+          // single copy of the features and the network in the kernel's code.
+#pragma unroll 1
+          for (int ps = 0; ps < 2; ++ps) {
+            float fv[4];
+            mlp_features(wk.pos, N, S.nuc, nn, i, ps == 0 ? wk.pos + 3 * i : wk.mv, t, fv);
+            const f32x4 o = mlp_forward(a.net, features_bf16(fv), nullptr);
+            if (t == 0) {
+              const double lsg = mlp_log_sigma((double)o[3]);
+              const double sg = exp_m(lsg);
+              if (ps == 0) {
+                double z2 = 0.0;
+                for (int q = 0; q < 3; ++q) {
+                  const double z = wk.rng[4 * i + q];
+                  wk.mv[q] = (xi[q] + (double)o[q]) + sg * z;
+                  z2 += z * z;
+                }
+                wk.mv[3] = -3.0 * lsg - 0.5 * z2;  // log q(x'|x) + const
+              } else {
+                double e2 = 0.0;
+                for (int q = 0; q < 3; ++q) {
+                  const double e = (xi[q] - wk.mv[q]) - (double)o[q];
+                  e2 += e * e;
+                }
+                wk.mv[4] = (-3.0 * lsg - e2 / (2.0 * sg * sg)) - wk.mv[3];  // log q(x|x') - log q(x'|x)
+              }
+            }
+            sync_wave();
           }
-          const double b = ((j < nu ? 0 : 1) == s) ? S.p[1] : S.p[0];
-          wk.jn[j] = pair_term<T>(b, S.p[2], xn, wk.pos + 3 * j);
-          wk.jo[j] = pair_term<T>(b, S.p[2], xi, wk.pos + 3 * j);
+          xn[0] = wk.mv[0];
+          xn[1] = wk.mv[1];
+          xn[2] = wk.mv[2];
         } else {
-          const int I = j - N;
-          const double aZ = S.p[3] * S.charge[I];
-          wk.jn[j] = en_term<T>(aZ, S.p[4], xn, S.nuc + 3 * I);
-          wk.jo[j] = en_term<T>(aZ, S.p[4], xi, S.nuc + 3 * I);
+          // drift at x (metrop.rs:150-163): x' = (x_i + tau v) + sqrt(tau) z
+          basis_to_lds(S, lb, xi, wk.chi, t, L, gto, pk);
+          drift_terms(S, wk.pos, i, xi, wk.chi, gch, jg, t, L, gto, pk);
+          sync_wave();
+          orbital_gradients(S, n, gch, og, t, L);
+          sync_wave();
+          drift_sum<T>(og, B, n, c, jg, M, 1.0, v);
+          for (int q = 0; q < 3; ++q) xn[q] = (xi[q] + v[q] * a.tau) + a.sqrt_tau * wk.rng[4 * i + q];
+          sync_wave();
         }
-      }
-      basis_to_lds(S, xn, wk.rn, wk.chi, t, L, gto, pk);
-      for (int k = t; k < n; k += L) wk.phin[k] = (T)orbital_value(S, k, wk.chi);
-      if constexpr (PROP == kSJPropDiffuse) {
-        drift_terms(S, wk.pos, i, xn, wk.rn, wk.chi, gch, jg, t, L, gto, pk);
-        __syncthreads();
-        orbital_gradients(S, n, gch, og, t, L);
-      }
-      __syncthreads();
-      if (t == 0) {
-        const T rd = seq_dot<8>(wk.phin, B + c, n, n);
-        const T Jn = seq_sum<8>(wk.jn, N + S.n_nuc);
-        const T Jo = seq_sum<8>(wk.jo, N + S.n_nuc);
+        // Jastrow terms of electron i at r' and at r_i (lanes over electrons,
+        // then nuclei; electron i's own slot is 0 and adds nothing)
+        for (int j = t; j < M; j += L) {
+          const bool el = j < N;
+          const double *q = el ? wk.pos + 3 * j : nuc + 4 * (j - N);
+          const T num = el ? ((j < nu ? 0 : 1) == s ? bP : bA) : (T)q[3];
+          const T cd = el ? cee : cen;
+          const T fn = jastrow_term<T>(num, cd, xn, q), fo = jastrow_term<T>(num, cd, xi, q);
+          wk.jn[j] = j == i ? (T)0 : fn;
+          wk.jo[j] = j == i ? (T)0 : fo;
+        }
+        basis_to_lds(S, lb, xn, wk.chi, t, L, gto, pk);
+        if constexpr (PROP == kSJPropDiffuse) drift_terms(S, wk.pos, i, xn, wk.chi, gch, jg, t, L, gto, pk);
+        sync_wave();
+        for (int k = t; k < n; k += L) wk.phin[k] = (T)orbital_value(S, k, wk.chi);
+        if constexpr (PROP == kSJPropDiffuse) orbital_gradients(S, n, gch, og, t, L);
+        sync_wave();
+        // sum_k phi_k(r') B[k][l] of every column l: the determinant ratio for
+        // l = c, the Sherman-Morrison coefficients (times 1/ratio) for the rest
+        for (int l = t; l < n; l += L) wk.dots[l] = seq_dot<8>(wk.phin, B + l, n, n);
+        sync_wave();
+        const T rd = wk.dots[c];
+        const T Jn = seq_sum<8>(wk.jn, M);
+        const T Jo = seq_sum<8>(wk.jo, M);
         const T dJ = Jn - Jo;
         const double rdd = (double)rd;
         const double R2 = (rdd * rdd) * exp_m(2.0 * (double)dJ);
         bool accept;
         if constexpr (PROP == kSJPropBox) {
-          accept = min_one(R2) > wk.rng[4 * i + 3];
+          accept = min_one(R2) > u;
         } else if constexpr (PROP == kSJPropLearned) {
           // exact MH ratio of the learned proposal
-          accept = min_one(R2 * exp_m(wk.mv[4])) > wk.rng[4 * i + 3];
+          accept = min_one(R2 * exp_m(wk.mv[4])) > u;
         } else {
           // metrop.rs:178-197 over electron i's row: reject a sign change,
           // else min(T(x'->x) R^2 / T(x->x'), 1) > u
           double vn[3];
-          drift_sum<T>(og, B, n, c, jg, N + S.n_nuc, rdd, vn);
+          drift_sum<T>(og, B, n, c, jg, M, rdd, vn);
           double eh[3], el[3];
           for (int q = 0; q < 3; ++q) {
             eh[q] = (xi[q] - xn[q]) - vn[q] * a.tau;
-            el[q] = (xn[q] - xi[q]) - wk.mv[3 + q] * a.tau;
+            el[q] = (xn[q] - xi[q]) - v[q] * a.tau;
           }
           const double nh = norm3(eh[0], eh[1], eh[2]);
           const double nl = norm3(el[0], el[1], el[2]);
           const double t_high = exp_m(-(nh * nh) / (2.0 * a.tau));
           const double t_low = exp_m(-(nl * nl) / (2.0 * a.tau));
-          accept = !(rdd < 0.0) && min_one((t_high * R2) / t_low) > wk.rng[4 * i + 3];
+          accept = !(rdd < 0.0) && min_one((t_high * R2) / t_low) > u;
         }
-        wk.flag[0] = accept ? 1.0 : 0.0;
-        wk.flag[1] = (double)((T)1 / rd);
-        // det A_s' = R_D det A_s, carried in FP64
-        if (accept && track_ld) logdet_mul(acc[ncol + 2 * s], acc[ncol + 2 * s + 1], rdd);
-      }
-      __syncthreads();
-      const bool accept = wk.flag[0] != 0.0;
-      const T inv = (T)wk.flag[1];
-      if (accept)
-        for (int l = t; l < n; l += L) {
-          if (l == c) continue;
-          wk.f[l] = seq_dot<8>(wk.phin, B + l, n, n) * inv;
-        }
-      __syncthreads();
-      if (accept) {
-        // B[k][l] -= B[k][c] f_l for l != c; loads of a group ahead of its
-        // stores (column c is only read here)
-        const float inv_n = 1.0f / (float)n;
-        for (int e0 = t; e0 < n * n; e0 += 4 * L) {
-          T bkc[4], fl[4], be[4];
-          int ee[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int e = e0 + u * L;
-            const int k = small_div(e, inv_n), l = e - k * n;
-            ee[u] = (e < n * n && l != c) ? e : -1;
-            if (ee[u] >= 0) {
-              bkc[u] = B[k * n + c];
-              fl[u] = wk.f[l];
-              be[u] = B[e];
-            }
+        sync_wave();
+        if (accept) {
+          const T inv = (T)1 / rd;
+          // det A_s' = R_D det A_s, carried in FP64
+          if (track_ld) {
+            double m = s ? bk.ld[2] : bk.ld[0], e = s ? bk.ld[3] : bk.ld[1];
+            logdet_mul(m, e, rdd);
+            bk.ld[0] = s ? bk.ld[0] : m;
+            bk.ld[1] = s ? bk.ld[1] : e;
+            bk.ld[2] = s ? m : bk.ld[2];
+            bk.ld[3] = s ? e : bk.ld[3];
           }
+          // row k: B[k][l] -= B[k][c] f_l (l != c), B[k][c] /= R_D -- a row
+          // needs no other lane's elements
+          for (int k = t; k < n; k += L) {
+            T *row = B + k * n;
+            const T bkc = row[c];
+            int l = 0;
+            for (; l + 4 <= n; l += 4) {
+              T be[4], f[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (ee[u] >= 0) B[ee[u]] = fma_t(-bkc[u], fl[u], be[u]);
-        }
-      }
-      __syncthreads();
-      if (accept) {
-        for (int k = t; k < n; k += L) B[k * n + c] = B[k * n + c] * inv;
-        if (t == 0) {
-          wk.pos[3 * i] = xn[0];
-          wk.pos[3 * i + 1] = xn[1];
-          wk.pos[3 * i + 2] = xn[2];
+              for (int q = 0; q < 4; ++q) {
+                be[q] = row[l + q];
+                f[q] = wk.dots[l + q];
+              }
+#pragma unroll
+              for (int q = 0; q < 4; ++q) row[l + q] = fma_t(-bkc, f[q] * inv, be[q]);
+            }
+            for (; l < n; ++l) row[l] = fma_t(-bkc, wk.dots[l] * inv, row[l]);
+            row[c] = bkc * inv;
+          }
+          if (t == 0) {
+            wk.pos[3 * i] = xn[0];
+            wk.pos[3 * i + 1] = xn[1];
+            wk.pos[3 * i + 2] = xn[2];
+          }
           mask |= (uint64_t)1 << i;
-          acc[kSJAccepted] += 1.0;
+          ++n_acc;
         }
+        sync_wave();
       }
-      __syncthreads();
-      ++m;
-      if (lu_period && m % lu_period == 0) {
-        // the FP64 log|det| the update chain carried is checked against the re-inversion's
-        refresh_walker<T>(S, wk, acc, t, L, gto, pk, true, true, track_ld ? 2 : 0);
+      bool due = !sweep && entry_refresh;
+      if (sweep && lu_period && --lu_left == 0) {
+        due = true;
+        lu_left = lu_period;
+      }
+      if (due) {
+        // at entry (new configurations) the determinants are taken from the
+        // re-inversion, refresh 2 keeping the inverses; after lu_period moves the
+        // FP64 log|det| the update chain carried is checked against it
+        const bool wb = sweep || a.init || a.refresh == 1;
+        refresh_walker<T>(S, lb, wk, bk, t, L, gto, pk, wb, wb, track_ld ? (sweep ? 2 : 1) : 0);
       }
     }
-    p += DPM * (uint64_t)N;
-    if (t == 0 && live && S.trace_mask && ls.trace_sweeps + sw < a.cap_sweeps)
+    if (sweep && t == 0 && live && S.trace_mask && ls.trace_sweeps + sw < a.cap_sweeps)
       S.trace_mask[(size_t)w * a.cap_sweeps + ls.trace_sweeps + sw] = mask;
-    if (EXT && sw >= a.sample_start && a.dmc == kSJDmcStep) {
+    const bool sample = sweep && sw >= a.sample_start;
+    if (!(sample || (!sweep && entry_energy))) continue;
+
+    double *gw = nullptr;
+    if (EXT && a.dmc == kSJEval && live && S.ev_grad) gw = S.ev_grad + (size_t)w * 3 * N;
+    double *vec;
+    SJParts parts;
+    const double E = local_energy<T, EXT>(S, wk, t, L, &vec, parts, gw);
+    if (EXT && a.dmc == kSJDmcInit) {
+      // DmcRunner::new: weight 1; the local energy of the starting configuration
+      if (t == 0 && live) {
+        S.dmc[w] = 1.0;
+        S.dmc[(size_t)W + w] = E;
+      }
+    } else if (EXT && a.dmc == kSJEval) {
+      // mole_eval: psi = sign exp(log|det up| + log|det dn| + J) from the
+      // re-inversion's determinants, d psi = psi grad ln psi, lap psi = psi
+      // sum_i lap_i psi/psi, E_L and d psi/dp = psi d ln psi/dp
+      if (live) {
+        const double psi = sj_psi(S, bk.ld, vec + 2);
+        if (t == 0) {
+          if (S.ev_value) S.ev_value[w] = psi;
+          if (S.ev_lap) S.ev_lap[w] = psi * parts.kin;
+          if (S.ev_el) S.ev_el[w] = E;
+          if (S.ev_pgrad)
+            for (int k = 0; k < np; ++k) S.ev_pgrad[(size_t)w * np + k] = psi * vec[2 + k];
+        }
+        // a lane rescales the gradients it wrote
+        if (gw)
+          for (int i = t; i < N; i += L)
+            for (int q = 0; q < 3; ++q) gw[3 * i + q] = psi * gw[3 * i + q];
+      }
+    } else if (dmc_step) {
       // DmcRunner::diffuse (src/dmc/src/dmc.rs:88-128): the ensemble terms
       // with the weight before the step, then
       // w *= exp(-tau ((E_old + E_new)/2 - E_ref))
-      double dlg[kSJNParam];
-      const double E = local_energy<T, EXT>(S, wk, t, L, dlg);
       if (t == 0 && live) {
-        const double eo = S.dmc_el_in[w], wt = S.dmc_w_in[w];
-        S.dmc[2 * (size_t)W + w] = wt * eo;
-        S.dmc[3 * (size_t)W + w] = wt;
-        S.dmc[w] = wt * exp_m(-a.dmc_tau * ((eo + E) / 2.0 - *S.dmc_eref));
+        S.dmc[2 * (size_t)W + w] = dmc_w * dmc_el;
+        S.dmc[3 * (size_t)W + w] = dmc_w;
+        S.dmc[w] = dmc_w * exp_m(-a.dmc_tau * ((dmc_el + E) / 2.0 - dmc_eref));
         S.dmc[(size_t)W + w] = E;
       }
-    } else if (sw >= a.sample_start) {
-      double dlg[kSJNParam];
-      SJParts parts;
-      const double E = local_energy<T, EXT>(S, wk, t, L, dlg, &parts);
+    } else {
       if (EXT && t == 0 && live && S.n_obs) {
         // further observables: per-walker sums in HBM (opt-in, sampled sweeps only)
         for (int k = 0; k < S.n_obs; ++k) {
-          const double v = operator_value(S.ops[1 + k], parts, S, wk.pos);
+          const double val = operator_value(S.ops[1 + k], parts, S, wk.pos);
           double *o = S.obs_acc + (size_t)(2 * k) * W + w;
-          o[0] += v;
-          o[(size_t)W] = fma(v, v, o[(size_t)W]);
+          o[0] += val;
+          o[(size_t)W] = fma(val, val, o[(size_t)W]);
         }
       }
-      if (t == 0) {
-        acc[kSJSumE] += E;
-        acc[kSJSumE2] = fma(E, E, acc[kSJSumE2]);
-        acc[kSJBlockSum] += E;
-        int q = 0;
-        for (int k = 0; k < np; ++k) {
-          acc[kSJSumO + k] += dlg[k];
-          acc[sj_sum_oe(np) + k] = fma(dlg[k], E, acc[sj_sum_oe(np) + k]);
-          for (int l = k; l < np; ++l, ++q) acc[sj_sum_oo(np) + q] = fma(dlg[k], dlg[l], acc[sj_sum_oo(np) + q]);
+      // sample sums in HBM, lanes over columns: += v[a] v[b] in one rounding
+      if (live) {
+        for (int q0 = t; q0 < nsum; q0 += 4 * L) {
+          double old[4], va[4], vb[4];
+          double *at[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int q = q0 + r * L < nsum ? q0 + r * L : q0;
+            const int col = q < 2 ? q : kSJSumO - 2 + q;
+            at[r] = S.acc + (size_t)col * W + w;
+            old[r] = *at[r];
+            const uint8_t f = pairs[q];
+            va[r] = vec[f & 15];
+            vb[r] = vec[f >> 4];
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (q0 + r * L < nsum) *at[r] = fma(va[r], vb[r], old[r]);
         }
-        if (live && S.trace_e && sidx < a.cap_samples) S.trace_e[(size_t)w * a.cap_samples + sidx] = E;
-        if (EXT && live && S.samp_psi && sidx < a.cap_samples)
-          sj_compat_sample(S, acc + ncol, dlg, np, (size_t)w * a.cap_samples + sidx);
+        if (t == 0 && S.trace_e && sidx < a.cap_samples) S.trace_e[(size_t)w * a.cap_samples + sidx] = E;
+        if (EXT && t == 0 && S.samp_psi && sidx < a.cap_samples) {
+          const double ld[4] = {bk.ld[0], bk.ld[1], bk.ld[2], bk.ld[3]};  // a copy: bk stays in registers
+          sj_compat_sample(S, ld, vec + 2, np, (size_t)w * a.cap_samples + sidx);
+        }
       }
+      block_sum += E;
       if (++fill == a.block_size) {
-        if (t == 0) {
-          const double bm = acc[kSJBlockSum] * inv_block;
-          acc[kSJSumBm] += bm;
-          acc[kSJSumBm2] = fma(bm, bm, acc[kSJSumBm2]);
-          acc[kSJBlockSum] = 0.0;
+        if (t == 0 && live) {
+          const double bm = block_sum * inv_block;
+          double *s1 = S.acc + (size_t)kSJSumBm * W + w, *s2 = S.acc + (size_t)kSJSumBm2 * W + w;
+          *s1 += bm;
+          *s2 = fma(bm, bm, *s2);
         }
+        block_sum = 0.0;
         fill = 0;
       }
       ++sidx;
@@ -1121,22 +1231,32 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
   }
 
   // ---- state out ----
-  __syncthreads();
+  sync_wave();
   for (int e = lane; e < 3 * N * nslots; e += 64) {
     const int k = e >> lg_slots, sl = e & (nslots - 1);
-    if (sl < tile.nw) S.pos[(size_t)k * W + tile.w0 + sl] = ((double *)(lds + (size_t)sl * lay.bytes + lay.pos))[k];
+    if (sl < tile.nw)
+      S.pos[(size_t)k * W + tile.w0 + sl] = ((double *)(walkers + (size_t)sl * lay.bytes + lay.pos))[k];
   }
   T *Bo = (T *)S.B;
   for (int e = lane; e < nB * nslots; e += 64) {
     const int k = e >> lg_slots, sl = e & (nslots - 1);
-    if (sl < tile.nw) Bo[(size_t)k * W + tile.w0 + sl] = ((T *)(lds + (size_t)sl * lay.bytes + lay.B))[k];
+    if (sl < tile.nw) Bo[(size_t)k * W + tile.w0 + sl] = ((T *)(walkers + (size_t)sl * lay.bytes + lay.B))[k];
   }
   if (t == 0 && live) {
-    for (int k = 0; k < ncol; ++k)
-      if (!(EXT && a.dmc == kSJDmcStep) || k == kSJAccepted || k == kSJCondMax || k == kSJSingular)
-        S.acc[(size_t)k * W + w] = acc[k];
-    if (track_ld)
-      for (int k = 0; k < kSJLdColumns; ++k) S.ld[(size_t)k * W + w] = acc[ncol + k];
+    auto column = [&](int k) -> double & { return S.acc[(size_t)k * W + w]; };
+    column(kSJAccepted) = acc_in + (double)n_acc;
+    if (lu_period || entry_refresh) {
+      const double c = column(kSJCondMax), g = column(kSJSingular);
+      column(kSJCondMax) = fmax(c, bk.cond);
+      column(kSJSingular) = g + bk.singular;
+    }
+    if (!dmc_step) {
+      const double d = column(kSJLdDrift);
+      column(kSJBlockSum) = block_sum;
+      column(kSJLdDrift) = fmax(d, bk.drift);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) S.ld[(size_t)k * W + w] = bk.ld[k];
+    }
   }
 }
 
