@@ -349,9 +349,41 @@ size_t sj_footprint(const mole_ctx *ctx, const SysState &s, int L, int tsize) {
                                               (int)s.params.size(), sj_prop(ctx));
 }
 
+// Lanes per walker where the caller sets none.  A wave's instructions cost the
+// same however many lanes they use, so a full chip wants few lanes per walker
+// (`least`: below it the walkers' LDS leaves too few waves), and a chip with
+// SIMDs to spare more, up to two waves per SIMD or the width of a move
+// (`most`).  Measured, us per sampled sweep by lanes (box proposal, mixed):
+//   N   W       2     4     8    16    32    64
+//   2   65,536  14    24    45    88
+//   2   4,096   11     9     9    10
+//   3   65,536  32    42    74   142
+//   10  65,536  269   173   226  349
+//   10  16,384  116   78    59   88   170
+//   10  4,096   112   73    51   41    44    83
+//   17  16,384  850   518   352  261   395   753
+//   17  4,096   426   248   165  115   104   195
+//   36  16,384        7002  4199 3011  2000  2772
+//   36  512           1757  1013 650   429   311
+// The learned proposal's network passes take 4.
 int sj_default_lanes(const mole_ctx *ctx, const SysState &s) {
   if (ctx->run.proposal == MOLE_PROPOSAL_LEARNED) return 4;
-  return s.N <= 4 ? 4 : s.N <= 10 ? 8 : s.N <= 20 ? 16 : 32;
+  const int N = (int)s.N;
+  int64_t walkers = 0;
+  for (const SysState &o : ctx->sys) walkers += o.W;
+  // (FP64 inverses of 10 electrons at 4 lanes fit seven workgroups a CU: 253
+  // against 239 us at 8)
+  const int least = N <= 5 ? 2 : N <= (sj_tsize(ctx) == 8 ? 9 : 10) ? 4 : N <= 16 ? 8 : N <= 24 ? 16 : 32;
+  int most = 4;
+  while (most < N) most *= 2;
+  int L = 1;
+  while (2 * L <= most && walkers * (2 * L) <= (int64_t)64 * 8 * ctx->cu_count) L *= 2;
+  L = std::max(L, least);
+  // large bases: within a quarter of a CU's LDS, in FP64 too (mole_eval), up to
+  // the lanes that keep any accepted basis within the LDS
+  const int wide = N <= 4 ? 4 : N <= 10 ? 8 : N <= 20 ? 16 : 32;
+  while (L < wide && sj_footprint(ctx, s, L, 8) > ctx->lds_limit / 4) L *= 2;
+  return L;
 }
 
 // Tiles of 64/L walkers grouped by LDS footprint class (4 KiB steps, the

@@ -637,3 +637,23 @@ def test_eval_matches_oracle(make, precision):
         V += sum(1.0 / np.linalg.norm(pos[i] - pos[k]) for i in range(N) for k in range(i + 1, N))
         kin = -2.0 * (e - V - v_nn)
         assert abs(out["lap"][j] / v - kin) <= 1e-8 * max(1.0, abs(kin)), j
+
+
+@pytest.mark.parametrize("Z_or_n,W", [(2, 64), (3, 40000), (5, 9000), (10, 3000), (10, 20000), (17, 500), (36, 70)])
+def test_default_lanes_leave_the_results_unchanged(Z_or_n, W):
+    # the library's choice of lanes (by electrons and walkers; every width of
+    # the rule is met here) against 16 lanes per walker
+    sj = S.atom(Z_or_n) if Z_or_n <= 10 else S.hydrogen_chain(Z_or_n, seed=3)
+    res = []
+    for lanes in (0, 16):
+        with M.Context([M.slater_jastrow(sj, W)], seed=9, step=0.6, block_size=2, precision=M.PREC_MIXED,
+                       lu_period=16) as ctx:
+            ctx.set_walker_lanes(lanes)
+            ctx.init_walkers()
+            ctx.sweep(2)
+            ctx.sweep(2, sample=True)
+            res.append((ctx.get_configs(), ctx.stats(), ctx.sr_sums(), ctx.logdet()))
+    (c0, s0, r0, l0), (c1, s1, r1, l1) = res
+    assert np.array_equal(bits(c0), bits(c1)) and s0 == s1
+    assert all(np.array_equal(r0[k], r1[k]) for k in r0)
+    assert np.array_equal(bits(l0[0]), bits(l1[0])) and np.array_equal(l0[1], l1[1])
