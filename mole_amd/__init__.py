@@ -450,7 +450,7 @@ class Context:
 
     def get_configs(self, sys=0):
         s = self.systems[sys]
-        a = np.zeros((s.n_walkers, s.n_electrons * 3))
+        a = np.empty((s.n_walkers, s.n_electrons * 3))
         check(lib().mole_get_configs(self.h, sys, _dp(a), s.n_walkers))
         return a
 
@@ -520,7 +520,7 @@ class Context:
         """mole_tau_int: per-walker integrated autocorrelation time of the
         local-energy samples [first, first + n) of the trace, on the device."""
         W = self.systems[sys].n_walkers
-        t = np.zeros(W)
+        t = np.empty(W)
         check(lib().mole_tau_int(self.h, sys, first, n, _dp(t), W))
         return t
 
@@ -546,8 +546,8 @@ class Context:
         D = 3 * s.n_electrons
         a = np.ascontiguousarray(cfg, dtype=np.float64).reshape(-1, D)
         n = a.shape[0]
-        out = dict(value=np.zeros(n), grad=np.zeros((n, D)), lap=np.zeros(n),
-                   e_local=np.zeros(n), pgrad=np.zeros((n, s.params.size)))
+        out = dict(value=np.empty(n), grad=np.empty((n, D)), lap=np.empty(n),
+                   e_local=np.empty(n), pgrad=np.empty((n, s.params.size)))
         check(lib().mole_eval(self.h, sys, n, _dp(a), _dp(out["value"]), _dp(out["grad"]),
                               _dp(out["lap"]), _dp(out["e_local"]), _dp(out["pgrad"])))
         return out
@@ -646,7 +646,7 @@ class Context:
 
     def dmc_read_walkers(self, sys=0):
         W = self.systems[sys].n_walkers
-        w, e = np.zeros(W), np.zeros(W)
+        w, e = np.empty(W), np.empty(W)
         check(lib().mole_dmc_read_walkers(self.h, sys, _dp(w), _dp(e), W))
         return w, e
 

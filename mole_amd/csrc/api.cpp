@@ -171,6 +171,9 @@ struct mole_ctx {
   // diffusion Monte Carlo
   bool dmc_ready = false;
   uint32_t dmc_brancher = 0;
+  // pinned staging of large host transfers (two halves, made on first use)
+  char *stage[2] = {nullptr, nullptr};
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
 };
 
 // The learned proposal's network, its Adam state and its training data.
@@ -326,10 +329,128 @@ void free_ctx(mole_ctx *ctx) {
   if (ctx->d_tiles) (void)hipFree(ctx->d_tiles);
   if (ctx->d_tiles_lpt) (void)hipFree(ctx->d_tiles_lpt);
   if (ctx->d_ticket) (void)hipFree(ctx->d_ticket);
+  for (int b = 0; b < 2; ++b) {
+    if (ctx->stage_ev[b]) (void)hipEventDestroy(ctx->stage_ev[b]);
+    if (ctx->stage[b]) (void)hipHostFree(ctx->stage[b]);
+  }
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
+}
+
+// ---- large host transfers -----------------------------------------------------
+// A copy between device and pageable host memory costs 0.4 ms from about 1 MB
+// on whatever its size (the runtime pins the pages) and a configuration array
+// had to be transposed between [3N][W] and [walker][3N] through a zeroed
+// buffer of its size on the host (16 MB: 3 ms to zero, 0.6 ms to transpose).
+// Transfers from kStageMin on instead go through two pinned halves, the
+// device working on one (transposing straight into or out of it) while the
+// host copies the other: 0.06 ms for 1 MB, 0.9 for 16 MB of touched pages.
+constexpr size_t kStageChunk = (size_t)1 << 20, kStageMin = (size_t)128 << 10;
+
+hipError_t stage_init(mole_ctx *ctx) {
+  hipError_t e = hipSuccess;
+  for (int b = 0; b < 2 && e == hipSuccess; ++b) {
+    if (!ctx->stage[b]) {
+      void *p = nullptr;
+      e = hipHostMalloc(&p, kStageChunk, hipHostMallocDefault);
+      if (e == hipSuccess) ctx->stage[b] = (char *)p;
+    }
+    if (e == hipSuccess && !ctx->stage_ev[b]) e = hipEventCreateWithFlags(&ctx->stage_ev[b], hipEventDisableTiming);
+  }
+  return e;
+}
+
+// total units in chunks of `per`: fill(buffer, first, n) enqueues the device's
+// part into the pinned buffer, drain(buffer, first, n) copies it out on the
+// host once it is there.  Returns with the stream idle.
+template <class Fill, class Drain>
+hipError_t stage_read(mole_ctx *ctx, size_t total, size_t per, Fill fill, Drain drain) {
+  hipError_t e = stage_init(ctx);
+  const size_t nc = (total + per - 1) / per;
+  auto start = [&](size_t c) {
+    const int b = (int)(c & 1);
+    e = fill(ctx->stage[b], c * per, std::min(per, total - c * per));
+    if (e == hipSuccess) e = hipEventRecord(ctx->stage_ev[b], ctx->stream);
+  };
+  for (size_t c = 0; c < std::min<size_t>(2, nc) && e == hipSuccess; ++c) start(c);
+  for (size_t c = 0; c < nc && e == hipSuccess; ++c) {
+    e = hipEventSynchronize(ctx->stage_ev[c & 1]);
+    if (e != hipSuccess) break;
+    drain(ctx->stage[c & 1], c * per, std::min(per, total - c * per));
+    if (c + 2 < nc) start(c + 2);
+  }
+  const hipError_t es = hipStreamSynchronize(ctx->stream);  // no device access to the halves is left pending
+  return e == hipSuccess ? es : e;
+}
+
+// The other way: fill on the host, then the device's part.
+template <class Fill, class Drain>
+hipError_t stage_write(mole_ctx *ctx, size_t total, size_t per, Fill fill, Drain drain) {
+  hipError_t e = stage_init(ctx);
+  const size_t nc = (total + per - 1) / per;
+  for (size_t c = 0; c < nc && e == hipSuccess; ++c) {
+    const int b = (int)(c & 1);
+    if (c >= 2) e = hipEventSynchronize(ctx->stage_ev[b]);
+    if (e != hipSuccess) break;
+    fill(ctx->stage[b], c * per, std::min(per, total - c * per));
+    e = drain(ctx->stage[b], c * per, std::min(per, total - c * per));
+    if (e == hipSuccess) e = hipEventRecord(ctx->stage_ev[b], ctx->stream);
+  }
+  const hipError_t es = hipStreamSynchronize(ctx->stream);
+  return e == hipSuccess ? es : e;
+}
+
+// bytes of device memory to the host; returns with the stream idle.
+hipError_t read_back(mole_ctx *ctx, void *host, const void *dev, size_t bytes) {
+  if (bytes < kStageMin) {
+    const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    return e == hipSuccess ? es : e;
+  }
+  return stage_read(
+      ctx, bytes, kStageChunk,
+      [&](char *b, size_t first, size_t n) {
+        return hipMemcpyAsync(b, (const char *)dev + first, n, hipMemcpyDeviceToHost, ctx->stream);
+      },
+      [&](const char *b, size_t first, size_t n) { std::memcpy((char *)host + first, b, n); });
+}
+
+// cfg [W][D] from columns [D][W] on the device; returns with the stream idle.
+hipError_t read_rows(mole_ctx *ctx, double *cfg, const double *cols, size_t D, size_t W) {
+  if (sizeof(double) * D * W < kStageMin) {
+    std::vector<double> soa(D * W);
+    const hipError_t e = read_back(ctx, soa.data(), cols, soa.size() * sizeof(double));
+    for (size_t w = 0; w < W; ++w)
+      for (size_t k = 0; k < D; ++k) cfg[w * D + k] = soa[k * W + w];
+    return e;
+  }
+  return stage_read(
+      ctx, W, kStageChunk / (sizeof(double) * D),
+      [&](char *b, size_t first, size_t n) {
+        return launch_columns_to_rows(cols, W, (int)D, first, n, (double *)b, ctx->stream);
+      },
+      [&](const char *b, size_t first, size_t n) { std::memcpy(cfg + first * D, b, sizeof(double) * D * n); });
+}
+
+// columns [D][W] on the device from cfg [W][D]; returns with the stream idle.
+hipError_t write_rows(mole_ctx *ctx, const double *cfg, double *cols, size_t D, size_t W) {
+  if (sizeof(double) * D * W < kStageMin) {
+    std::vector<double> soa(D * W);
+    for (size_t w = 0; w < W; ++w)
+      for (size_t k = 0; k < D; ++k) soa[k * W + w] = cfg[w * D + k];
+    const hipError_t e =
+        hipMemcpyAsync(cols, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    return e == hipSuccess ? es : e;
+  }
+  return stage_write(
+      ctx, W, kStageChunk / (sizeof(double) * D),
+      [&](char *b, size_t first, size_t n) { std::memcpy(b, cfg + first * D, sizeof(double) * D * n); },
+      [&](const char *b, size_t first, size_t n) {
+        return launch_rows_to_columns((const double *)b, W, (int)D, first, n, cols, ctx->stream);
+      });
 }
 
 // ---- Slater-Jastrow launch plumbing ----------------------------------------
@@ -954,14 +1075,8 @@ mole_status mole_set_configs(mole_ctx *ctx, uint32_t sys, const double *cfg, siz
   SysState &s = ctx->sys[sys];
   if (!cfg) return fail(MOLE_ERR_INVALID_ARGUMENT, "null cfg");
   if (n_walkers != (size_t)s.W) return fail(MOLE_ERR_SHAPE, "expected %d walkers", s.W);
-  const size_t D = 3 * s.N, W = s.W;
-  std::vector<double> soa(D * W);
-  for (size_t w = 0; w < W; ++w)
-    for (size_t k = 0; k < D; ++k) soa[k * W + w] = cfg[w * D + k];
   HIP_TRY(hipSetDevice(ctx->device));
-  HIP_TRY(hipMemcpyAsync(s.d_pos, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice,
-                         ctx->stream));
-  HIP_TRY(hipStreamSynchronize(ctx->stream));
+  HIP_TRY(write_rows(ctx, cfg, s.d_pos, 3 * (size_t)s.N, (size_t)s.W));
   if (ctx->family == kFamSJ) {
     st = sj_prepare(ctx, false);
     if (st != MOLE_OK) return st;
@@ -975,14 +1090,8 @@ mole_status mole_get_configs(mole_ctx *ctx, uint32_t sys, double *cfg, size_t n_
   SysState &s = ctx->sys[sys];
   if (!cfg) return fail(MOLE_ERR_INVALID_ARGUMENT, "null cfg");
   if (n_walkers != (size_t)s.W) return fail(MOLE_ERR_SHAPE, "expected %d walkers", s.W);
-  const size_t D = 3 * s.N, W = s.W;
-  std::vector<double> soa(D * W);
   HIP_TRY(hipSetDevice(ctx->device));
-  HIP_TRY(hipMemcpyAsync(soa.data(), s.d_pos, soa.size() * sizeof(double), hipMemcpyDeviceToHost,
-                         ctx->stream));
-  HIP_TRY(hipStreamSynchronize(ctx->stream));
-  for (size_t w = 0; w < W; ++w)
-    for (size_t k = 0; k < D; ++k) cfg[w * D + k] = soa[k * W + w];
+  HIP_TRY(read_rows(ctx, cfg, s.d_pos, 3 * (size_t)s.N, (size_t)s.W));
   return ok();
 }
 
@@ -1235,8 +1344,7 @@ mole_status mole_tau_int(mole_ctx *ctx, uint32_t sys, size_t first, size_t n, do
   double *d = nullptr;
   HIP_TRY(hipMalloc(&d, sizeof(double) * (size_t)s.W));
   hipError_t e = launch_tau_corr(s.d_trace_e, s.W, ctx->run.record_sweeps, first, (int)n, d, ctx->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(tau, d, sizeof(double) * (size_t)s.W, hipMemcpyDeviceToHost, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  if (e == hipSuccess) e = read_back(ctx, tau, d, sizeof(double) * (size_t)s.W);
   (void)hipFree(d);
   if (e != hipSuccess) return fail(MOLE_ERR_DEVICE, "mole_tau_int: %s", hipGetErrorString(e));
   return ok();
@@ -1325,7 +1433,7 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
   const SysState &s = ctx->sys[sys];
   const size_t D = 3 * (size_t)s.N, np = s.params.size();
   const size_t nB = (size_t)s.n_up * s.n_up + (size_t)s.n_down * s.n_down;
-  const size_t ncol = (size_t)sj_columns((int)np);
+  const size_t ncol = kSJSumO;  // no samples: only the counters' columns are touched
   const int wpt = 64 / s.L;
   if (n > ((size_t)1 << 28)) return fail(MOLE_ERR_SHAPE, "mole_eval: at most 2^28 configurations per call");
   // evaluated in FP64 whatever the context's precision (Function::value and
@@ -1350,9 +1458,6 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
   if (e == hipSuccess) e = hipMalloc(&d_sys, sizeof(SJSysDev));
   if (e == hipSuccess) e = hipMalloc(&d_tiles, sizeof(SJTile) * n_tiles);
   if (e == hipSuccess) {
-    std::vector<double> soa(D * n);
-    for (size_t w = 0; w < n; ++w)
-      for (size_t k = 0; k < D; ++k) soa[k * n + w] = cfg[w * D + k];
     SJSysDev v = sj_sysdev_of(ctx, sys);
     v.W = (int)n;
     v.lds_per_walker = (uint32_t)lds_walker;
@@ -1382,8 +1487,7 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
     if (e == hipSuccess) e = hipMemcpy(d_sys, &v, sizeof(SJSysDev), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_tiles, tiles.data(), sizeof(SJTile) * n_tiles, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = launch_fill(d + o_B, o_val - o_B, 0.0, ctx->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(d + o_pos, soa.data(), sizeof(double) * D * n, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) e = write_rows(ctx, cfg, d + o_pos, D, n);
     if (e == hipSuccess) {
       SJArgs a = sj_args(ctx);
       a.systems = d_sys;
@@ -1399,8 +1503,7 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
       e = launch_sj(a, (int)n_tiles, 0, kSJPropBox, lds, ctx->stream);
     }
     auto back = [&](double *host, size_t off, size_t cnt) {
-      if (e == hipSuccess && host)
-        e = hipMemcpyAsync(host, d + off, sizeof(double) * cnt, hipMemcpyDeviceToHost, ctx->stream);
+      if (e == hipSuccess && host) e = read_back(ctx, host, d + off, sizeof(double) * cnt);
     };
     back(value, o_val, n);
     back(grad, o_grad, D * n);
@@ -2396,9 +2499,9 @@ mole_status mole_dmc_read_walkers(mole_ctx *ctx, uint32_t sys, double *weights, 
   const SysState &s = ctx->sys[sys];
   if (n_walkers != (size_t)s.W) return fail(MOLE_ERR_SHAPE, "system %u has %d walkers", sys, s.W);
   HIP_TRY(hipSetDevice(ctx->device));
-  HIP_TRY(hipStreamSynchronize(ctx->stream));
-  if (weights) HIP_TRY(hipMemcpy(weights, s.dmc.dmc, sizeof(double) * s.W, hipMemcpyDeviceToHost));
-  if (e_local) HIP_TRY(hipMemcpy(e_local, s.dmc.dmc + s.W, sizeof(double) * s.W, hipMemcpyDeviceToHost));
+  if (weights) HIP_TRY(read_back(ctx, weights, s.dmc.dmc, sizeof(double) * s.W));
+  if (e_local) HIP_TRY(read_back(ctx, e_local, s.dmc.dmc + s.W, sizeof(double) * s.W));
+  if (!weights && !e_local) HIP_TRY(hipStreamSynchronize(ctx->stream));
   return ok();
 }
 

@@ -92,6 +92,12 @@ hipError_t launch_eval2(const Eval2Args &a, hipStream_t stream);
 // columns [max_first, max_first + max_count) by their maximum instead
 hipError_t launch_reduce_columns(const double *acc, int W, int K, double *out,
                                  int max_first, int max_count, hipStream_t stream);
+// rows[(w - w0) D + k] = cols[k W + w] for w in [w0, w0 + n), and back; rows
+// may be pinned host memory
+hipError_t launch_columns_to_rows(const double *cols, size_t W, int D, size_t w0, size_t n, double *rows,
+                                  hipStream_t stream);
+hipError_t launch_rows_to_columns(const double *rows, size_t W, int D, size_t w0, size_t n, double *cols,
+                                  hipStream_t stream);
 hipError_t launch_fill(double *p, size_t n, double v, hipStream_t stream);
 // tau_out[w] = integrated autocorrelation time (scripts/statfor.rs:30-54) of
 // samples [first, first + n) of walker w's series in trace_e [W][cap], n >= 2

@@ -852,6 +852,36 @@ __global__ void __launch_bounds__(256) block_records_kernel(const double *trace_
   }
 }
 
+// Transposition between columns [D][W] and rows [n][D] of walkers w0 .. w0+n-1
+// through a 64 x 32 LDS tile: 512-byte runs of a column, 256-byte runs of a
+// row.  The row side is usually pinned host memory, whose link bounds it.
+template <bool TO_ROWS>
+__global__ void __launch_bounds__(256) transpose_kernel(double *cols, size_t W, int D, size_t w0, size_t n,
+                                                        double *rows) {
+  __shared__ double tile[32][65];
+  const size_t r0 = (size_t)blockIdx.x * 64;
+  const int k0 = (int)blockIdx.y * 32;
+  auto by_column = [&](auto f) {  // consecutive lanes on consecutive walkers
+    const size_t r = r0 + (threadIdx.x & 63);
+    for (int k = (int)(threadIdx.x >> 6); k < 32; k += 4)
+      if (r < n && k0 + k < D) f(cols[(size_t)(k0 + k) * W + w0 + r], tile[k][threadIdx.x & 63]);
+  };
+  auto by_row = [&](auto f) {  // consecutive lanes on consecutive columns
+    const int k = (int)(threadIdx.x & 31);
+    for (int q = (int)(threadIdx.x >> 5); q < 64; q += 8)
+      if (r0 + q < n && k0 + k < D) f(rows[(r0 + q) * (size_t)D + k0 + k], tile[k][q]);
+  };
+  if constexpr (TO_ROWS) {
+    by_column([](double &g, double &t) { t = g; });
+    __syncthreads();
+    by_row([](double &g, double &t) { g = t; });
+  } else {
+    by_row([](double &g, double &t) { t = g; });
+    __syncthreads();
+    by_column([](double &g, double &t) { g = t; });
+  }
+}
+
 __global__ void fill_kernel(double *p, size_t n, double v) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -934,6 +964,20 @@ hipError_t launch_eval2(const Eval2Args &a, hipStream_t stream) {
 hipError_t launch_reduce_columns(const double *acc, int W, int K, double *out, int max_first, int max_count,
                                  hipStream_t stream) {
   hipLaunchKernelGGL(reduce_columns_kernel, dim3(K), dim3(256), 0, stream, acc, W, out, max_first, max_count);
+  return hipGetLastError();
+}
+
+hipError_t launch_columns_to_rows(const double *cols, size_t W, int D, size_t w0, size_t n, double *rows,
+                                  hipStream_t stream) {
+  hipLaunchKernelGGL(transpose_kernel<true>, dim3((unsigned)((n + 63) / 64), (unsigned)((D + 31) / 32)), dim3(256), 0,
+                     stream, const_cast<double *>(cols), W, D, w0, n, rows);
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_to_columns(const double *rows, size_t W, int D, size_t w0, size_t n, double *cols,
+                                  hipStream_t stream) {
+  hipLaunchKernelGGL(transpose_kernel<false>, dim3((unsigned)((n + 63) / 64), (unsigned)((D + 31) / 32)), dim3(256), 0,
+                     stream, cols, W, D, w0, n, const_cast<double *>(rows));
   return hipGetLastError();
 }
 

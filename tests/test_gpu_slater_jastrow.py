@@ -657,3 +657,14 @@ def test_default_lanes_leave_the_results_unchanged(Z_or_n, W):
     assert np.array_equal(bits(c0), bits(c1)) and s0 == s1
     assert all(np.array_equal(r0[k], r1[k]) for k in r0)
     assert np.array_equal(bits(l0[0]), bits(l1[0])) and np.array_equal(l0[1], l1[1])
+
+
+@pytest.mark.parametrize("N,W", [(1, 5461), (1, 5462), (2, 21846), (3, 14563), (11, 3973), (40, 200), (40, 2185)])
+def test_configurations_round_trip_through_staged_transfers(N, W):
+    # both sides of the staging rule (128 KiB), chunks of 1 MiB with a partial
+    # last one, partial 64 x 32 tiles, more than one column tile
+    sj = S.hydrogenic() if N == 1 else S.hydrogen_chain(N, seed=1)
+    cfg = np.random.default_rng(N).normal(size=(W, 3 * N))
+    with M.Context([M.slater_jastrow(sj, W)], seed=1, step=0.5, block_size=2) as ctx:
+        ctx.set_configs(cfg)
+        assert np.array_equal(bits(ctx.get_configs()), bits(cfg))
