@@ -465,7 +465,7 @@ int sj_prop(const mole_ctx *ctx) {
 
 // LDS bytes of a workgroup of system s at L lanes per walker.
 size_t sj_footprint(const mole_ctx *ctx, const SysState &s, int L, int tsize) {
-  return sj_lds_per_group(s.n_nuc) +
+  return sj_lds_per_group(s.n_nuc, s.n_basis, s.n_orb) +
          (size_t)(64 / L) * sj_lds_per_walker((int)s.N, (int)s.n_up, (int)s.n_down, s.n_nuc, s.n_basis, tsize,
                                               (int)s.params.size(), sj_prop(ctx));
 }
@@ -1440,7 +1440,7 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
   // its derivatives at given configurations, no update chain to save)
   const size_t lds_walker =
       sj_lds_per_walker((int)s.N, (int)s.n_up, (int)s.n_down, s.n_nuc, s.n_basis, 8, (int)np, kSJPropBox);
-  const size_t lds = sj_lds_per_group(s.n_nuc) + (size_t)wpt * lds_walker;
+  const size_t lds = sj_lds_per_group(s.n_nuc, s.n_basis, s.n_orb) + (size_t)wpt * lds_walker;
   if (lds > ctx->lds_limit)
     return fail(MOLE_ERR_UNSUPPORTED, "mole_eval: %zu B of LDS per workgroup at %d lanes per walker (limit %zu)",
                 lds, s.L, ctx->lds_limit);

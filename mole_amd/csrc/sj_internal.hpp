@@ -148,7 +148,7 @@ struct SJArgs {
 
 // LDS bytes of one walker (prop: SJProposal) and of what a workgroup shares.
 size_t sj_lds_per_walker(int N, int nu, int nd, int nn, int K, int tsize, int np, int prop);
-size_t sj_lds_per_group(int nn);
+size_t sj_lds_per_group(int nn, int K, int n_orb);
 // Doubles read past the end of the coefficient table (register chunks of the
 // local energy): the host pads it.
 constexpr int kSJCoefPad = 8;

@@ -39,7 +39,7 @@ namespace mole {
 // scratch: the stage arrays of a move, or a Gauss-Jordan re-inversion; the
 // local energy's per-electron results take the draws and the scratch together
 // (no draw is pending after a sweep).  Per workgroup, ahead of the walkers:
-// the nuclei (x, y, z, -a Z) and the factor pairs of the sample sums.
+// SJShared.
 struct SJLayout {
   uint32_t pos, B, rng, scr, mv, chi, phin, jn, jo, dots, gch, og, jg, le, bytes;
   __host__ __device__ SJLayout(int N, int nu, int nd, int nn, int K, int tsize, int np, int prop) {
@@ -80,12 +80,35 @@ struct SJLayout {
 // follow from kSJSumO on (O, O E, upper triangle of O O^T).
 __host__ __device__ constexpr int sj_sample_sums(int np) { return 2 + 2 * np + np * (np + 1) / 2; }
 constexpr uint32_t kSJPairBytes = (sj_sample_sums(kSJNParam) + 7) / 8 * 8;
-__host__ __device__ constexpr uint32_t sj_lds_shared(int nn) { return kSJPairBytes + 32u * (uint32_t)nn; }
+
+// What the walkers of a workgroup share, at the start of its LDS: the factor
+// pairs, the nuclei (x, y, z, -a Z), and -- where they are small -- the basis
+// functions (centre x, y, z, exponent, kind) and the orbital coefficients,
+// which the lanes of a move read by function and by orbital.  From HBM each of
+// these reads is a dependent chain (centre index, then coordinates) of cache
+// latencies that two waves per SIMD do not hide (3-4 % of the atoms' sweeps).
+// Larger tables cost resident workgroups instead: with up to 128 functions
+// staged, a 36-electron molecule of 39 functions went from eight to seven a CU
+// and 8,192 walkers of it from 1,066 to 1,487 us per sweep.
+constexpr int kSJTabBasis = 8;         // functions
+constexpr uint32_t kSJTabCoef = 512;  // bytes
+struct SJShared {
+  uint32_t nuc, fn, coef, bytes;
+  bool has_fn, has_coef;
+  __host__ __device__ SJShared(int nn, int K, int n_orb) {
+    has_fn = K <= kSJTabBasis;
+    has_coef = 8u * (uint32_t)K * (uint32_t)n_orb <= kSJTabCoef;
+    nuc = kSJPairBytes;
+    fn = nuc + 32u * (uint32_t)nn;
+    coef = fn + (has_fn ? 40u * (uint32_t)K : 0u);
+    bytes = coef + (has_coef ? 8u * (uint32_t)K * (uint32_t)n_orb : 0u);
+  }
+};
 
 __host__ size_t sj_lds_per_walker(int N, int nu, int nd, int nn, int K, int tsize, int np, int prop) {
   return SJLayout(N, nu, nd, nn, K, tsize, np, prop).bytes;
 }
-__host__ size_t sj_lds_per_group(int nn) { return sj_lds_shared(nn); }
+__host__ size_t sj_lds_per_group(int nn, int K, int n_orb) { return SJShared(nn, K, n_orb).bytes; }
 
 namespace {
 
@@ -128,42 +151,67 @@ __device__ __forceinline__ float fma_t(float a, float b, float c) { return fmaf(
 // lies at least 1/(2n) from an integer, far beyond the rounding error.
 __device__ __forceinline__ int small_div(int e, float inv_n) { return (int)(((float)e + 0.5f) * inv_n); }
 
-// The first basis function a lane evaluates (m = t), kept in registers: with
-// as many lanes as functions the sweep reads no basis table.  (Eight orbital
-// coefficients kept the same way cost 2-3 % in spills.)
-struct SJLaneBasis {
-  double zeta, R[3];
-  int kind;
-  __device__ __forceinline__ void load(const SJSysDev &S, int t) {
-    const int m = t < S.n_basis ? t : 0;
-    zeta = S.zeta[m];
-    kind = S.kind[m];
-    const int I = S.center[m];
-    for (int q = 0; q < 3; ++q) R[q] = S.nuc[3 * I + q];
-  }
+// The workgroup's shared tables (LDS).
+struct SJTab {
+  const double *nuc, *fn, *coef;
+  bool has_fn, has_coef;
 };
+
+// A basis function at the point r: displacement, distance, exponent, kind.
+struct SJFn {
+  double d0, d1, d2, r, z;
+  int kind;
+};
+__device__ __forceinline__ SJFn basis_at(const SJSysDev &S, const SJTab &tab, int m, const double *r) {
+  SJFn f;
+  double R0, R1, R2;
+  if (tab.has_fn) {
+    const double *e = tab.fn + 5 * m;
+    R0 = e[0];
+    R1 = e[1];
+    R2 = e[2];
+    f.z = e[3];
+    f.kind = __double2loint(e[4]);
+  } else {
+    const double *R = tab.nuc + 4 * S.center[m];
+    R0 = R[0];
+    R1 = R[1];
+    R2 = R[2];
+    f.z = S.zeta[m];
+    f.kind = S.kind[m];
+  }
+  f.d0 = r[0] - R0;
+  f.d1 = r[1] - R1;
+  f.d2 = r[2] - R2;
+  f.r = norm3(f.d0, f.d1, f.d2);
+  return f;
+}
 
 // Basis values chi[m] of the point r into LDS (lanes over basis functions, each
 // with its own centre's distance).  gto/pk: Gaussians / p-type STOs may occur
-// (otherwise every function is an s-type STO).  rn (optional): the distances
-// by function.  No barrier.
-__device__ __forceinline__ void basis_to_lds(const SJSysDev &S, const SJLaneBasis &lb, const double *r, double *chi,
-                                             int t, int L, bool gto, bool pk) {
-  double z = lb.zeta, R0 = lb.R[0], R1 = lb.R[1], R2 = lb.R[2];
-  int kd = lb.kind;
-  for (int m = t;;) {
-    if (m >= S.n_basis) break;
-    const double d0 = r[0] - R0, d1 = r[1] - R1, d2 = r[2] - R2;
-    const double rr = norm3(d0, d1, d2);
-    chi[m] = (gto || pk) ? basis_value<true>(kd, z, d0, d1, d2, rr) : exp_m(-z * rr);
-    m += L;
-    if (m >= S.n_basis) break;
-    const int I = S.center[m];
-    z = S.zeta[m];
-    kd = S.kind[m];
-    R0 = S.nuc[3 * I];
-    R1 = S.nuc[3 * I + 1];
-    R2 = S.nuc[3 * I + 2];
+// (otherwise every function is an s-type STO).  No barrier.
+__device__ __forceinline__ void basis_to_lds(const SJSysDev &S, const SJTab &tab, const double *r, double *chi, int t,
+                                             int L, bool gto, bool pk) {
+#pragma unroll 1
+  for (int m = t; m < S.n_basis; m += L) {
+    const SJFn f = basis_at(S, tab, m, r);
+    chi[m] = (gto || pk) ? basis_value<true>(f.kind, f.z, f.d0, f.d1, f.d2, f.r) : exp_m(-f.z * f.r);
+  }
+}
+
+// The same with the gradients gch[3m + q] (the drift-diffusion proposal, FP64;
+// metrop.rs:153-155): the value and the gradient share the exponential.
+__device__ __forceinline__ void basis_gradients_to_lds(const SJSysDev &S, const SJTab &tab, const double *r,
+                                                       double *chi, double *gch, int t, int L) {
+#pragma unroll 1
+  for (int m = t; m < S.n_basis; m += L) {
+    const SJFn f = basis_at(S, tab, m, r);
+    double v, g0, g1, g2, l;
+    basis_vgl<true>(f.kind, f.z, f.d0, f.d1, f.d2, f.r, v, g0, g1, g2, l);
+    chi[m] = v;
+    gch[3 * m] = g0;
+    gch[3 * m + 1] = g1;
+    gch[3 * m + 2] = g2;
   }
 }
 
@@ -206,11 +254,26 @@ __device__ __forceinline__ T seq_dot(const T *a, const T *b, int stride, int n) 
 
 // phi_k = sum_m c_km chi_m, fma chain in m order; coefficients from the
 // [n_basis][n_orb] table (consecutive k on consecutive lanes)
-__device__ __forceinline__ double orbital_value(const SJSysDev &S, int k, const double *chi) {
-  const double *c = S.coef_t + k;
+__device__ __forceinline__ double orbital_value(const SJSysDev &S, const SJTab &tab, int k, const double *chi) {
   const int K = S.n_basis, no = S.n_orb;
   double phi = 0.0;
   int m = 0;
+  if (tab.has_coef) {
+    const double *c = tab.coef + k;
+    for (; m + 4 <= K; m += 4) {
+      double cv[4], xv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        cv[u] = c[(m + u) * no];
+        xv[u] = chi[m + u];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) phi = fma(cv[u], xv[u], phi);
+    }
+    for (; m < K; ++m) phi = fma(c[m * no], chi[m], phi);
+    return phi;
+  }
+  const double *c = S.coef_t + k;
   for (; m + 8 <= K; m += 8) {
     double cv[8], xv[8];
 #pragma unroll
@@ -264,7 +327,7 @@ struct SJRefresh {
 // the determinant reads 0.  All lanes of the workgroup must call it; the
 // norms and the pivot search run on every lane alike.
 template <typename T>
-__device__ __forceinline__ SJRefresh refresh_spin(const SJSysDev &S, const SJLaneBasis &lb, SJWalker<T> &wk, int s,
+__device__ __forceinline__ SJRefresh refresh_spin(const SJSysDev &S, const SJTab &tab, SJWalker<T> &wk, int s,
                                                   int t, int L, bool gto, bool pk, bool write_B) {
   SJRefresh res{1.0, 1.0, 0.0, false};
   const int n = s == 0 ? S.n_up : S.n_dn;
@@ -274,9 +337,9 @@ __device__ __forceinline__ SJRefresh refresh_spin(const SJSysDev &S, const SJLan
   double *M = wk.scr, *I = wk.scr + n * n, *colp = wk.scr + 2 * n * n, *chi = I;
   sync_wave();
   for (int c = 0; c < n; ++c) {
-    basis_to_lds(S, lb, wk.pos + 3 * (first + c), chi, t, L, gto, pk);
+    basis_to_lds(S, tab, wk.pos + 3 * (first + c), chi, t, L, gto, pk);
     sync_wave();
-    for (int k = t; k < n; k += L) M[c * n + k] = orbital_value(S, k, chi);
+    for (int k = t; k < n; k += L) M[c * n + k] = orbital_value(S, tab, k, chi);
     sync_wave();
   }
   double anorm = 0.0;
@@ -350,12 +413,12 @@ __device__ __forceinline__ SJRefresh refresh_spin(const SJSysDev &S, const SJLan
 // (taken from the re-inversion) or 2 (the same, after recording how far the
 // value the updates carried drifted from it).
 template <typename T>
-__device__ __forceinline__ void refresh_walker(const SJSysDev &S, const SJLaneBasis &lb, SJWalker<T> &wk, SJBooks &bk,
+__device__ __forceinline__ void refresh_walker(const SJSysDev &S, const SJTab &tab, SJWalker<T> &wk, SJBooks &bk,
                                                int t, int L, bool gto, bool pk, bool write_B, bool count,
                                                int ld_mode) {
 #pragma unroll 1
   for (int q = 0; q < 2; ++q) {
-    const SJRefresh r = refresh_spin<T>(S, lb, wk, q, t, L, gto, pk, write_B);
+    const SJRefresh r = refresh_spin<T>(S, tab, wk, q, t, L, gto, pk, write_B);
     if (count) {
       bk.cond = fmax(bk.cond, r.cond);
       if (r.singular) bk.singular += 1.0;
@@ -700,69 +763,38 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
   return E;
 }
 
-// Pieces of grad_i ln psi at r for the drift-diffusion proposal, FP64
-// (metrop.rs:153-155).  Basis gradients into gch[3m + q] (lanes over basis
-// functions; chi of r by the same lane) and the Jastrow gradient terms
-// of electron i at r into jg[3j + q] (lanes over partners, i's slot zero).
-// No barrier.
-__device__ __forceinline__ void drift_terms(const SJSysDev &S, const double *pos, int i, const double *r,
-                                            const double *chi, double *gch, double *jg, int t, int L, bool gto,
-                                            bool pk) {
-  for (int m = t; m < S.n_basis; m += L) {
-    const int I = S.center[m];
-    const double d0 = r[0] - S.nuc[3 * I], d1 = r[1] - S.nuc[3 * I + 1], d2 = r[2] - S.nuc[3 * I + 2];
-    const double rr = norm3(d0, d1, d2);
-    const int kd = (gto || pk) ? S.kind[m] : MOLE_BASIS_STO;
-    if (kd == MOLE_BASIS_STO) {
-      // chi[m] = exp(-z r) is in LDS; basis_vgl's operations
-      const double gf = (-S.zeta[m] * chi[m]) * (1.0 / rr);
-      gch[3 * m] = gf * d0;
-      gch[3 * m + 1] = gf * d1;
-      gch[3 * m + 2] = gf * d2;
-    } else {
-      basis_grad<true>(kd, S.zeta[m], d0, d1, d2, rr, gch[3 * m], gch[3 * m + 1], gch[3 * m + 2]);
-    }
-  }
+// Jastrow gradient terms of electron i at r into jg[3j + q] (lanes over
+// partners, i's slot zero), FP64.  No barrier.
+__device__ __forceinline__ void drift_terms(const SJSysDev &S, const double *nuc, const double *pos, int i,
+                                            const double *r, double *jg, int t, int L) {
   const int N = S.N, si = i < S.n_up ? 0 : 1;
+#pragma unroll 1
   for (int j = t; j < N + S.n_nuc; j += L) {
     double *o = jg + 3 * j;
-    if (j < N) {
-      if (j == i) {
-        o[0] = o[1] = o[2] = 0.0;
-        continue;
-      }
-      const double *xj = pos + 3 * j;
-      const double dv0 = r[0] - xj[0], dv1 = r[1] - xj[1], dv2 = r[2] - xj[2];
-      const double rr = norm3(dv0, dv1, dv2);
-      const double b = ((j < S.n_up ? 0 : 1) == si) ? S.p[1] : S.p[0];
-      const double den = 1.0 + S.p[2] * rr;
-      const double up = b / (den * den);
-      o[0] = up * dv0 / rr;
-      o[1] = up * dv1 / rr;
-      o[2] = up * dv2 / rr;
-    } else {
-      const int I = j - N;
-      const double d0 = r[0] - S.nuc[3 * I], d1 = r[1] - S.nuc[3 * I + 1], d2 = r[2] - S.nuc[3 * I + 2];
-      const double rr = norm3(d0, d1, d2);
-      const double den = 1.0 + S.p[4] * rr;
-      const double vp = -(S.p[3] * S.charge[I]) / (den * den);
-      o[0] = vp * d0 / rr;
-      o[1] = vp * d1 / rr;
-      o[2] = vp * d2 / rr;
-    }
+    const bool el = j < N;
+    const double *xj = el ? pos + 3 * j : nuc + 4 * (j - N);
+    const double d0 = r[0] - xj[0], d1 = r[1] - xj[1], d2 = r[2] - xj[2];
+    const double rr = norm3(d0, d1, d2);
+    // b/(1 + c r)^2 of a pair, -(a Z)/(1 + d r)^2 of a nucleus
+    const double num = el ? (((j < S.n_up ? 0 : 1) == si) ? S.p[1] : S.p[0]) : xj[3];
+    const double den = 1.0 + (el ? S.p[2] : S.p[4]) * rr;
+    const double up = num / (den * den);
+    const bool self = j == i;
+    o[0] = self ? 0.0 : up * d0 / rr;
+    o[1] = self ? 0.0 : up * d1 / rr;
+    o[2] = self ? 0.0 : up * d2 / rr;
   }
 }
 
 // Orbital gradients og[3k + q] = sum_m c_km gch[3m + q] (lanes over
 // orbitals, chains in m order).  No barrier.
-__device__ __forceinline__ void orbital_gradients(const SJSysDev &S, int n, const double *gch, double *og,
-                                                  int t, int L) {
+__device__ __forceinline__ void orbital_gradients(const SJSysDev &S, const SJTab &tab, int n, const double *gch,
+                                                  double *og, int t, int L) {
   const int K = S.n_basis, no = S.n_orb;
   for (int k = t; k < n; k += L) {
-    const double *cf = S.coef_t + k;
     double g0 = 0.0, g1 = 0.0, g2 = 0.0;
     for (int m = 0; m < K; ++m) {
-      const double cm = cf[(size_t)m * no];
+      const double cm = tab.has_coef ? tab.coef[m * no + k] : S.coef_t[(size_t)m * no + k];
       g0 = fma(cm, gch[3 * m], g0);
       g1 = fma(cm, gch[3 * m + 1], g1);
       g2 = fma(cm, gch[3 * m + 2], g2);
@@ -831,8 +863,10 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
   const SJLayout lay(N, nu, nd, nn, S.n_basis, (int)sizeof(T), np, PROP);
   // shared by the workgroup: the sample sums' factor pairs, the nuclei
   uint8_t *pairs = lds;
-  double *nuc = (double *)(lds + kSJPairBytes);
-  unsigned char *walkers = lds + sj_lds_shared(nn);
+  const SJShared sh(nn, S.n_basis, S.n_orb);
+  double *nuc = (double *)(lds + sh.nuc);
+  unsigned char *walkers = lds + sh.bytes;
+  const SJTab tab{nuc, (const double *)(lds + sh.fn), (const double *)(lds + sh.coef), sh.has_fn, sh.has_coef};
   unsigned char *base = walkers + (size_t)slot * lay.bytes;
   SJWalker<T> wk;
   wk.pos = (double *)(base + lay.pos);
@@ -889,8 +923,18 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
     }
     pairs[lane] = (uint8_t)(fa | fb << 4);
   }
-  SJLaneBasis lb;
-  lb.load(S, t);
+  if (tab.has_fn)
+    for (int m = lane; m < S.n_basis; m += 64) {
+      double *e = (double *)(lds + sh.fn) + 5 * m;
+      const int I = S.center[m];
+      e[0] = S.nuc[3 * I];
+      e[1] = S.nuc[3 * I + 1];
+      e[2] = S.nuc[3 * I + 2];
+      e[3] = S.zeta[m];
+      e[4] = __longlong_as_double((long long)S.kind[m]);
+    }
+  if (tab.has_coef)
+    for (int e = lane; e < S.n_basis * S.n_orb; e += 64) ((double *)(lds + sh.coef))[e] = S.coef_t[e];
   SJBooks bk{{1.0, 0.0, 1.0, 0.0}, 0.0, 0.0, 0.0};
   double block_sum = 0.0, acc_in = 0.0;
   [[maybe_unused]] double dmc_el = 0.0, dmc_w = 0.0, dmc_eref = 0.0;
@@ -1024,10 +1068,10 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
           xn[2] = wk.mv[2];
         } else {
           // drift at x (metrop.rs:150-163): x' = (x_i + tau v) + sqrt(tau) z
-          basis_to_lds(S, lb, xi, wk.chi, t, L, gto, pk);
-          drift_terms(S, wk.pos, i, xi, wk.chi, gch, jg, t, L, gto, pk);
+          basis_gradients_to_lds(S, tab, xi, wk.chi, gch, t, L);
+          drift_terms(S, nuc, wk.pos, i, xi, jg, t, L);
           sync_wave();
-          orbital_gradients(S, n, gch, og, t, L);
+          orbital_gradients(S, tab, n, gch, og, t, L);
           sync_wave();
           drift_sum<T>(og, B, n, c, jg, M, 1.0, v);
           for (int q = 0; q < 3; ++q) xn[q] = (xi[q] + v[q] * a.tau) + a.sqrt_tau * wk.rng[4 * i + q];
@@ -1044,11 +1088,15 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
           wk.jn[j] = j == i ? (T)0 : fn;
           wk.jo[j] = j == i ? (T)0 : fo;
         }
-        basis_to_lds(S, lb, xn, wk.chi, t, L, gto, pk);
-        if constexpr (PROP == kSJPropDiffuse) drift_terms(S, wk.pos, i, xn, wk.chi, gch, jg, t, L, gto, pk);
+        if constexpr (PROP == kSJPropDiffuse) {
+          basis_gradients_to_lds(S, tab, xn, wk.chi, gch, t, L);
+          drift_terms(S, nuc, wk.pos, i, xn, jg, t, L);
+        } else {
+          basis_to_lds(S, tab, xn, wk.chi, t, L, gto, pk);
+        }
         sync_wave();
-        for (int k = t; k < n; k += L) wk.phin[k] = (T)orbital_value(S, k, wk.chi);
-        if constexpr (PROP == kSJPropDiffuse) orbital_gradients(S, n, gch, og, t, L);
+        for (int k = t; k < n; k += L) wk.phin[k] = (T)orbital_value(S, tab, k, wk.chi);
+        if constexpr (PROP == kSJPropDiffuse) orbital_gradients(S, tab, n, gch, og, t, L);
         sync_wave();
         // sum_k phi_k(r') B[k][l] of every column l: the determinant ratio for
         // l = c, the Sherman-Morrison coefficients (times 1/ratio) for the rest
@@ -1133,7 +1181,7 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
         // re-inversion, refresh 2 keeping the inverses; after lu_period moves the
         // FP64 log|det| the update chain carried is checked against it
         const bool wb = sweep || a.init || a.refresh == 1;
-        refresh_walker<T>(S, lb, wk, bk, t, L, gto, pk, wb, wb, track_ld ? (sweep ? 2 : 1) : 0);
+        refresh_walker<T>(S, tab, wk, bk, t, L, gto, pk, wb, wb, track_ld ? (sweep ? 2 : 1) : 0);
       }
     }
     if (sweep && t == 0 && live && S.trace_mask && ls.trace_sweeps + sw < a.cap_sweeps)

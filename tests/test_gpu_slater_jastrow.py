@@ -668,3 +668,18 @@ def test_configurations_round_trip_through_staged_transfers(N, W):
     with M.Context([M.slater_jastrow(sj, W)], seed=1, step=0.5, block_size=2) as ctx:
         ctx.set_configs(cfg)
         assert np.array_equal(bits(ctx.get_configs()), bits(cfg))
+
+
+@pytest.mark.parametrize("proposal", [M.PROPOSAL_BOX, M.PROPOSAL_DIFFUSE])
+@pytest.mark.parametrize("n,per", [(4, 2), (3, 3), (5, 2), (8, 2), (9, 2)])
+def test_shared_basis_tables_at_their_edges(n, per, proposal):
+    # basis tables in LDS up to 8 functions (8: yes; 9, 10, 16, 18: no) and
+    # coefficients up to 512 bytes (128, 144, 240, 512: yes; 720: no)
+    system = S.hydrogen_chain(n, basis_per_nucleus=per, seed=2)
+    W, steps, B = 37, 6, 2
+    side = 0.6 if proposal == M.PROPOSAL_BOX else 0.05
+    d = run_device([system], W, steps, B, lu=7, seed=4, side=side, proposal=proposal)[0]
+    o = run_oracle(system, W, steps, B, lu=7, seed=4, side=side, proposal=proposal)
+    assert np.array_equal(d["masks"], o["accept_mask"])
+    assert np.array_equal(bits(d["cfg"]), bits(o["cfg"]))
+    assert np.max(np.abs(d["el"] - o["e_local"]) / np.maximum(1.0, np.abs(o["e_local"]))) <= E_TOL
