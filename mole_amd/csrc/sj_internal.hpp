@@ -151,7 +151,7 @@ size_t sj_lds_per_walker(int N, int nu, int nd, int nn, int K, int tsize, int np
 size_t sj_lds_per_group(int nn, int K, int n_orb);
 // Doubles read past the end of the coefficient table (register chunks of the
 // local energy): the host pads it.
-constexpr int kSJCoefPad = 8;
+constexpr int kSJCoefPad = 10;
 
 // Draws start at draw_base + D N sweeps_done (D draws per move of the
 // proposal) and moves at move_base + N sweeps_done for every system; sample

@@ -60,8 +60,8 @@ struct SJLayout {
     og = gch + (prop == kSJPropDiffuse ? 24u * K : 0u);
     jg = og + (prop == kSJPropDiffuse ? 24u * n : 0u);
     uint32_t end = jg + (prop == kSJPropDiffuse ? 24u * M : 0u);
-    // Gauss-Jordan: A, then I and the pivot column (the basis values while A is built)
-    const uint32_t second = n * n + n > (uint32_t)K ? n * n + n : (uint32_t)K;
+    // Gauss-Jordan: A, then I (the basis values while A is built)
+    const uint32_t second = n * n > (uint32_t)K ? n * n : (uint32_t)K;
     const uint32_t lu = scr + 8u * (n * n + second);
     end = end > lu ? end : lu;
     // per-electron local-energy results, then (1, E, d ln psi/dp)
@@ -215,21 +215,32 @@ __device__ __forceinline__ void basis_gradients_to_lds(const SJSysDev &S, const 
   }
 }
 
-// Sequential sums whose loads are issued U at a time ahead of the
-// arithmetic: the same operations in the same order as a plain loop, with
-// the LDS/cache latency paid once per group instead of once per term.
-template <int U, typename T>
-__device__ __forceinline__ T seq_sum(const T *x, int n) {
-  T s = (T)0;
+// Sequential sums whose loads are issued ahead of the arithmetic, eight bytes
+// at a time (x is 8-byte aligned): the same operations in the same order as a
+// plain loop.
+__device__ __forceinline__ double seq_sum(const double *x, int n) {
+  double s = 0.0;
   int j = 0;
-  for (; j + U <= n; j += U) {
-    T v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = x[j + u];
-#pragma unroll
-    for (int u = 0; u < U; ++u) s = s + v[u];
+  for (; j + 4 <= n; j += 4) {
+    const double a = x[j], b = x[j + 1], c = x[j + 2], d = x[j + 3];
+    s = (((s + a) + b) + c) + d;
   }
   for (; j < n; ++j) s = s + x[j];
+  return s;
+}
+__device__ __forceinline__ float seq_sum(const float *x, int n) {
+  struct alignas(8) F2 {
+    float a, b;
+  };
+  const F2 *v = (const F2 *)x;
+  float s = 0.0f;
+  int j = 0;
+  for (; 2 * j + 8 <= n; j += 4) {
+    const F2 p = v[j], q = v[j + 1], r = v[j + 2], t = v[j + 3];
+    s = (((s + p.a) + p.b) + q.a) + q.b;
+    s = (((s + r.a) + r.b) + t.a) + t.b;
+  }
+  for (j *= 2; j < n; ++j) s = s + x[j];
   return s;
 }
 
@@ -334,7 +345,7 @@ __device__ __forceinline__ SJRefresh refresh_spin(const SJSysDev &S, const SJTab
   if (n == 0) return res;
   const int first = s == 0 ? 0 : S.n_up;
   T *B = s == 0 ? wk.Bup : wk.Bdn;
-  double *M = wk.scr, *I = wk.scr + n * n, *colp = wk.scr + 2 * n * n, *chi = I;
+  double *M = wk.scr, *I = wk.scr + n * n, *chi = I;
   sync_wave();
   for (int c = 0; c < n; ++c) {
     basis_to_lds(S, tab, wk.pos + 3 * (first + c), chi, t, L, gto, pk);
@@ -371,23 +382,37 @@ __device__ __forceinline__ SJRefresh refresh_spin(const SJSysDev &S, const SJTab
     }
     sync_wave();
     const double ip = bad ? 0.0 : 1.0 / pv;
-    // rows p and piv swapped, row p scaled
+    // rows p and piv swapped, row p scaled (columns of A before p are done with)
     for (int j = t; j < n; j += L) {
       const double mp = M[p * n + j], mv = M[piv * n + j], ap = I[p * n + j], av = I[piv * n + j];
-      M[piv * n + j] = mp;
+      if (j >= p) {
+        M[piv * n + j] = mp;
+        M[p * n + j] = mv * ip;
+      }
       I[piv * n + j] = ap;
-      M[p * n + j] = mv * ip;
       I[p * n + j] = av * ip;
     }
     sync_wave();
-    for (int r = t; r < n; r += L) colp[r] = M[r * n + p];
-    sync_wave();
-    // row p's own column entry was just scaled; colp[p] is unused
-    for (int e = t; e < n * n; e += L) {
-      const int r = small_div(e, inv_n), j = e - r * n;
+    // the other rows, one to a lane: row r needs its own element of column p
+    // and row p only
+    for (int r = t; r < n; r += L) {
       if (r == p) continue;
-      M[e] = fma(-colp[r], M[p * n + j], M[e]);
-      I[e] = fma(-colp[r], I[p * n + j], I[e]);
+      const double f = -M[r * n + p];
+      auto sweep_row = [&](double *x, const double *y, int j) {
+        for (; j + 4 <= n; j += 4) {
+          double v[4], w[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            v[u] = x[j + u];
+            w[u] = y[j + u];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) x[j + u] = fma(f, w[u], v[u]);
+        }
+        for (; j < n; ++j) x[j] = fma(f, y[j], x[j]);
+      };
+      sweep_row(M + r * n, M + p * n, p + 1);
+      sweep_row(I + r * n, I + p * n, 0);
     }
     sync_wave();
   }
@@ -443,7 +468,10 @@ __device__ __forceinline__ void refresh_walker(const SJSysDev &S, const SJTab &t
 // parameter derivatives in registers; the electrons' results are then added in
 // electron order.  Every sum has a fixed order, so the result does not depend
 // on L.
-constexpr int kSJLanesNMax = 8;  // orbitals per register chunk
+// Orbitals per register chunk: 10 take a spin block of up to 10 in one pass
+// over the basis and the largest (20) in two (with 8, 9 electrons per spin
+// evaluated every basis function twice, and 18 three times).
+constexpr int kSJLanesNMax = 10;
 
 // The pieces of the local energy the operator terms need (sub-lane 0).
 struct SJParts {
@@ -566,6 +594,7 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
   double *res = wk.le;
   const int RS = 8 + S.opt_exp;
   const bool kinds = (EXT && S.any_gto) || S.any_p;
+  const int nmax = S.n_up > S.n_dn ? S.n_up : S.n_dn;
   sync_wave();
   for (int i = t; i < N; i += L) {
     const int s = i < S.n_up ? 0 : 1;
@@ -573,13 +602,13 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
     const int n = s == 0 ? S.n_up : S.n_dn;
     const T *B = s == 0 ? wk.Bup : wk.Bdn;
     const double xi[3] = {wk.pos[3 * i], wk.pos[3 * i + 1], wk.pos[3 * i + 2]};
-    // orbitals in register chunks of kCh; the basis values are recomputed
-    // per chunk (bit-identical each time), and the chunks add in orbital
-    // order, so the width does not change the sums.  The extended
-    // instantiations (DMC, operators, Gaussians) carry more live state and
-    // take 6, which keeps their spills down.  Coefficients past the last
-    // orbital are read (the table is padded) and their chains not used.
-    constexpr int kCh = EXT ? 6 : kSJLanesNMax;
+    // orbitals in register chunks of two halves; the basis values are
+    // recomputed per chunk (bit-identical each time), and the chunks add in
+    // orbital order, so the width does not change the sums.  Coefficients past
+    // the last orbital are read (the table is padded) and their chains not used.
+    // The extended instantiations (DMC, operators, Gaussians) carry more live
+    // state and take 6, which keeps their spills down.
+    constexpr int kHalf = EXT ? 3 : kSJLanesNMax / 2, kCh = 2 * kHalf;
     double Dg0 = 0.0, Dg1 = 0.0, Dg2 = 0.0, Dl = 0.0;
 #pragma unroll 1
     for (int k0 = 0; k0 < n; k0 += kCh) {
@@ -617,14 +646,18 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
           basis_vgl_sto(kd, z, d0, d1, d2, e, ir, ch, g0, g1, g2, lc);
         }
         const double *cm = S.coef_t + (size_t)m * no + k0;
+        auto half = [&](int h) {
 #pragma unroll
-        for (int k = 0; k < kCh; ++k) {
-          const double cv = cm[k];
-          og[k][0] = fma(cv, g0, og[k][0]);
-          og[k][1] = fma(cv, g1, og[k][1]);
-          og[k][2] = fma(cv, g2, og[k][2]);
-          og[k][3] = fma(cv, lc, og[k][3]);
-        }
+          for (int k = h; k < h + kHalf; ++k) {
+            const double cv = cm[k];
+            og[k][0] = fma(cv, g0, og[k][0]);
+            og[k][1] = fma(cv, g1, og[k][1]);
+            og[k][2] = fma(cv, g2, og[k][2]);
+            og[k][3] = fma(cv, lc, og[k][3]);
+          }
+        };
+        half(0);
+        if (nmax - k0 > kHalf) half(kHalf);  // the same for all lanes
       }
 #pragma unroll
       for (int k = 0; k < kCh; ++k)
@@ -1103,8 +1136,8 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
         for (int l = t; l < n; l += L) wk.dots[l] = seq_dot<8>(wk.phin, B + l, n, n);
         sync_wave();
         const T rd = wk.dots[c];
-        const T Jn = seq_sum<8>(wk.jn, M);
-        const T Jo = seq_sum<8>(wk.jo, M);
+        const T Jn = seq_sum(wk.jn, M);
+        const T Jo = seq_sum(wk.jo, M);
         const T dJ = Jn - Jo;
         const double rdd = (double)rd;
         const double R2 = (rdd * rdd) * exp_m(2.0 * (double)dJ);

@@ -683,3 +683,16 @@ def test_shared_basis_tables_at_their_edges(n, per, proposal):
     assert np.array_equal(d["masks"], o["accept_mask"])
     assert np.array_equal(bits(d["cfg"]), bits(o["cfg"]))
     assert np.max(np.abs(d["el"] - o["e_local"]) / np.maximum(1.0, np.abs(o["e_local"]))) <= E_TOL
+
+
+@pytest.mark.parametrize("N", [10, 11, 20, 21, 22, 40])
+def test_spin_blocks_at_the_chunk_edges(N):
+    # spin blocks of 5, 6, 10, 11 and 20: the halves and chunks of the local
+    # energy's orbital registers and the rows of the re-inversion (every 5 moves)
+    system = S.hydrogen_chain(N, seed=6)
+    W, steps, B = 9, 4, 2
+    d = run_device([system], W, steps, B, lu=5, seed=2)[0]
+    o = run_oracle(system, W, steps, B, lu=5, seed=2)
+    assert np.array_equal(d["masks"], o["accept_mask"])
+    assert np.array_equal(bits(d["cfg"]), bits(o["cfg"]))
+    assert np.max(np.abs(d["el"] - o["e_local"]) / np.maximum(1.0, np.abs(o["e_local"]))) <= E_TOL
