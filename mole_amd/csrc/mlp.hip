@@ -99,22 +99,24 @@ __global__ void mlp_pack_kernel(const float *w, bf16x4 *fwd1, bf16x8 *fwd, bf16x
   }
 }
 
-// LDS transpose of one accumulator-layout tile T (lane l: T[4q + j][l % 16])
-// into the operand layout lane l: T[l % 16][4q + j], rounded to bf16.
-__device__ __forceinline__ bf16x4 transpose_tile(f32x4 v, float *stage) {
-  const int l = threadIdx.x & 63, r = l % 16, q = l / 16;
+// Transposition through LDS of NT accumulator-layout tiles T (lane l:
+// T[4q + j][l % 16]) into the operand layout (lane l: T[l % 16][4q + j]),
+// rounded to bf16.  The tiles are rounded first and go out together, so a batch
+// waits for LDS once; rows of 20 values keep a quarter-wave's 2-byte stores and
+// the 8-byte loads on different banks.  stage: NT kStageTile values.
+constexpr int kStageTile = 16 * 20, kStageTiles = 8;
+template <int NT>
+__device__ __forceinline__ void transpose_tiles(const bf16x4 (&v)[NT], bf16x4 (&o)[NT], short *stage, int l) {
+  const int r = l % 16, q = l / 16;
+  static_assert(NT <= kStageTiles, "the stage's tiles");
   __syncthreads();
-  for (int j = 0; j < 4; ++j) stage[(4 * q + j) * 16 + r] = v[j];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) stage[n * kStageTile + (4 * q + j) * 20 + r] = v[n][j];
   __syncthreads();
-  f32x4 t;
-  for (int j = 0; j < 4; ++j) t[j] = stage[r * 16 + 4 * q + j];
-  return to_bf16x4(t);
-}
-
-__device__ __forceinline__ f32x4 bf16x4_to_f32(bf16x4 b) {
-  f32x4 r;
-  for (int j = 0; j < 4; ++j) r[j] = bf16_float((uint16_t)b[j]);
-  return r;
+#pragma unroll
+  for (int n = 0; n < NT; ++n) o[n] = *(const bf16x4 *)(stage + n * kStageTile + r * 20 + 4 * q);
 }
 
 // dW[in][out] (+)= Xa^T dZa + Xb^T dZb over the wave's 16 samples of two
@@ -123,28 +125,33 @@ __device__ __forceinline__ f32x4 bf16x4_to_f32(bf16x4 b) {
 // Input tiles X (operand layout, lane l: X^T[in 16 mi + l%16][s 4q+j]) and
 // output-gradient tiles D (operand layout of dZ^T).  store: this
 // workgroup's first contribution to its partial, written without reading it.
-__device__ __forceinline__ void weight_grads2(const bf16x4 *Xa, const bf16x4 *Da, const bf16x4 *Xb,
-                                              const bf16x4 *Db, int n_in_tiles, int n_out_tiles, int woff,
-                                              int boff, int nin, int nout, float *g, bool store) {
-  const int l = threadIdx.x & 63, r = l % 16, q = l / 16;
+template <int IN_TILES, int OUT_TILES, int NIN, int NOUT>
+__device__ __forceinline__ void weight_grads2(const bf16x4 *Xa, const bf16x4 *Da, const bf16x4 *Xb, const bf16x4 *Db,
+                                              int woff, int boff, float *g, bool store, int l) {
+  const int r = l % 16, q = l / 16;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   bf16x4 ones;
   for (int j = 0; j < 4; ++j) ones[j] = (short)0x3F80;  // bf16 1.0
-  for (int no = 0; no < n_out_tiles; ++no) {
-    const int out = 16 * no + r;
-    for (int mi = 0; mi < n_in_tiles; ++mi) {
-      const f32x4 d = mfma16(Xb[mi], Db[no], mfma16(Xa[mi], Da[no], zero));
-      for (int j = 0; j < 4; ++j) {
-        const int in = 16 * mi + 4 * q + j;
-        if (in < nin && out < nout) {
-          float *gp = g + woff + in * nout + out;
-          *gp = store ? d[j] : *gp + d[j];
-        }
-      }
-    }
+  const uint32_t at = (uint32_t)(4 * q * NOUT + r);  // a lane's offset from each tile element's uniform address
+#pragma unroll
+  for (int no = 0; no < OUT_TILES; ++no) {
+    const bool out_ok = NOUT % 16 == 0 || 16 * no + r < NOUT;
+    f32x4 d[IN_TILES];
+#pragma unroll
+    for (int mi = 0; mi < IN_TILES; ++mi) d[mi] = mfma16(Xa[mi], Da[no], zero);
+#pragma unroll
+    for (int mi = 0; mi < IN_TILES; ++mi) d[mi] = mfma16(Xb[mi], Db[no], d[mi]);
     const f32x4 db = mfma16(ones, Db[no], mfma16(ones, Da[no], zero));
-    if (q == 0 && out < nout) {
-      float *gp = g + boff + out;
+#pragma unroll
+    for (int mi = 0; mi < IN_TILES; ++mi)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (out_ok && (NIN % 16 == 0 || 16 * mi + 4 * q + j < NIN)) {
+          float *gp = (g + woff + (16 * mi + j) * NOUT + 16 * no) + at;
+          *gp = store ? d[mi][j] : *gp + d[mi][j];
+        }
+    if (q == 0 && out_ok) {
+      float *gp = (g + boff + 16 * no) + (uint32_t)r;
       *gp = store ? db[0] : *gp + db[0];
     }
   }
@@ -154,73 +161,84 @@ __device__ __forceinline__ void weight_grads2(const bf16x4 *Xa, const bf16x4 *Da
 // layer: a with output gradient dOa, activation tiles ha (registers) and
 // bf16 input operand xa; b with dOb, its activation tiles in LDS (hb[k][l])
 // and xb.  Adds (stores, with store) both passes' dO/dtheta into g: each
-// weight-gradient element is read and written once for the two passes.
-__device__ void mlp_backward2(const MlpDev &net, f32x4 dOa, const f32x4 *ha, bf16x4 xa, f32x4 dOb,
-                              const f32x4 (*hb)[64], bf16x4 xb, float *stage, float *g, bool store) {
-  const int l = threadIdx.x & 63;
+// weight-gradient element is read and written once for the two passes.  l:
+// the lane.
+__device__ __forceinline__ void mlp_backward2(const MlpDev &net, f32x4 dOa, const f32x4 *ha, bf16x4 xa, f32x4 dOb,
+                                              const f32x4 (*hb)[64], bf16x4 xb, short *stage, float *g, bool store,
+                                              int l) {
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  bf16x4 Xa[4], Da[4], Xb[4], Db[4];
+  bf16x4 Xt[8], Dt[8], v[8];  // operands of pass a in 0..3, of pass b in 4..7
   f32x4 dza[4], dzb[4];
-  // layer 4 (64 -> 4)
-  Da[0] = transpose_tile(dOa, stage);
-  Db[0] = transpose_tile(dOb, stage);
-  for (int mi = 0; mi < 4; ++mi) {
-    Xa[mi] = transpose_tile(ha[8 + mi], stage);
-    Xb[mi] = transpose_tile(hb[8 + mi][l], stage);
-  }
-  weight_grads2(Xa, Da, Xb, Db, 4, 1, kMlpW4, kMlpB4, kMlpHid, kMlpOut, g, store);
-  {
-    const bf16x4 oa = to_bf16x4(dOa), ob = to_bf16x4(dOb);
-    for (int mt = 0; mt < 4; ++mt) {
-      const f32x4 A = mfma16(net.bwd[(kBwdL4 + mt) * 64 + l], oa, zero);
-      const f32x4 B = mfma16(net.bwd[(kBwdL4 + mt) * 64 + l], ob, zero);
-      const f32x4 tha = ha[8 + mt], thb = hb[8 + mt][l];
-      for (int j = 0; j < 4; ++j) {
-        dza[mt][j] = A[j] * (1.0f - tha[j] * tha[j]);
-        dzb[mt][j] = B[j] * (1.0f - thb[j] * thb[j]);
-      }
+  auto activations = [&](int k0) {
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi) {
+      v[mi] = to_bf16x4(ha[k0 + mi]);
+      v[4 + mi] = to_bf16x4(hb[k0 + mi][l]);
     }
+    transpose_tiles(v, Xt, stage, l);
+  };
+  auto through_tanh = [&](int k0, int mt, f32x4 A, f32x4 B) {
+    const f32x4 tha = ha[k0 + mt], thb = hb[k0 + mt][l];
+    for (int j = 0; j < 4; ++j) {
+      dza[mt][j] = A[j] * (1.0f - tha[j] * tha[j]);
+      dzb[mt][j] = B[j] * (1.0f - thb[j] * thb[j]);
+    }
+  };
+  // layer 4 (64 -> 4)
+  {
+    bf16x4 w[4];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) w[mt] = (net.bwd + (kBwdL4 + mt) * 64)[(uint32_t)l];
+    const bf16x4 oa = to_bf16x4(dOa), ob = to_bf16x4(dOb);
+    const bf16x4 d2[2] = {oa, ob};
+    bf16x4 t2[2];
+    transpose_tiles(d2, t2, stage, l);
+    activations(8);
+    weight_grads2<4, 1, kMlpHid, kMlpOut>(Xt, t2, Xt + 4, t2 + 1, kMlpW4, kMlpB4, g, store, l);
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) through_tanh(8, mt, mfma16(w[mt], oa, zero), mfma16(w[mt], ob, zero));
   }
-  // layers 3 and 2 (64 -> 64)
+  // layers 3 and 2 (64 -> 64): inputs h2, then h1
+#pragma unroll
   for (int layer = 2; layer >= 1; --layer) {
-    const int hin = layer == 2 ? 4 : 0;  // inputs of this layer: h2 (layer 3) or h1 (layer 2)
+    const int hin = layer == 2 ? 4 : 0;
     const int woff = layer == 2 ? kMlpW3 : kMlpW2, boff = layer == 2 ? kMlpB3 : kMlpB2;
     const int bfr = layer == 2 ? kBwdL3 : kBwdL2;
+    // the layer's weight fragments on their way while the tiles are transposed
+    bf16x4 w[16];
+#pragma unroll
+    for (int f = 0; f < 16; ++f) w[f] = (net.bwd + (bfr + f) * 64)[(uint32_t)l];
+    bf16x4 z[8];
+#pragma unroll
     for (int no = 0; no < 4; ++no) {
-      Da[no] = transpose_tile(dza[no], stage);
-      Db[no] = transpose_tile(dzb[no], stage);
+      z[no] = to_bf16x4(dza[no]);
+      z[4 + no] = to_bf16x4(dzb[no]);
     }
-    for (int mi = 0; mi < 4; ++mi) {
-      Xa[mi] = transpose_tile(ha[hin + mi], stage);
-      Xb[mi] = transpose_tile(hb[hin + mi][l], stage);
-    }
-    weight_grads2(Xa, Da, Xb, Db, 4, 4, woff, boff, kMlpHid, kMlpHid, g, store);
-    bf16x4 za[4], zb[4];
-    for (int kc = 0; kc < 4; ++kc) {
-      za[kc] = to_bf16x4(dza[kc]);
-      zb[kc] = to_bf16x4(dzb[kc]);
-    }
+    transpose_tiles(z, Dt, stage, l);
+    activations(hin);
+    weight_grads2<4, 4, kMlpHid, kMlpHid>(Xt, Dt, Xt + 4, Dt + 4, woff, boff, g, store, l);
+#pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
       f32x4 A = zero, B = zero;
+#pragma unroll
       for (int kc = 0; kc < 4; ++kc) {
-        A = mfma16(net.bwd[(bfr + mt * 4 + kc) * 64 + l], za[kc], A);
-        B = mfma16(net.bwd[(bfr + mt * 4 + kc) * 64 + l], zb[kc], B);
+        A = mfma16(w[mt * 4 + kc], z[kc], A);
+        B = mfma16(w[mt * 4 + kc], z[4 + kc], B);
       }
-      const f32x4 tha = ha[hin + mt], thb = hb[hin + mt][l];
-      for (int j = 0; j < 4; ++j) {
-        dza[mt][j] = A[j] * (1.0f - tha[j] * tha[j]);
-        dzb[mt][j] = B[j] * (1.0f - thb[j] * thb[j]);
-      }
+      through_tanh(hin, mt, A, B);
     }
   }
   // layer 1 (13 -> 64): inputs are the features
+#pragma unroll
   for (int no = 0; no < 4; ++no) {
-    Da[no] = transpose_tile(dza[no], stage);
-    Db[no] = transpose_tile(dzb[no], stage);
+    v[no] = to_bf16x4(dza[no]);
+    v[4 + no] = to_bf16x4(dzb[no]);
   }
-  Xa[0] = transpose_tile(bf16x4_to_f32(xa), stage);
-  Xb[0] = transpose_tile(bf16x4_to_f32(xb), stage);
-  weight_grads2(Xa, Da, Xb, Db, 1, 4, kMlpW1, kMlpB1, kMlpIn, kMlpHid, g, store);
+  transpose_tiles(v, Dt, stage, l);
+  const bf16x4 x2[2] = {xa, xb};
+  bf16x4 t2[2];
+  transpose_tiles(x2, t2, stage, l);
+  weight_grads2<1, 4, kMlpIn, kMlpHid>(t2, Dt, t2 + 1, Dt + 4, kMlpW1, kMlpB1, g, store, l);
 }
 
 // Spin blocks of the training systems hold at most this many electrons.
@@ -230,65 +248,111 @@ constexpr int kMlpMaxSpin = 8;
 // right-hand side e_c of A y = e_c into scr (n^2 + n doubles): the four lanes
 // of a sample (sub = 0..3) build rows sub, sub + 4, ... (each row by the
 // same operations as one lane would).  A barrier must follow.
-__device__ void slater_rows(const SJSysDev &S, const double *cfg, int i, double *scr, int sub) {
+__device__ __forceinline__ void slater_rows(const SJSysDev &S, const double *cfg, int i, double *scr, int sub) {
   const int sp = i < S.n_up ? 0 : 1;
   const int n = sp == 0 ? S.n_up : S.n_dn, first = sp == 0 ? 0 : S.n_up, c = i - first;
   const int K = S.n_basis, no = S.n_orb;
   double *A = scr, *y = scr + n * n;
+#pragma unroll 1
   for (int row = sub; row < n; row += 4) {
-    const double *re = cfg + 3 * (first + row);
-    for (int k = 0; k < n; ++k) A[row * n + k] = 0.0;
+    const double r0 = cfg[3 * (first + row)], r1 = cfg[3 * (first + row) + 1], r2 = cfg[3 * (first + row) + 2];
+    double phi[kMlpMaxSpin];  // the row in registers (coefficients past the last orbital are padding)
+#pragma unroll
+    for (int k = 0; k < kMlpMaxSpin; ++k) phi[k] = 0.0;
+#pragma unroll 1
     for (int m = 0; m < K; ++m) {
       const int I = S.center[m];
-      const double d0 = re[0] - S.nuc[3 * I], d1 = re[1] - S.nuc[3 * I + 1], d2 = re[2] - S.nuc[3 * I + 2];
+      const double d0 = r0 - S.nuc[3 * I], d1 = r1 - S.nuc[3 * I + 1], d2 = r2 - S.nuc[3 * I + 2];
       const double ch = basis_value<false>(S.any_p ? S.kind[m] : MOLE_BASIS_STO, S.zeta[m], d0, d1, d2,
                                            norm3(d0, d1, d2));
-      for (int k = 0; k < n; ++k) A[row * n + k] = fma(S.coef_t[(size_t)m * no + k], ch, A[row * n + k]);
+      const double *cm = S.coef_t + (size_t)m * no;
+#pragma unroll
+      for (int k = 0; k < kMlpMaxSpin; ++k) phi[k] = fma(cm[k], ch, phi[k]);
     }
+#pragma unroll
+    for (int k = 0; k < kMlpMaxSpin; ++k)
+      if (k < n) A[row * n + k] = phi[k];
     y[row] = row == c ? 1.0 : 0.0;
   }
 }
 
+// v summed over a sample's four lanes (l, l ^ 16, l ^ 32, l ^ 48), on all four
+__device__ __forceinline__ double sum4(double v) {
+  v += __shfl_xor(v, 16);
+  return v + __shfl_xor(v, 32);
+}
+
 // ln (psi(x')/psi(x))^2 and grad_{x'} ln|psi(x')| of moving electron i of
-// cfg to xn (FP64, one lane), from the rows slater_rows left in scr:
-// Gaussian elimination with partial pivoting of A y = e_c gives column c of
-// A^-1.
-__device__ void move_terms(const SJSysDev &S, const double *cfg, int i, const double *xn, double *scr,
-                           double *lR2, double *gx) {
+// cfg to xn (FP64), from the rows slater_rows left in scr: Gaussian
+// elimination with partial pivoting of A y = e_c gives column c of A^-1.  The
+// sample's four lanes (sub = 0..3) take the rows below a pivot and the Jastrow
+// partners in turn and search pivots, substitute back and evaluate the
+// orbitals alike; all four return the results.  All lanes of the wave call it.
+__device__ __forceinline__ void move_terms(const SJSysDev &S, const double *cfg, int i, const double *xn, double *scr,
+                                           int sub, double *lR2, double *gx) {
   const int N = S.N, sp = i < S.n_up ? 0 : 1;
   const int n = sp == 0 ? S.n_up : S.n_dn;
+  const int nmax = S.n_up > S.n_dn ? S.n_up : S.n_dn;
   const int K = S.n_basis, no = S.n_orb;
   double *A = scr, *y = scr + n * n;
-  for (int p = 0; p < n; ++p) {
-    int piv = p;
-    for (int r = p + 1; r < n; ++r)
-      if (fabs(A[r * n + p]) > fabs(A[piv * n + p])) piv = r;
-    if (piv != p) {
-      for (int k = 0; k < n; ++k) {
-        const double t = A[p * n + k];
-        A[p * n + k] = A[piv * n + k];
-        A[piv * n + k] = t;
+  // (the samples of a wave may differ in their spin block: the barriers count
+  // to the larger one)
+#pragma unroll 1
+  for (int p = 0; p < nmax; ++p) {
+    if (p < n) {
+      int piv = p;
+      double best = fabs(A[p * n + p]);
+      for (int r = p + 1; r < n; ++r) {
+        const double v = fabs(A[r * n + p]);
+        if (v > best) {
+          best = v;
+          piv = r;
+        }
       }
-      const double t = y[p];
-      y[p] = y[piv];
-      y[piv] = t;
+      if (piv != p)
+        for (int k = p + sub; k <= n; k += 4) {  // column n: y
+          double *u = k < n ? A + p * n + k : y + p, *v = k < n ? A + piv * n + k : y + piv;
+          const double t = *u;
+          *u = *v;
+          *v = t;
+        }
     }
-    for (int r = p + 1; r < n; ++r) {
-      const double f = A[r * n + p] / A[p * n + p];
-      for (int k = p; k < n; ++k) A[r * n + k] = fma(-f, A[p * n + k], A[r * n + k]);
-      y[r] = fma(-f, y[p], y[r]);
+    __syncthreads();
+    if (p < n) {
+      const double app = A[p * n + p], yp = y[p];
+      for (int r = p + 1 + sub; r < n; r += 4) {
+        const double f = A[r * n + p] / app;
+        int k = p + 1;
+        for (; k + 2 <= n; k += 2) {
+          const double a0 = A[p * n + k], a1 = A[p * n + k + 1], b0 = A[r * n + k], b1 = A[r * n + k + 1];
+          A[r * n + k] = fma(-f, a0, b0);
+          A[r * n + k + 1] = fma(-f, a1, b1);
+        }
+        if (k < n) A[r * n + k] = fma(-f, A[p * n + k], A[r * n + k]);
+        y[r] = fma(-f, yp, y[r]);
+      }
+    }
+    __syncthreads();
+  }
+  double ys[kMlpMaxSpin];  // y in registers, n <= kMlpMaxSpin
+#pragma unroll
+  for (int p = kMlpMaxSpin - 1; p >= 0; --p) {
+    ys[p] = 0.0;
+    if (p < n) {
+      double s = y[p];
+#pragma unroll
+      for (int k = p + 1; k < kMlpMaxSpin; ++k)
+        if (k < n) s = fma(-A[p * n + k], ys[k], s);
+      ys[p] = s / A[p * n + p];
     }
   }
-  for (int p = n - 1; p >= 0; --p) {
-    double s = y[p];
-    for (int k = p + 1; k < n; ++k) s = fma(-A[p * n + k], y[k], s);
-    y[p] = s / A[p * n + p];
-  }
-  // orbitals and their gradients at x': each basis function once, the
-  // orbitals' sums over m in m order as before
+  // rd = sum_k phi_k(x') y_k and its gradient: each basis function once, with
+  // its weight sum_k c_km y_k
+  double rd = 0.0, gd[3] = {0.0, 0.0, 0.0};
   double phi[kMlpMaxSpin], g0[kMlpMaxSpin], g1[kMlpMaxSpin], g2[kMlpMaxSpin];
 #pragma unroll
   for (int k = 0; k < kMlpMaxSpin; ++k) phi[k] = g0[k] = g1[k] = g2[k] = 0.0;
+#pragma unroll 1
   for (int m = 0; m < K; ++m) {
     const int I = S.center[m];
     const double d0 = xn[0] - S.nuc[3 * I], d1 = xn[1] - S.nuc[3 * I + 1], d2 = xn[2] - S.nuc[3 * I + 2];
@@ -297,53 +361,47 @@ __device__ void move_terms(const SJSysDev &S, const double *cfg, int i, const do
     basis_vgl<false>(S.any_p ? S.kind[m] : MOLE_BASIS_STO, S.zeta[m], d0, d1, d2, rr, ch, b0, b1, b2, bl);
     const double *cm = S.coef_t + (size_t)m * no;
 #pragma unroll
-    for (int k = 0; k < kMlpMaxSpin; ++k)
-      if (k < n) {
-        phi[k] = fma(cm[k], ch, phi[k]);
-        g0[k] = fma(cm[k], b0, g0[k]);
-        g1[k] = fma(cm[k], b1, g1[k]);
-        g2[k] = fma(cm[k], b2, g2[k]);
-      }
+    for (int k = 0; k < kMlpMaxSpin; ++k) {
+      phi[k] = fma(cm[k], ch, phi[k]);
+      g0[k] = fma(cm[k], b0, g0[k]);
+      g1[k] = fma(cm[k], b1, g1[k]);
+      g2[k] = fma(cm[k], b2, g2[k]);
+    }
   }
-  double rd = 0.0, gd[3] = {0.0, 0.0, 0.0};
-  for (int k = 0; k < n; ++k) {
-    rd = fma(phi[k], y[k], rd);
-    gd[0] = fma(g0[k], y[k], gd[0]);
-    gd[1] = fma(g1[k], y[k], gd[1]);
-    gd[2] = fma(g2[k], y[k], gd[2]);
-  }
-  // Jastrow difference and gradient at x'
+#pragma unroll
+  for (int k = 0; k < kMlpMaxSpin; ++k)
+    if (k < n) {
+      rd = fma(phi[k], ys[k], rd);
+      gd[0] = fma(g0[k], ys[k], gd[0]);
+      gd[1] = fma(g1[k], ys[k], gd[1]);
+      gd[2] = fma(g2[k], ys[k], gd[2]);
+    }
+  // Jastrow difference and gradient at x': electrons, then nuclei, a quarter to
+  // each lane
   const double *r = cfg + 3 * i;
-  const double bA = S.p[0], bP = S.p[1], cc = S.p[2], a = S.p[3], d = S.p[4];
+  const double bA = S.p[0], bP = S.p[1], a = S.p[3];
   double dJ = 0.0, gj[3] = {0.0, 0.0, 0.0};
-  for (int j = 0; j < N; ++j) {
+#pragma unroll 1
+  for (int j = sub; j < N + S.n_nuc; j += 4) {
     if (j == i) continue;
-    const double *xj = cfg + 3 * j;
-    const double b = ((j < S.n_up ? 0 : 1) == sp) ? bP : bA;
+    const bool el = j < N;
+    const double *xj = el ? cfg + 3 * j : S.nuc + 3 * (j - N);
+    // u(r) = num r / (1 + c r): num = b of a pair, -a Z of a nucleus
+    const double num = el ? (((j < S.n_up ? 0 : 1) == sp) ? bP : bA) : -(a * S.charge[j - N]);
+    const double c = el ? S.p[2] : S.p[4];
     const double dv0 = xn[0] - xj[0], dv1 = xn[1] - xj[1], dv2 = xn[2] - xj[2];
     const double rn = norm3(dv0, dv1, dv2);
     const double ro = norm3(r[0] - xj[0], r[1] - xj[1], r[2] - xj[2]);
-    dJ += (b * rn) / (1.0 + cc * rn) - (b * ro) / (1.0 + cc * ro);
-    const double den = 1.0 + cc * rn;
-    const double up = b / (den * den);
+    const double den = 1.0 + c * rn;
+    dJ += (num * rn) / den - (num * ro) / (1.0 + c * ro);
+    const double up = num / (den * den);
     gj[0] += up * dv0 / rn;
     gj[1] += up * dv1 / rn;
     gj[2] += up * dv2 / rn;
   }
-  for (int I = 0; I < S.n_nuc; ++I) {
-    const double aZ = a * S.charge[I];
-    const double d0 = xn[0] - S.nuc[3 * I], d1 = xn[1] - S.nuc[3 * I + 1], d2 = xn[2] - S.nuc[3 * I + 2];
-    const double rn = norm3(d0, d1, d2);
-    const double ro = norm3(r[0] - S.nuc[3 * I], r[1] - S.nuc[3 * I + 1], r[2] - S.nuc[3 * I + 2]);
-    dJ += -(aZ * rn) / (1.0 + d * rn) + (aZ * ro) / (1.0 + d * ro);
-    const double den = 1.0 + d * rn;
-    const double vp = -aZ / (den * den);
-    gj[0] += vp * d0 / rn;
-    gj[1] += vp * d1 / rn;
-    gj[2] += vp * d2 / rn;
-  }
+  dJ = sum4(dJ);
   *lR2 = 2.0 * log_m(fabs(rd)) + 2.0 * dJ;
-  for (int q = 0; q < 3; ++q) gx[q] = gd[q] / rd + gj[q];
+  for (int q = 0; q < 3; ++q) gx[q] = gd[q] / rd + sum4(gj[q]);
 }
 
 // Per-wave LDS of the training kernel.
@@ -351,9 +409,9 @@ struct TrainLds {
   static constexpr int kMaxN = 16, kMaxSpin = kMlpMaxSpin;
   double cfg[16][3 * kMaxN];
   double ge[16][kMaxSpin * kMaxSpin + kMaxSpin];
-  double smp[16][16];      // per sample: x'[3], z[3], mu[3], ls, out3 ... (see below)
+  double smp[16][13];      // per sample: x'[3], z[3], dx[3], ln sigma, sigma, out3 (odd stride)
   f32x4 h1[12][64];        // activations of the forward pass at x
-  float stage[256];
+  alignas(8) short stage[kStageTiles * kStageTile];
   double obj[16];
 };
 
@@ -390,6 +448,7 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(MlpTrainArgs a) {
     const f32x4 o1 = mlp_forward(a.net, x1, h);
     for (int k = 0; k < 12; ++k) s.h1[k][l] = h[k];
     __syncthreads();
+    double *sp = s.smp[sl];
     if (q == 0) {
       Stream st;
       st.init(a.seed, kMlpTrainSys, (uint32_t)gi, (uint32_t)(gi >> 32));
@@ -398,7 +457,6 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(MlpTrainArgs a) {
       box_muller(st.draw(2), st.draw(3), &z[2], &z[3]);
       const double ls = mlp_log_sigma((double)o1[3]);
       const double sg = exp_m(ls);
-      double *sp = s.smp[sl];
       for (int k = 0; k < 3; ++k) {
         sp[k] = (r[k] + (double)o1[k]) + sg * z[k];  // x'
         sp[3 + k] = z[k];
@@ -407,16 +465,11 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(MlpTrainArgs a) {
       sp[9] = ls;
       sp[10] = sg;
       sp[11] = (double)o1[3];
-      double lR2, gx[3];
-      move_terms(S, cfg, i, sp, s.ge[sl], &lR2, gx);
-      sp[12] = lR2;
-      sp[13] = gx[0];
-      sp[14] = gx[1];
-      sp[15] = gx[2];
     }
     __syncthreads();
+    double lR2, gmv[3];
+    move_terms(S, cfg, i, sp, s.ge[sl], q, &lR2, gmv);
     // forward at x' (electron i moved; the inputs are constants of the gradient)
-    const double *sp = s.smp[sl];
     mlp_features(cfg, N, S.nuc, S.n_nuc, i, sp, q, fv);
     const bf16x4 x2 = features_bf16(fv);
     const f32x4 o2 = mlp_forward(a.net, x2, h);
@@ -428,7 +481,7 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(MlpTrainArgs a) {
       const double dm = dn > (double)fv[0] ? dn : (double)fv[0];
       double wgt = a.objective == MOLE_MLP_OBJ_ESJD_RELATIVE ? 1.0 / (dm * dm + kMlpRelD0 * kMlpRelD0) : 1.0;
       const double ls = sp[9], sg = sp[10], ls2 = mlp_log_sigma((double)o2[3]), sg2 = exp_m(ls2);
-      double e[3], dx[3], z[3], gx[3] = {sp[13], sp[14], sp[15]};
+      double e[3], dx[3], z[3], gx[3] = {gmv[0], gmv[1], gmv[2]};
       double e2 = 0.0, z2 = 0.0, d2 = 0.0;
       for (int k = 0; k < 3; ++k) {
         e[k] = (r[k] - sp[k]) - (double)o2[k];
@@ -440,7 +493,7 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(MlpTrainArgs a) {
       }
       const double lq_rev = -3.0 * ls2 - e2 / (2.0 * sg2 * sg2);
       const double lq_fwd = -3.0 * ls - 0.5 * z2;
-      const double logr = sp[12] + lq_rev - lq_fwd;
+      const double logr = lR2 + lq_rev - lq_fwd;
       const double A = logr < 0.0 ? exp_m(logr) : 1.0;
       if (a.objective == MOLE_MLP_OBJ_LOG_ESJD) {
         // d log(eps + O) = dO / (eps + O): the ESJD derivatives scaled by
@@ -467,7 +520,11 @@ __global__ void __launch_bounds__(64) mlp_train_kernel(MlpTrainArgs a) {
       const double dls2 = d2 * Aact * (-3.0 + e2 * is2);
       dO2[3] = (float)(dls2 * mlp_log_sigma_slope(o23));
     }
-    mlp_backward2(a.net, dO2, h, x2, dO1, s.h1, x1, s.stage, g, mb == (int)blockIdx.x);
+    // the lane, opaque: the pass's addresses are not computed ahead of the loop
+    // and held (512 registers and 600 bytes of scratch a lane otherwise)
+    int lo = l;
+    asm volatile("" : "+v"(lo));
+    mlp_backward2(a.net, dO2, h, x2, dO1, s.h1, x1, s.stage, g, mb == (int)blockIdx.x, lo);
   }
   // objective: fixed-order sum over the wave's sample lanes
   __syncthreads();
@@ -492,18 +549,71 @@ __device__ __forceinline__ void adam_update(const MlpAdamStep &a, int p, float g
   a.w[p] = a.w[p] - a.lr * mh / (sqrtf(vh) + a.eps);
 }
 
-// First stage when many workgroups wrote partials: slice h = blockIdx.y of
-// the rows, [h S, min(G, (h + 1) S)) with S = kMlpSlice, summed in row order
-// per parameter into mid[h][p] (loads 16 at a time, added in that order),
-// and the objective partials of the slice into mid_obj[h] by the thread
-// after the last parameter.  Slices in parallel: G = 1,024 partials are
-// read by 32 x 38 workgroups instead of 38.
-__global__ void mlp_reduce_slices_kernel(const float *partial, const double *obj, int G, float *mid,
-                                         double *mid_obj) {
-  constexpr int kBatch = 16;
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  const int g0 = blockIdx.y * kMlpSlice, g1 = min(G, g0 + kMlpSlice);
-  if (p < kMlpParams) {
+// Parameter p's places in the packed fragments (the inverse of
+// mlp_pack_kernel's indexing), written with its updated value.
+__device__ __forceinline__ void pack_param(const MlpAdamStep &a, int p, float w) {
+  const __bf16 b = (__bf16)w;
+  auto weight = [&](int e, int layer, int fwd_frag, int bwd_frag) {
+    // element e = in nout + out of layer `layer`
+    const int nout = layer == 3 ? kMlpOut : kMlpHid;
+    const int in = e / nout, out = e % nout;
+    if (layer == 0) {
+      ((__bf16 *)a.fwd1)[((out / 16) * 64 + (in / 4) * 16 + out % 16) * 4 + in % 4] = b;
+      return;
+    }
+    // forward, K = 32: two 16-feature blocks side by side (pack_k32's order)
+    const int kk = in % 32, half = kk / 16, kq = (kk % 16) / 4, kj = 4 * half + kk % 4;
+    const int frag = fwd_frag + (layer == 3 ? in / 32 : (out / 16) * 2 + in / 32);
+    ((__bf16 *)a.fwd)[(frag * 64 + kq * 16 + out % 16) * 8 + kj] = b;
+    const int bf = bwd_frag + (layer == 3 ? in / 16 : (in / 16) * 4 + out / 16);
+    ((__bf16 *)a.bwd)[(bf * 64 + (out % 16 / 4) * 16 + in % 16) * 4 + out % 4] = b;
+  };
+  if (p < kMlpB1) weight(p - kMlpW1, 0, 0, 0);
+  else if (p < kMlpW2) a.bias[p - kMlpB1] = w;
+  else if (p < kMlpB2) weight(p - kMlpW2, 1, kFwdL2, kBwdL2);
+  else if (p < kMlpW3) a.bias[64 + p - kMlpB2] = w;
+  else if (p < kMlpB3) weight(p - kMlpW3, 2, kFwdL3, kBwdL3);
+  else if (p < kMlpW4) a.bias[128 + p - kMlpB3] = w;
+  else if (p < kMlpB4) weight(p - kMlpW4, 3, kFwdL4, kBwdL4);
+  else a.bias[192 + p - kMlpB4] = w;
+}
+
+// grad[p] = the G partials of parameter p summed in a fixed order: slices of
+// kMlpSlice consecutive rows in row order, then the slice sums in slice order;
+// with do_adam the parameter's Adam step and its new value's places in the
+// packed fragments follow in the same thread, so a training step is this launch
+// after the training kernel (three launches of reductions, Adam and packing
+// took 17 us of a step's 80).  A workgroup takes 32 parameters and a thread one
+// of their slices: rows are read in runs of 128 bytes, G = 1,024 partials by
+// 297 workgroups.  Bound by reading the partials (39 MB at G = 1,024).  The
+// last workgroup sums the objective the same way.
+constexpr int kReduceParams = 32, kReduceSlices = 32;
+static_assert(kReduceSlices * kMlpSlice >= kMlpMaxGroups, "every partial has a slice");
+__global__ void __launch_bounds__(kReduceParams *kReduceSlices)
+    mlp_update_kernel(const float *partial, const double *obj, int G, float *grad, double *obj_sum, MlpAdamStep adam,
+                      int do_adam) {
+  __shared__ float mid[kReduceSlices][kReduceParams];
+  __shared__ double mid_obj[kReduceSlices];
+  const int h = threadIdx.x / kReduceParams, c = threadIdx.x % kReduceParams;
+  const int p = blockIdx.x * kReduceParams + c;
+  const int H = (G + kMlpSlice - 1) / kMlpSlice;
+  const int g0 = h * kMlpSlice, g1 = min(G, g0 + kMlpSlice);
+  if (blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x < H) {
+      double t = 0.0;
+      for (int gi = threadIdx.x * kMlpSlice; gi < min(G, (int)(threadIdx.x + 1) * kMlpSlice); ++gi) t += obj[gi];
+      mid_obj[threadIdx.x] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t = 0.0;
+      for (int k = 0; k < H; ++k) t += mid_obj[k];
+      *obj_sum = t;
+    }
+    return;
+  }
+  if (p < kMlpParams && h < H) {
+    constexpr int kBatch = 16;
     float t = 0.0f;
     int gi = g0;
     for (; gi + kBatch <= g1; gi += kBatch) {
@@ -514,51 +624,19 @@ __global__ void mlp_reduce_slices_kernel(const float *partial, const double *obj
       for (int q = 0; q < kBatch; ++q) t += v[q];
     }
     for (; gi < g1; ++gi) t += partial[(size_t)gi * kMlpParams + p];
-    mid[(size_t)blockIdx.y * kMlpParams + p] = t;
-  } else if (p == kMlpParams) {
-    double t = 0.0;
-    for (int gi = g0; gi < g1; ++gi) t += obj[gi];
-    mid_obj[blockIdx.y] = t;
+    mid[h][c] = t;
   }
-}
-
-// Per parameter the partials of the G workgroups (or the G slice sums of
-// the first stage) summed in order; the loads go out 16 at a time and are
-// added in that order.  With do_adam the thread then takes the Adam step
-// of its parameter.
-__global__ void mlp_reduce_kernel(const float *partial, const double *obj, int G, float *grad, double *obj_sum,
-                                  MlpAdamStep adam, int do_adam) {
-  constexpr int kBatch = 16;
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < kMlpParams) {
+  __syncthreads();
+  if (h == 0 && p < kMlpParams) {
     float t = 0.0f;
-    int gi = 0;
-    for (; gi + kBatch <= G; gi += kBatch) {
-      float v[kBatch];
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) v[q] = partial[(size_t)(gi + q) * kMlpParams + p];
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) t += v[q];
-    }
-    for (; gi < G; ++gi) t += partial[(size_t)gi * kMlpParams + p];
+    for (int k = 0; k < H; ++k) t += mid[k][c];
     grad[p] = t;
-    if (do_adam) adam_update(adam, p, t);
-  }
-  if (p == 0) {
-    double t = 0.0;
-    int gi = 0;
-    for (; gi + kBatch <= G; gi += kBatch) {
-      double v[kBatch];
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) v[q] = obj[gi + q];
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q) t += v[q];
+    if (do_adam) {
+      adam_update(adam, p, t);
+      pack_param(adam, p, adam.w[p]);
     }
-    for (; gi < G; ++gi) t += obj[gi];
-    *obj_sum = t;
   }
 }
-
 
 // out[4 e + k] = network output k for electron electron[e] of configuration e
 __global__ void __launch_bounds__(64) mlp_eval_kernel(MlpDev net, const double *cfg, int N, const double *nuc,
@@ -595,19 +673,12 @@ hipError_t launch_mlp_train(const MlpTrainArgs &a, int n_groups, hipStream_t str
   return hipGetLastError();
 }
 
-hipError_t launch_mlp_reduce(const float *partial, const double *obj, int n_groups, float *mid, double *mid_obj,
-                             float *grad, double *obj_sum, const MlpAdamStep *adam, hipStream_t stream) {
+hipError_t launch_mlp_update(const float *partial, const double *obj, int n_groups, float *grad, double *obj_sum,
+                             const MlpAdamStep *adam, hipStream_t stream) {
   const MlpAdamStep none{};
-  if (n_groups > kMlpSlice) {
-    const int H = (n_groups + kMlpSlice - 1) / kMlpSlice;
-    hipLaunchKernelGGL(mlp_reduce_slices_kernel, dim3((kMlpParams + 1 + 255) / 256, H), dim3(256), 0, stream,
-                       partial, obj, n_groups, mid, mid_obj);
-    partial = mid;
-    obj = mid_obj;
-    n_groups = H;
-  }
-  hipLaunchKernelGGL(mlp_reduce_kernel, dim3((kMlpParams + 255) / 256), dim3(256), 0, stream, partial, obj,
-                     n_groups, grad, obj_sum, adam ? *adam : none, adam ? 1 : 0);
+  hipLaunchKernelGGL(mlp_update_kernel, dim3((kMlpParams + kReduceParams - 1) / kReduceParams + 1),
+                     dim3(kReduceParams * kReduceSlices), 0, stream, partial, obj, n_groups, grad, obj_sum,
+                     adam ? *adam : none, adam ? 1 : 0);
   return hipGetLastError();
 }
 

@@ -41,20 +41,24 @@ hipError_t launch_mlp_pack(const float *w, bf16x4 *fwd1, bf16x8 *fwd, bf16x4 *bw
                            hipStream_t stream);
 hipError_t launch_mlp_train(const MlpTrainArgs &a, int n_groups, hipStream_t stream);
 // One Adam step on the loss -mean(A |dx|^2) (g = -grad / batch) of the FP32
-// master weights; step counts from 1 (bias correction)
+// master weights, whose new values also go into the packed fragments; step
+// counts from 1 (bias correction)
 struct MlpAdamStep {
   float *w, *m, *v;
   float inv_batch, lr, beta1, beta2, eps;
   int step;
+  bf16x4 *fwd1;
+  bf16x8 *fwd;
+  bf16x4 *bwd;
+  float *bias;
 };
-// grad[p] = sum_g partial[g][p], obj_sum = sum_g obj[g] (fixed order: with
-// more than kMlpSlice groups, sums of consecutive slices of kMlpSlice rows
-// into mid [ceil(G / kMlpSlice)][kMlpParams] and mid_obj first, then those in
-// slice order); with adam, the same thread then applies the Adam step to
-// parameter p
-constexpr int kMlpSlice = 32;
-hipError_t launch_mlp_reduce(const float *partial, const double *obj, int n_groups, float *mid, double *mid_obj,
-                             float *grad, double *obj_sum, const MlpAdamStep *adam, hipStream_t stream);
+// grad[p] = sum_g partial[g][p], obj_sum = sum_g obj[g] (fixed order: sums of
+// consecutive slices of kMlpSlice rows, then those in slice order); with adam,
+// the same thread then applies the Adam step to parameter p.  At most
+// kMlpMaxGroups groups.
+constexpr int kMlpSlice = 32, kMlpMaxGroups = 1024;
+hipError_t launch_mlp_update(const float *partial, const double *obj, int n_groups, float *grad, double *obj_sum,
+                             const MlpAdamStep *adam, hipStream_t stream);
 // features and network outputs of given configurations (debug / tests)
 hipError_t launch_mlp_eval(const MlpDev &net, const double *cfg, int N, const double *nuc, int n_nuc,
                            const int *electron, int n, float *out, hipStream_t stream);

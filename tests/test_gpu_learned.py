@@ -285,3 +285,24 @@ def test_features_match_oracle(Z):
     want = np.array([ML.features(wv, cfg[e].ravel(), int(el[e])) for e in range(n)])
     assert np.array_equal(got[:, :13], want.astype(np.float32))
     assert np.all(got[:, 13:] == 0.0)
+
+
+@pytest.mark.parametrize("batch", [16, 512, 528, 16384, 16400])
+def test_update_packs_what_a_reload_of_the_weights_packs(batch):
+    # one group, one slice of 32 partials, a slice of one, all 1,024 groups, a
+    # second minibatch of one group: after training steps the fragments the
+    # update wrote in place give bit for bit the outputs (forward) and the
+    # gradient (forward and backward) of the same weights set afresh
+    sj = S.atom(5)
+    with M.Context([M.slater_jastrow(sj, 64)], seed=3, step=0.3, block_size=10, lu_period=16) as ctx, M.Mlp(4) as net:
+        ctx.init_walkers()
+        net.collect(ctx, 2, 3)
+        net.train(ctx, 3, batch=batch, seed=5, objective=M.MLP_OBJ_LOG_ESJD)
+        cfg = np.random.default_rng(1).normal(size=(40, 15))
+        electron = np.arange(40) % 5
+        out = net.eval(cfg, sj.nuclei, electron)
+        g, o = net.gradient(ctx, 64, seed=9)
+        net.set_weights(net.weights())
+        out2 = net.eval(cfg, sj.nuclei, electron)
+        g2, o2 = net.gradient(ctx, 64, seed=9)
+    assert np.array_equal(out, out2) and np.array_equal(g, g2) and o == o2
