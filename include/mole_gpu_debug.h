@@ -37,6 +37,7 @@ mole_status mole_debug_copy(size_t n_doubles, int32_t repeats, double *ms_per_co
 #define MOLE_DEBUG_BOXMULLER1 10 /* out = second normal */
 #define MOLE_DEBUG_BF16 11    /* out = bf16 round-to-nearest-even of (float)a */
 #define MOLE_DEBUG_SQRT_NORMAL 12 /* out = sqrt(a) by the chain kernels' root, 2^-767 <= a < 2^1000 */
+#define MOLE_DEBUG_RECIP_NORMAL 13 /* out = 1/a without scaling, 2^-500 < |a| < 2^500 */
 mole_status mole_debug_math(int32_t op, size_t n, const double *a, const double *b, double *out);
 
 /* D = A B for 16x16 row-major FP32 matrices rounded to bf16, through one

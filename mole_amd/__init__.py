@@ -84,6 +84,7 @@ DEBUG_BOXMULLER0 = 9
 DEBUG_BOXMULLER1 = 10
 DEBUG_BF16 = 11
 DEBUG_SQRT_NORMAL = 12
+DEBUG_RECIP_NORMAL = 13
 
 
 class MoleError(RuntimeError):

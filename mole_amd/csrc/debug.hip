@@ -31,6 +31,7 @@ __global__ void math_kernel(int op, size_t n, const double *a, const double *b, 
   switch (op) {
     case MOLE_DEBUG_EXP: r = exp_m(x); break;
     case MOLE_DEBUG_SQRT: r = sqrt(x); break;
+    case MOLE_DEBUG_RECIP_NORMAL: r = recip_normal(x); break;
     case MOLE_DEBUG_SQRT_NORMAL: r = sqrt_normal(x); break;
     case MOLE_DEBUG_DIV: r = x / y; break;
     case MOLE_DEBUG_STANDARD: r = u64_standard((uint64_t)__double_as_longlong(x)); break;
@@ -170,7 +171,7 @@ extern "C" mole_status mole_debug_philox(uint64_t seed, uint32_t sys, uint32_t w
 
 extern "C" mole_status mole_debug_math(int32_t op, size_t n, const double *a, const double *b,
                                        double *out) {
-  if (!a || !out || op < 0 || op > MOLE_DEBUG_SQRT_NORMAL) return MOLE_ERR_INVALID_ARGUMENT;
+  if (!a || !out || op < 0 || op > MOLE_DEBUG_RECIP_NORMAL) return MOLE_ERR_INVALID_ARGUMENT;
   if ((op == MOLE_DEBUG_DIV || op == MOLE_DEBUG_RANGE || op == MOLE_DEBUG_NORM3 ||
        op == MOLE_DEBUG_BOXMULLER0 || op == MOLE_DEBUG_BOXMULLER1) && !b)
     return MOLE_ERR_INVALID_ARGUMENT;

@@ -146,6 +146,30 @@ __device__ __forceinline__ double sqrt_normal(double x) {
   return fma(fma(-g, g, x), h, g);
 }
 
+// 1/x for 2^-500 < |x| < 2^500: the division's own steps (v_rcp_f64, two
+// Newton iterations, the residual correction) without its operand scaling and
+// fix-up, so the same rounding.  0 and infinity give NaN.
+__device__ __forceinline__ double recip_normal(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(y, fma(-x, y, 1.0), y);
+  y = fma(y, fma(-x, y, 1.0), y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+
+// Tracks whether square root arguments stay in [2^-767, 2^400), where
+// sqrt_normal of them and recip_normal of the roots hold: the largest distance
+// of a high word above the lower bound's (wrapping below it; NaN lies above).
+struct RootRange {
+  static constexpr uint32_t kLow = (1023u - 767u) << 20, kSpan = (767u + 400u) << 20;
+  uint32_t top = 0;
+  __device__ __forceinline__ double root(double ss) {
+    const uint32_t h = (uint32_t)__double2hiint(ss) - kLow;
+    top = h > top ? h : top;
+    return sqrt_normal(ss);
+  }
+  __device__ __forceinline__ bool held() const { return top < kSpan; }
+};
+
 // x^2 + y^2 + z^2 as norm3 sums it
 __device__ __forceinline__ double sumsq3(double x, double y, double z) {
   double s = x * x;

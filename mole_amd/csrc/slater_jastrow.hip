@@ -32,6 +32,8 @@
 #include "sj_internal.hpp"
 #include "sr_math.hpp"
 
+#include <type_traits>
+
 namespace mole {
 
 // LDS layout (bytes); identical on host and device.  Per walker:
@@ -596,7 +598,23 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
   const bool kinds = (EXT && S.any_gto) || S.any_p;
   const int nmax = S.n_up > S.n_dn ? S.n_up : S.n_dn;
   sync_wave();
-  for (int i = t; i < N; i += L) {
+  // FAST leaves out the square root's and the divisions' range handling (a
+  // third of a pair's instructions); its results are the same bits while every
+  // root's argument is in range, and an electron for which one is not, or a
+  // result is NaN, is evaluated again without it.
+  const bool tame = fabs(c) < 0x1p100 && fabs(d) < 0x1p100;
+  auto electron = [&](int i, auto fast) {
+    constexpr bool FAST = decltype(fast)::value;
+    RootRange range;
+    auto root = [&](double v0, double v1, double v2) {
+      const double ss = sumsq3(v0, v1, v2);
+      if constexpr (FAST) return range.root(ss);
+      else return sqrt(ss);
+    };
+    auto recip = [](double v) {
+      if constexpr (FAST) return recip_normal(v);
+      else return 1.0 / v;
+    };
     const int s = i < S.n_up ? 0 : 1;
     const int cc = s == 0 ? i : i - S.n_up;
     const int n = s == 0 ? S.n_up : S.n_dn;
@@ -629,8 +647,8 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
           d0 = xi[0] - S.nuc[3 * I];
           d1 = xi[1] - S.nuc[3 * I + 1];
           d2 = xi[2] - S.nuc[3 * I + 2];
-          r = norm3(d0, d1, d2);
-          ir = 1.0 / r;
+          r = root(d0, d1, d2);
+          ir = recip(r);
           Ip = I;
           have_e = false;
         }
@@ -678,12 +696,12 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
       if (j == i) continue;
       const double *xj = wk.pos + 3 * j;
       const double dv0 = xi[0] - xj[0], dv1 = xi[1] - xj[1], dv2 = xi[2] - xj[2];
-      const double r = norm3(dv0, dv1, dv2);
+      const double r = root(dv0, dv1, dv2);
       const bool same = (j < S.n_up ? 0 : 1) == s;
       const double b = same ? bP : bA;
       // two divisions per pair: 1/r and 1/(1 + c r)
-      const double ir = 1.0 / r;
-      const double iden = 1.0 / (1.0 + c * r);
+      const double ir = recip(r);
+      const double iden = recip(1.0 + c * r);
       const double iden2 = iden * iden;
       const double up = b * iden2;
       const double upp = (-2.0 * b * c) * (iden2 * iden);
@@ -705,10 +723,10 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
 #pragma unroll 1
     for (int I = 0; I < nn; ++I) {
       const double d0 = xi[0] - S.nuc[3 * I], d1 = xi[1] - S.nuc[3 * I + 1], d2 = xi[2] - S.nuc[3 * I + 2];
-      const double r = norm3(d0, d1, d2);
+      const double r = root(d0, d1, d2);
       const double Z = S.charge[I];
-      const double ir = 1.0 / r;
-      const double iden = 1.0 / (1.0 + d * r);
+      const double ir = recip(r);
+      const double iden = recip(1.0 + d * r);
       const double iden2 = iden * iden;
       const double aZ = a * Z;
       const double vp = -aZ * iden2;
@@ -739,6 +757,13 @@ __device__ __forceinline__ double local_energy(const SJSysDev &S, SJWalker<T> &w
     o[6] = e4;
     if constexpr (EXT) o[7] = Vee;
     if (S.opt_exp) o[8] = ez;
+    if constexpr (FAST) return range.held() && !(o[0] != o[0]) && !(o[1] != o[1]);
+    else return true;
+  };
+#pragma unroll 1
+  for (int i = t; i < N; i += L) {
+    const bool ok = tame && electron(i, std::true_type{});
+    if (__builtin_expect(__any(!ok), 0)) electron(i, std::false_type{});
   }
   sync_wave();
   // sums over electrons, in electron order: lane q forms component q into

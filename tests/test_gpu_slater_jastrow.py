@@ -696,3 +696,28 @@ def test_spin_blocks_at_the_chunk_edges(N):
     assert np.array_equal(d["masks"], o["accept_mask"])
     assert np.array_equal(bits(d["cfg"]), bits(o["cfg"]))
     assert np.max(np.abs(d["el"] - o["e_local"]) / np.maximum(1.0, np.abs(o["e_local"]))) <= E_TOL
+
+
+@pytest.mark.parametrize("side", [1e-60, 1e-130, 1e-200])
+def test_local_energy_outside_the_fast_roots(side):
+    # an electron that stays within 1e-60 (inside the fast roots' range), 1e-130
+    # (a square below it) or 1e-200 (a square that underflows: r = 0, E_L
+    # infinite or NaN) of its nucleus: the electron is evaluated in full
+    system = S.atom(4)
+    W, steps, B = 20, 4, 2
+    cfg = np.random.default_rng(2).normal(size=(W, 12))
+    cfg[:, :3] = 0.0
+    with M.Context([M.slater_jastrow(system, W)], seed=3, step=side, block_size=B, flags=M.FLAG_TRACE,
+                   record_sweeps=steps, lu_period=64) as ctx:
+        ctx.set_configs(cfg)
+        ctx.set_stream(0, 12)
+        ctx.run(steps)
+        masks, el = ctx.trace(steps, steps - B)
+        got = ctx.get_configs()
+    o = SJ.run(SJ.SjWave(system), seed=3, walkers=W, steps=steps, block_size=B, box_side=side, lu_period=64, cfg=cfg,
+               pos0=12)
+    assert np.array_equal(masks, o["accept_mask"]) and np.array_equal(bits(got), bits(o["cfg"]))
+    want = o["e_local"].reshape(el.shape)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(el), fin) and np.array_equal(np.isnan(el), np.isnan(want))
+    assert np.all(np.abs(el[fin] - want[fin]) <= E_TOL * np.maximum(1.0, np.abs(want[fin])))

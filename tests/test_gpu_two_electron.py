@@ -63,6 +63,15 @@ def test_chain_root_is_correctly_rounded_in_its_range():
     assert np.all(np.isnan(M.debug_math(M.DEBUG_SQRT_NORMAL, np.array([0.0, np.inf, np.nan]))))
 
 
+def test_chain_reciprocal_is_the_division_in_its_range():
+    rng = np.random.default_rng(5)
+    m = rng.uniform(1, 2, 400000) * rng.choice([-1.0, 1.0], 400000)
+    a = np.concatenate([m * 2.0 ** rng.integers(-499, 499, m.size), rng.uniform(1, 60, 400000),
+                        np.nextafter(2.0 ** np.arange(-490.0, 490.0), 0.0), 2.0 ** np.arange(-490.0, 490.0)])
+    assert np.array_equal(bits(M.debug_math(M.DEBUG_RECIP_NORMAL, a)), bits(1.0 / a))
+    assert np.all(np.isnan(M.debug_math(M.DEBUG_RECIP_NORMAL, np.array([0.0, np.inf, np.nan]))))
+
+
 def test_device_u64_maps_match_oracle():
     L = O.lib()
     rng = np.random.default_rng(2)
