@@ -142,7 +142,7 @@ struct mole_ctx {
   SJTile *d_tiles = nullptr;
   int n_tiles = 0;
   size_t lds_bytes = 0, lds_limit = 65536;
-  // tiles of one LDS footprint class (4 KiB steps) are launched together with
+  // tiles of one LDS footprint class (sj_build_tiles) are launched together with
   // that class's dynamic LDS, so small walkers are not held to the largest
   // footprint's occupancy
   struct TileGroup {
@@ -507,8 +507,9 @@ int sj_default_lanes(const mole_ctx *ctx, const SysState &s) {
   return L;
 }
 
-// Tiles of 64/L walkers grouped by LDS footprint class (4 KiB steps, the
-// largest class first), most expensive first within a group
+// Tiles of 64/L walkers grouped by LDS footprint class (4 KiB steps above an
+// eighth of a CU's LDS, one class below it; the largest class first), most
+// expensive first within a group
 // (longest-processing-time order, so the tail of each launch is short
 // tiles); each group's dynamic LDS is its largest tile footprint.
 mole_status sj_build_tiles(mole_ctx *ctx) {
@@ -531,7 +532,14 @@ mole_status sj_build_tiles(mole_ctx *ctx) {
   if (lds > ctx->lds_limit)
     return fail(MOLE_ERR_UNSUPPORTED, "walker state needs %zu B of LDS per workgroup (limit %zu): use "
                 "more lanes per walker", lds, ctx->lds_limit);
-  auto cls = [](size_t fp) { return (fp + 4095) / 4096; };
+  // Footprints that leave eight workgroups on a CU -- the two waves per SIMD the
+  // kernels' registers allow -- are one class: more LDS than a tile needs costs
+  // it nothing there, a launch of its own a drain of the chip (ms per 10 sampled
+  // sweeps with 4 KiB steps throughout and so: 24 molecules, 8,000 walkers 13.8
+  // and 7.1, 49,152 walkers 30.8 and 28.3; 256 molecules, 262,144 walkers 206.5
+  // and 205.2).
+  const size_t free_fp = ctx->lds_limit / 8;
+  auto cls = [free_fp](size_t fp) { return fp <= free_fp ? (free_fp + 4095) / 4096 : (fp + 4095) / 4096; };
   std::stable_sort(tiles.begin(), tiles.end(), [&](const T &a, const T &b) {
     return cls(a.fp) != cls(b.fp) ? cls(a.fp) > cls(b.fp) : a.cost > b.cost;
   });

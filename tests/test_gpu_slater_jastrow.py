@@ -180,6 +180,41 @@ def test_heterogeneous_systems_in_one_launch():
         assert np.max(rel) <= E_TOL, k
 
 
+@pytest.mark.parametrize("wide", [0, 2])
+def test_small_footprints_share_a_launch(wide):
+    # tiles up to an eighth of a CU's LDS (20 KiB) are one class whatever their
+    # footprints, larger ones classes of their own: every system at the fewest
+    # lanes below the line, then the last two at the most lanes above it
+    systems = [S.helium_product(1.7, 0.5), S.hydrogen_chain(6), S.atom(10), S.random_molecule(14, seed=3),
+               S.hydrogen_chain(24)]
+    lanes = []
+    for k, s in enumerate(systems):
+        above = k >= len(systems) - wide
+        L = 64
+        while L > 2 and tile_footprint(s, L) > 20480:
+            L //= 2
+        while L > 2 and tile_footprint(s, L // 2) <= 20480:
+            L //= 2
+        lanes.append(L // 2 if above and L > 2 else L)
+    print(f"small footprints: lanes {lanes}", flush=True)
+    W, steps, B = 33, 6, 2
+    dev = [M.slater_jastrow(s, W) for s in systems]
+    with M.Context(dev, seed=5, step=0.6, block_size=B, flags=M.FLAG_TRACE, record_sweeps=steps,
+                   precision=M.PREC_MIXED, lu_period=64) as ctx:
+        for k, L in enumerate(lanes):
+            ctx.set_walker_lanes(L, sys=k)
+        ctx.init_walkers()
+        ctx.run(steps)
+        got = [(ctx.trace(steps, steps - B, sys=k), ctx.get_configs(sys=k)) for k in range(len(systems))]
+    for k, system in enumerate(systems):
+        (masks, el), cfg = got[k]
+        o = run_oracle(system, W, steps, B, sys=k, precision=SJ.PREC_MIXED, lu=64, seed=5)
+        assert np.array_equal(masks, o["accept_mask"]), k
+        assert np.array_equal(bits(cfg), bits(o["cfg"])), k
+        rel = np.abs(el - o["e_local"]) / np.maximum(1.0, np.abs(o["e_local"]))
+        assert np.max(rel) <= E_TOL, k
+
+
 def test_zero_variance_anchors():
     d = run_device([S.hydrogenic(1)], 128, 20, 5)[0]
     assert np.max(np.abs(d["el"] + 0.5)) <= 1e-12
