@@ -649,8 +649,16 @@ hipError_t sj_launch_groups(const mole_ctx *ctx, SJArgs a) {
     a.ticket = ctx->d_ticket;
     return launch_sj_persistent(a, ctx->persist_wg, fp32, ctx->lds_bytes, ctx->stream);
   }
+  // The learned proposal's kernel for one wave per SIMD is faster only where a
+  // second wave has no place: its tiles fill the SIMDs at most once, or their LDS
+  // leaves four workgroups a CU.  us per sampled sweep, two waves' kernel and one
+  // wave's: 14 electrons, 16,384 walkers, FP64 308 and 301; 28 electrons, 4,096
+  // 1,010 and 997; but Ne, 65,536 walkers, mixed 338 and 535, FP64 455 and 539, O
+  // 237 and 366.  (The extended kernel keeps one wave from 8 electrons on.)
+  const int one_wave = a.one_wave;
   for (const mole_ctx::TileGroup &g : ctx->tile_groups) {
     a.tiles = ctx->d_tiles + g.first;
+    a.one_wave = one_wave && (a.ext || g.count <= 4 * ctx->cu_count || g.lds > ctx->lds_limit / 5);
     const hipError_t e = launch_sj(a, g.count, fp32, sj_prop(ctx), g.lds, ctx->stream);
     if (e != hipSuccess) return e;
   }
@@ -677,10 +685,8 @@ SJArgs sj_args(const mole_ctx *ctx) {
   for (const SysState &s : ctx->sys) {
     // compat samples are written by the extended instantiation only
     if (s.any_gto || s.custom_h || s.n_obs || (ctx->run.flags & MOLE_FLAG_SAMPLES)) a.ext = 1;
-    // learned proposal: from 8 electrons on, the register budget of one
-    // wave per SIMD (no spills) beats two waves (FP64 atoms, 65,536 walkers:
-    // Li, Be 1.4x and B..N 1.1x faster with two; O 1.08x, F and Ne 1.19x
-    // faster with one)
+    // learned proposal: from 8 electrons on, the kernel with the registers of
+    // one wave per SIMD (no spills) where a launch can use it (sj_launch_groups)
     if (s.N >= 8) a.one_wave = 1;
   }
   return a;

@@ -898,8 +898,8 @@ __device__ __forceinline__ void drift_sum(const double *og, const T *B, int n, i
 // compiled in (the plain VMC instantiations leave them out, keeping their
 // register budget).
 // MINW: minimum waves per SIMD the register budget is fitted to (2: up to
-// 256 registers; 1: 512, for the learned proposal's larger systems, where
-// spills cost more than the lost occupancy).
+// 256 registers; 1: 512, for the learned proposal's larger systems where a
+// launch holds no second wave per SIMD anyway).
 // One tile's launch: its walkers' state into the workgroup's LDS, the sweeps,
 // the state out.
 template <typename T, int PROP, bool EXT>

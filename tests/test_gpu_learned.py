@@ -306,3 +306,19 @@ def test_update_packs_what_a_reload_of_the_weights_packs(batch):
         out2 = net.eval(cfg, sj.nuclei, electron)
         g2, o2 = net.gradient(ctx, 64, seed=9)
     assert np.array_equal(out, out2) and np.array_equal(g, g2) and o == o2
+
+
+@pytest.mark.parametrize("precision", [M.PREC_MIXED, M.PREC_FP64])
+def test_wide_launches_keep_the_narrow_launch_walkers(precision):
+    # from eight electrons on, launches that fill the SIMDs at most once run the
+    # kernel fitted to one wave per SIMD, wider ones the two-wave kernel: a
+    # walker's trajectory is the same in both
+    got = []
+    for W in (64, 64 * 4 * 304 + 5):
+        with M.Context([M.slater_jastrow(S.atom(8), W)], seed=6, step=0.3, block_size=2, precision=precision,
+                       lu_period=16, proposal=M.PROPOSAL_LEARNED) as ctx, M.Mlp(2) as net:
+            net.attach(ctx)
+            ctx.init_walkers()
+            ctx.run(6)
+            got.append(ctx.get_configs()[:64].copy())
+    assert np.array_equal(got[0].view(np.uint64), got[1].view(np.uint64))
