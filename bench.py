@@ -59,7 +59,7 @@ VARIANTS = {"auto": 0, "lane": 1, "ws": 2, "quad": 3}
 # that measurement.  The launches start the accumulators from zero, so the
 # algorithmic state traffic is positions in and out plus accumulators out:
 # 3.93e6 B.
-TRAFFIC_BYTES_PER_LAUNCH = (680.3 * 2.0 + 3328.0) * 1024
+TRAFFIC_BYTES_PER_LAUNCH = (503.2 * 2.0 + 3072.0) * 1024
 TRAFFIC_SOURCE = "profiles/sweep2_ws_kernel_h2_sr_16384w.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE)"
 METRIC = "walker-moves/s incl. E_L; effective samples/s learned vs plain proposal at matched sigma(E)"
 
