@@ -58,7 +58,7 @@ def tune(systems, walkers_of, *, candidates=CANDIDATES, sweeps=6, precision=M.PR
          lu_period=64, lds_budget=None, verbose=False):
     """Best L per electron count.  walkers_of(system) gives the walker count
     to time with; lds_budget caps the LDS of a workgroup (the tiles of one
-    4 KiB footprint class share a launch and its largest footprint, so the
+    footprint class share a launch and its largest footprint, so the
     cap bounds the occupancy the largest systems run at)."""
     table = {}
     timings = {}
