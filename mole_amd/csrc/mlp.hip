@@ -4,6 +4,7 @@
 // the Slater-Jastrow wavefunction), the fixed-order gradient reduction and
 // Adam.
 #include "basis.hpp"
+#include "lane_lu.hpp"
 #include "mlp_internal.hpp"
 
 namespace mole {
@@ -297,43 +298,7 @@ __device__ __forceinline__ void move_terms(const SJSysDev &S, const double *cfg,
   double *A = scr, *y = scr + n * n;
   // (the samples of a wave may differ in their spin block: the barriers count
   // to the larger one)
-#pragma unroll 1
-  for (int p = 0; p < nmax; ++p) {
-    if (p < n) {
-      int piv = p;
-      double best = fabs(A[p * n + p]);
-      for (int r = p + 1; r < n; ++r) {
-        const double v = fabs(A[r * n + p]);
-        if (v > best) {
-          best = v;
-          piv = r;
-        }
-      }
-      if (piv != p)
-        for (int k = p + sub; k <= n; k += 4) {  // column n: y
-          double *u = k < n ? A + p * n + k : y + p, *v = k < n ? A + piv * n + k : y + piv;
-          const double t = *u;
-          *u = *v;
-          *v = t;
-        }
-    }
-    __syncthreads();
-    if (p < n) {
-      const double app = A[p * n + p], yp = y[p];
-      for (int r = p + 1 + sub; r < n; r += 4) {
-        const double f = A[r * n + p] / app;
-        int k = p + 1;
-        for (; k + 2 <= n; k += 2) {
-          const double a0 = A[p * n + k], a1 = A[p * n + k + 1], b0 = A[r * n + k], b1 = A[r * n + k + 1];
-          A[r * n + k] = fma(-f, a0, b0);
-          A[r * n + k + 1] = fma(-f, a1, b1);
-        }
-        if (k < n) A[r * n + k] = fma(-f, A[p * n + k], A[r * n + k]);
-        y[r] = fma(-f, yp, y[r]);
-      }
-    }
-    __syncthreads();
-  }
+  eliminate_by_lanes(A, y, n, nmax, sub, [] { __syncthreads(); });
   double ys[kMlpMaxSpin];  // y in registers, n <= kMlpMaxSpin
 #pragma unroll
   for (int p = kMlpMaxSpin - 1; p >= 0; --p) {
