@@ -756,3 +756,29 @@ def test_local_energy_outside_the_fast_roots(side):
     fin = np.isfinite(want)
     assert np.array_equal(np.isfinite(el), fin) and np.array_equal(np.isnan(el), np.isnan(want))
     assert np.all(np.abs(el[fin] - want[fin]) <= E_TOL * np.maximum(1.0, np.abs(want[fin])))
+
+
+@pytest.mark.parametrize("precision", [M.PREC_MIXED, M.PREC_FP64])
+def test_absent_walkers_cost_a_wave_nothing(precision):
+    # one workgroup with one of its 4 walkers present against the same with all
+    # of them: fewer walkers never make a wave's sampled sweeps longer.  With a
+    # basis of 64 functions on 16 lanes the local energy (a lane per electron) is
+    # most of a sweep, and evaluating it a second time for the empty slots makes
+    # it a fifth longer.
+    system = S.hydrogen_chain(2, basis_per_nucleus=32, seed=2)
+    ctxs = []
+    for W in (1, 4):
+        c = M.Context([M.slater_jastrow(system, W)], seed=1, step=0.6, block_size=10, precision=precision, lu_period=64)
+        c.set_walker_lanes(16)
+        c.init_walkers()
+        ctxs.append(c)
+    best = [np.inf, np.inf]
+    for _ in range(12):
+        for k, c in enumerate(ctxs):
+            c.sweep(20, sample=True)
+            c.synchronize()
+            best[k] = min(best[k], c.last_timing()[0])
+    for c in ctxs:
+        c.close()
+    print(f"absent walkers: {best}", flush=True)
+    assert best[0] <= 1.08 * best[1], best
