@@ -504,6 +504,21 @@ int sj_default_lanes(const mole_ctx *ctx, const SysState &s) {
   // the lanes that keep any accepted basis within the LDS
   const int wide = N <= 4 ? 4 : N <= 10 ? 8 : N <= 20 ? 16 : 32;
   while (L < wide && sj_footprint(ctx, s, L, 8) > ctx->lds_limit / 4) L *= 2;
+  // The drift-diffusion proposal and FP64 inverses hold more LDS than the table
+  // above had: where fewer than eight workgroups fit a CU, twice the lanes (half
+  // the walkers and the LDS) are taken if the tiles then need no more rounds of
+  // resident workgroups, each of which is shorter.  us per sampled sweep at half
+  // the lanes and at those taken: 8 electrons, 65,536 walkers, drift-diffusion
+  // 743 and 539; 16 electrons, 16,384 walkers, FP64 377 and 291, drift-diffusion
+  // 972 and 778; 36 electrons, 4,096 walkers, mixed 1,156 and 975.  Where it does
+  // take more rounds: 6 electrons, 65,536 walkers, drift-diffusion 349 at 4 (3
+  // rounds), 378 at 8 (4).
+  auto rounds = [&](int lanes) {
+    const size_t resident = std::min<size_t>(8, ctx->lds_limit / sj_footprint(ctx, s, lanes, sj_tsize(ctx)));
+    const int64_t tiles = (walkers * lanes + 63) / 64, at_once = (int64_t)ctx->cu_count * (int64_t)resident;
+    return resident ? (tiles + at_once - 1) / at_once : 0;  // 0: refused with the tiles, as it is
+  };
+  while (2 * L <= most && rounds(2 * L) <= rounds(L)) L *= 2;
   return L;
 }
 

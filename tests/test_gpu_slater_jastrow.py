@@ -694,6 +694,31 @@ def test_default_lanes_leave_the_results_unchanged(Z_or_n, W):
     assert np.array_equal(bits(l0[0]), bits(l1[0])) and np.array_equal(l0[1], l1[1])
 
 
+@pytest.mark.parametrize("N,W,precision,proposal", [
+    (5, 65536, M.PREC_FP64, M.PROPOSAL_BOX), (6, 65536, M.PREC_MIXED, M.PROPOSAL_DIFFUSE),
+    (8, 65536, M.PREC_FP64, M.PROPOSAL_DIFFUSE), (10, 65536, M.PREC_MIXED, M.PROPOSAL_BOX),
+    (16, 16384, M.PREC_FP64, M.PROPOSAL_BOX), (16, 65536, M.PREC_FP64, M.PROPOSAL_DIFFUSE),
+    (36, 4096, M.PREC_MIXED, M.PROPOSAL_BOX), (3, 1, M.PREC_FP64, M.PROPOSAL_BOX)])
+def test_default_lanes_take_the_shorter_rounds(N, W, precision, proposal):
+    # a CU holds eight workgroups, or as many as its LDS (160 KiB) has room for;
+    # a launch is a number of rounds of that many on every CU, shorter the more
+    # lanes a walker has: the default is never half the lanes that need no more
+    # rounds (up to the width of a move)
+    cus = M.device_info()[1]
+
+    def rounds(c):
+        workgroups, lds = c.launch_info()
+        return -(-workgroups // (cus * min(8, 163840 // lds)))
+
+    with M.Context([M.slater_jastrow(S.hydrogen_chain(N, seed=3), W)], seed=1, step=0.1, block_size=2,
+                   precision=precision, lu_period=16, proposal=proposal) as c:
+        L = c.walker_lanes()
+        default = rounds(c)
+        if L < max(N, 4):
+            c.set_walker_lanes(2 * L)
+            assert rounds(c) > default, (L, default)
+
+
 @pytest.mark.parametrize("N,W", [(1, 5461), (1, 5462), (2, 21846), (3, 14563), (11, 3973), (40, 200), (40, 2185)])
 def test_configurations_round_trip_through_staged_transfers(N, W):
     # both sides of the staging rule (128 KiB), chunks of 1 MiB with a partial
