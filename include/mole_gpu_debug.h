@@ -56,6 +56,10 @@ mole_status mole_debug_mfma_bf16_k32(const float *A, const float *B, float *D);
 mole_status mole_debug_mlp_features(const double *cfg, uint32_t N, const double *nuc_xyz, uint32_t n_nuc,
                                     const int32_t *electron, size_t n, float *out);
 
+/* Lanes per configuration that mole_eval takes for n configurations of a
+ * Slater-Jastrow system. */
+mole_status mole_debug_eval_lanes(mole_ctx *ctx, uint32_t sys, size_t n, uint32_t *lanes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -290,6 +290,7 @@ _SIGS = [
     ("mole_debug_mfma_bf16_k32", C.c_int32, [_pf, _pf, _pf]),
     ("mole_debug_mlp_features", C.c_int32, [_pd, C.c_uint32, _pd, C.c_uint32, C.POINTER(C.c_int32), C.c_size_t,
                                             _pf]),
+    ("mole_debug_eval_lanes", C.c_int32, [_P, C.c_uint32, C.c_size_t, C.POINTER(C.c_uint32)]),
     ("mole_optimize", C.c_int32, [_P, C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, C.c_double, C.c_uint32,
                                   C.c_double, _pd, _pd]),
     ("mole_mlp_create", C.c_int32, [C.c_uint64, C.POINTER(_P)]),

@@ -76,6 +76,7 @@ struct SysState {
   // Slater-Jastrow
   std::vector<double> params;
   int n_nuc = 0, n_basis = 0, n_orb = 0, L = 0;
+  bool lanes_set = false;  // L is the caller's
   size_t lds_walker = 0;
   double *d_tab = nullptr;  // nuclei xyz, charges, zeta, coefficients
   int *d_center = nullptr;
@@ -464,13 +465,14 @@ int sj_prop(const mole_ctx *ctx) {
 }
 
 // LDS bytes of a workgroup of system s at L lanes per walker.
-size_t sj_footprint(const mole_ctx *ctx, const SysState &s, int L, int tsize) {
+size_t sj_footprint(const SysState &s, int L, int tsize, int prop) {
   return sj_lds_per_group(s.n_nuc, s.n_basis, s.n_orb) +
          (size_t)(64 / L) * sj_lds_per_walker((int)s.N, (int)s.n_up, (int)s.n_down, s.n_nuc, s.n_basis, tsize,
-                                              (int)s.params.size(), sj_prop(ctx));
+                                              (int)s.params.size(), prop);
 }
 
-// Lanes per walker where the caller sets none.  A wave's instructions cost the
+// Lanes per walker where the caller sets none, for a launch of `walkers` of them
+// in all (tsize: bytes of an inverse's element).  A wave's instructions cost the
 // same however many lanes they use, so a full chip wants few lanes per walker
 // (`least`: below it the walkers' LDS leaves too few waves), and a chip with
 // SIMDs to spare more, up to two waves per SIMD or the width of a move
@@ -487,23 +489,21 @@ size_t sj_footprint(const mole_ctx *ctx, const SysState &s, int L, int tsize) {
 //   36  16,384        7002  4199 3011  2000  2772
 //   36  512           1757  1013 650   429   311
 // The learned proposal's network passes take 4.
-int sj_default_lanes(const mole_ctx *ctx, const SysState &s) {
+int sj_lanes_rule(const mole_ctx *ctx, const SysState &s, int64_t walkers, int tsize, int prop) {
   if (ctx->run.proposal == MOLE_PROPOSAL_LEARNED) return 4;
   const int N = (int)s.N;
-  int64_t walkers = 0;
-  for (const SysState &o : ctx->sys) walkers += o.W;
   // (FP64 inverses of 10 electrons at 4 lanes fit seven workgroups a CU: 253
   // against 239 us at 8)
-  const int least = N <= 5 ? 2 : N <= (sj_tsize(ctx) == 8 ? 9 : 10) ? 4 : N <= 16 ? 8 : N <= 24 ? 16 : 32;
+  const int least = N <= 5 ? 2 : N <= (tsize == 8 ? 9 : 10) ? 4 : N <= 16 ? 8 : N <= 24 ? 16 : 32;
   int most = 4;
   while (most < N) most *= 2;
   int L = 1;
   while (2 * L <= most && walkers * (2 * L) <= (int64_t)64 * 8 * ctx->cu_count) L *= 2;
   L = std::max(L, least);
-  // large bases: within a quarter of a CU's LDS, in FP64 too (mole_eval), up to
-  // the lanes that keep any accepted basis within the LDS
+  // large bases: within a quarter of a CU's LDS (as FP64), up to the lanes that
+  // keep any accepted basis within the LDS
   const int wide = N <= 4 ? 4 : N <= 10 ? 8 : N <= 20 ? 16 : 32;
-  while (L < wide && sj_footprint(ctx, s, L, 8) > ctx->lds_limit / 4) L *= 2;
+  while (L < wide && sj_footprint(s, L, 8, prop) > ctx->lds_limit / 4) L *= 2;
   // The drift-diffusion proposal and FP64 inverses hold more LDS than the table
   // above had: where fewer than eight workgroups fit a CU, twice the lanes (half
   // the walkers and the LDS) are taken if the tiles then need no more rounds of
@@ -514,12 +514,24 @@ int sj_default_lanes(const mole_ctx *ctx, const SysState &s) {
   // take more rounds: 6 electrons, 65,536 walkers, drift-diffusion 349 at 4 (3
   // rounds), 378 at 8 (4).
   auto rounds = [&](int lanes) {
-    const size_t resident = std::min<size_t>(8, ctx->lds_limit / sj_footprint(ctx, s, lanes, sj_tsize(ctx)));
+    const size_t resident = std::min<size_t>(8, ctx->lds_limit / sj_footprint(s, lanes, tsize, prop));
     const int64_t tiles = (walkers * lanes + 63) / 64, at_once = (int64_t)ctx->cu_count * (int64_t)resident;
     return resident ? (tiles + at_once - 1) / at_once : 0;  // 0: refused with the tiles, as it is
   };
   while (2 * L <= most && rounds(2 * L) <= rounds(L)) L *= 2;
   return L;
+}
+
+int sj_default_lanes(const mole_ctx *ctx, const SysState &s) {
+  int64_t walkers = 0;
+  for (const SysState &o : ctx->sys) walkers += o.W;
+  return sj_lanes_rule(ctx, s, walkers, sj_tsize(ctx), sj_prop(ctx));
+}
+
+// Lanes of mole_eval for n configurations: those the caller set, or the rule's
+// for a launch of n, whatever the context's own walkers.
+int sj_eval_lanes(const mole_ctx *ctx, const SysState &s, size_t n) {
+  return s.lanes_set ? s.L : sj_lanes_rule(ctx, s, (int64_t)n, 8, kSJPropBox);
 }
 
 // Tiles of 64/L walkers grouped by LDS footprint class (4 KiB steps above an
@@ -536,7 +548,7 @@ mole_status sj_build_tiles(mole_ctx *ctx) {
     st.lds_walker = sj_lds_per_walker((int)st.N, (int)st.n_up, (int)st.n_down, st.n_nuc, st.n_basis,
                                       sj_tsize(ctx), (int)st.params.size(), sj_prop(ctx));
     const int wpt = 64 / st.L;
-    const size_t fp = sj_footprint(ctx, st, st.L, sj_tsize(ctx));
+    const size_t fp = sj_footprint(st, st.L, sj_tsize(ctx), sj_prop(ctx));
     lds = std::max(lds, fp);
     const int nmax = (int)std::max(st.n_up, st.n_down);
     const double per_walker = (double)st.N * (st.N + st.n_nuc + st.n_basis + (double)nmax * st.n_basis +
@@ -1463,16 +1475,14 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
   const size_t D = 3 * (size_t)s.N, np = s.params.size();
   const size_t nB = (size_t)s.n_up * s.n_up + (size_t)s.n_down * s.n_down;
   const size_t ncol = kSJSumO;  // no samples: only the counters' columns are touched
-  const int wpt = 64 / s.L;
   if (n > ((size_t)1 << 28)) return fail(MOLE_ERR_SHAPE, "mole_eval: at most 2^28 configurations per call");
   // evaluated in FP64 whatever the context's precision (Function::value and
   // its derivatives at given configurations, no update chain to save)
-  const size_t lds_walker =
-      sj_lds_per_walker((int)s.N, (int)s.n_up, (int)s.n_down, s.n_nuc, s.n_basis, 8, (int)np, kSJPropBox);
-  const size_t lds = sj_lds_per_group(s.n_nuc, s.n_basis, s.n_orb) + (size_t)wpt * lds_walker;
+  const int L = sj_eval_lanes(ctx, s, n), wpt = 64 / L;
+  const size_t lds = sj_footprint(s, L, 8, kSJPropBox);
   if (lds > ctx->lds_limit)
     return fail(MOLE_ERR_UNSUPPORTED, "mole_eval: %zu B of LDS per workgroup at %d lanes per walker (limit %zu)",
-                lds, s.L, ctx->lds_limit);
+                lds, L, ctx->lds_limit);
   const size_t n_tiles = (n + wpt - 1) / wpt;
   // one allocation of doubles: positions, inverses (8 bytes per element for
   // either precision), accumulators, determinants, then the outputs
@@ -1489,7 +1499,7 @@ static mole_status sj_eval(mole_ctx *ctx, uint32_t sys, size_t n, const double *
   if (e == hipSuccess) {
     SJSysDev v = sj_sysdev_of(ctx, sys);
     v.W = (int)n;
-    v.lds_per_walker = (uint32_t)lds_walker;
+    v.L = L;
     v.pos = d + o_pos;
     v.B = d + o_B;
     v.acc = d + o_acc;
@@ -1672,12 +1682,15 @@ mole_status mole_set_walker_lanes(mole_ctx *ctx, uint32_t sys, uint32_t lanes) {
     return fail(MOLE_ERR_UNSUPPORTED, "the learned proposal runs 16 walkers of 4 lanes per wave");
   SysState &s = ctx->sys[sys];
   const int old = s.L;
+  const bool was_set = s.lanes_set;
   s.L = lanes ? (int)lanes : sj_default_lanes(ctx, s);
+  s.lanes_set = lanes != 0;
   HIP_TRY(hipSetDevice(ctx->device));
   HIP_TRY(hipStreamSynchronize(ctx->stream));
   st = sj_build_tiles(ctx);
   if (st != MOLE_OK) {
     s.L = old;
+    s.lanes_set = was_set;
     (void)sj_build_tiles(ctx);
     return st;
   }
@@ -1691,6 +1704,15 @@ mole_status mole_get_walker_lanes(mole_ctx *ctx, uint32_t sys, uint32_t *lanes) 
   if (st != MOLE_OK) return st;
   if (!lanes) return fail(MOLE_ERR_INVALID_ARGUMENT, "null output");
   *lanes = (uint32_t)ctx->sys[sys].L;
+  return ok();
+}
+
+mole_status mole_debug_eval_lanes(mole_ctx *ctx, uint32_t sys, size_t n, uint32_t *lanes) {
+  mole_status st = check_ctx(ctx, sys);
+  if (st != MOLE_OK) return st;
+  if (ctx->family != kFamSJ) return fail(MOLE_ERR_UNSUPPORTED, "lanes per walker apply to Slater-Jastrow systems");
+  if (!lanes) return fail(MOLE_ERR_INVALID_ARGUMENT, "null output");
+  *lanes = (uint32_t)sj_eval_lanes(ctx, ctx->sys[sys], n);
   return ok();
 }
 

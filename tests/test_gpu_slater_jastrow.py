@@ -674,6 +674,44 @@ def test_eval_matches_oracle(make, precision):
         assert abs(out["lap"][j] / v - kin) <= 1e-8 * max(1.0, abs(kin)), j
 
 
+def test_eval_lanes_follow_the_configurations():
+    # mole_eval takes the lanes that a context of as many walkers as it is given
+    # configurations would (FP64, box proposal), not those of its own context's
+    # walkers, unless the caller set them; the values do not depend on them
+    import ctypes as C
+    sj = S.atom(10)
+    cfg = np.random.default_rng(3).normal(size=(9000, 30))
+
+    def eval_lanes(c, n):
+        L = C.c_uint32()
+        M.check(M.lib().mole_debug_eval_lanes(c.h, 0, n, C.byref(L)))
+        return L.value
+
+    def context(W, precision=M.PREC_FP64, proposal=M.PROPOSAL_BOX):
+        return M.Context([M.slater_jastrow(sj, W)], seed=1, step=0.1, block_size=2, precision=precision,
+                         proposal=proposal)
+
+    want = {}
+    for n in (1, 4096, 9000, 65536):
+        with context(n) as c:
+            want[n] = c.walker_lanes()
+    assert want[1] != want[65536]
+    res = []
+    for W, precision, proposal in ((64, M.PREC_FP64, M.PROPOSAL_BOX), (65536, M.PREC_MIXED, M.PROPOSAL_BOX),
+                                   (65536, M.PREC_MIXED, M.PROPOSAL_DIFFUSE)):
+        with context(W, precision, proposal) as c:
+            assert {n: eval_lanes(c, n) for n in want} == want
+            res.append(c.eval(cfg))
+            c.set_walker_lanes(32)
+            assert eval_lanes(c, 65536) == 32
+            res.append(c.eval(cfg))
+            c.set_walker_lanes(0)
+            assert eval_lanes(c, 65536) == want[65536]
+    for r in res[1:]:
+        for k in r:
+            assert np.array_equal(bits(r[k]), bits(res[0][k])), k
+
+
 @pytest.mark.parametrize("Z_or_n,W", [(2, 64), (3, 40000), (5, 9000), (10, 3000), (10, 20000), (17, 500), (36, 70)])
 def test_default_lanes_leave_the_results_unchanged(Z_or_n, W):
     # the library's choice of lanes (by electrons and walkers; every width of
