@@ -202,3 +202,22 @@ def test_dmc_graph_replays_equal_eager_steps():
     assert gs.size == es.size == 20
     assert np.array_equal(gs, es) and np.array_equal(gw, ew) and np.array_equal(ge, ee)
     assert np.array_equal(gc, ec)
+
+
+def test_small_reads_do_not_wait_per_array():
+    # dmc_read_walkers of two short arrays against get_configs, which is one copy
+    # and one wait: the second array adds a copy, not a round trip (1.1 times
+    # the one read; with an asynchronous copy and a wait each, 1.8 times)
+    import time
+    with M.Context([M.slater_jastrow(S.helium_product(1.6875, 0.5, 0.3), 64)], seed=2, step=0.01, block_size=10,
+                   proposal=M.PROPOSAL_DIFFUSE) as ctx:
+        ctx.dmc_init(-2.9, M.BRANCH_SR)
+        ctx.dmc_diffuse(0.01, 10, 5, 0)
+        best = {}
+        for _ in range(300):
+            for name, call in (("one", ctx.get_configs), ("two", ctx.dmc_read_walkers)):
+                t = time.perf_counter()
+                call()
+                best[name] = min(best.get(name, 1.0), time.perf_counter() - t)
+    print(f"small reads: {best}", flush=True)
+    assert best["two"] <= 1.45 * best["one"], best
