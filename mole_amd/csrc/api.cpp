@@ -172,8 +172,9 @@ struct mole_ctx {
   // diffusion Monte Carlo
   bool dmc_ready = false;
   uint32_t dmc_brancher = 0;
-  // pinned staging of large host transfers (two halves, made on first use)
+  // pinned staging of large host transfers (two halves, made where they pay)
   char *stage[2] = {nullptr, nullptr};
+  uint32_t mid_transfers = 0;  // transfers of kStageMin .. kStageAlways bytes so far
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
 };
 
@@ -345,14 +346,26 @@ void free_ctx(mole_ctx *ctx) {
 // on whatever its size (the runtime pins the pages) and a configuration array
 // had to be transposed between [3N][W] and [walker][3N] through a zeroed
 // buffer of its size on the host (16 MB: 3 ms to zero, 0.6 ms to transpose).
-// Transfers from kStageMin on instead go through two pinned halves, the
-// device working on one (transposing straight into or out of it) while the
-// host copies the other: 0.06 ms for 1 MB, 0.9 for 16 MB of touched pages.
-constexpr size_t kStageChunk = (size_t)1 << 20, kStageMin = (size_t)128 << 10;
+// Large transfers instead go through two pinned halves, the device working on
+// one (transposing straight into or out of it) while the host copies the other:
+// 0.06 ms for 1 MB, 0.9 for 16 MB of touched pages.  A half costs 17 us to make
+// and 45 to free.  From kStageAlways on a single read saves 20 and more; between
+// kStageMin and that a transfer saves up to 20 (at 256 KiB 7), so a context makes
+// the half there only after kStageAfter of them, and one that reads its walkers
+// once and closes does not pay for it (192 KiB: first read and close 147 us with
+// the half, 91 without).  Below kStageMin the plain copies are as fast.
+constexpr size_t kStageChunk = (size_t)1 << 20, kStageMin = (size_t)128 << 10, kStageAlways = (size_t)512 << 10;
+constexpr uint32_t kStageAfter = 8;
 
-hipError_t stage_init(mole_ctx *ctx) {
+bool staged(mole_ctx *ctx, size_t bytes) {
+  if (bytes < kStageMin || bytes >= kStageAlways) return bytes >= kStageAlways;
+  return ctx->stage[0] || ++ctx->mid_transfers > kStageAfter;
+}
+
+// (the halves that a transfer of nc chunks takes)
+hipError_t stage_init(mole_ctx *ctx, size_t nc) {
   hipError_t e = hipSuccess;
-  for (int b = 0; b < 2 && e == hipSuccess; ++b) {
+  for (int b = 0; b < (nc > 1 ? 2 : 1) && e == hipSuccess; ++b) {
     if (!ctx->stage[b]) {
       void *p = nullptr;
       e = hipHostMalloc(&p, kStageChunk, hipHostMallocDefault);
@@ -368,8 +381,8 @@ hipError_t stage_init(mole_ctx *ctx) {
 // host once it is there.  Returns with the stream idle.
 template <class Fill, class Drain>
 hipError_t stage_read(mole_ctx *ctx, size_t total, size_t per, Fill fill, Drain drain) {
-  hipError_t e = stage_init(ctx);
   const size_t nc = (total + per - 1) / per;
+  hipError_t e = stage_init(ctx, nc);
   auto start = [&](size_t c) {
     const int b = (int)(c & 1);
     e = fill(ctx->stage[b], c * per, std::min(per, total - c * per));
@@ -389,8 +402,8 @@ hipError_t stage_read(mole_ctx *ctx, size_t total, size_t per, Fill fill, Drain 
 // The other way: fill on the host, then the device's part.
 template <class Fill, class Drain>
 hipError_t stage_write(mole_ctx *ctx, size_t total, size_t per, Fill fill, Drain drain) {
-  hipError_t e = stage_init(ctx);
   const size_t nc = (total + per - 1) / per;
+  hipError_t e = stage_init(ctx, nc);
   for (size_t c = 0; c < nc && e == hipSuccess; ++c) {
     const int b = (int)(c & 1);
     if (c >= 2) e = hipEventSynchronize(ctx->stage_ev[b]);
@@ -403,11 +416,7 @@ hipError_t stage_write(mole_ctx *ctx, size_t total, size_t per, Fill fill, Drain
   return e == hipSuccess ? es : e;
 }
 
-// bytes of device memory to the host, there once the stream is idle: the caller
-// waits, once for all its arrays (a wait each made mole_eval of one Li
-// configuration 182 us instead of 151).
-hipError_t read_back(mole_ctx *ctx, void *host, const void *dev, size_t bytes) {
-  if (bytes < kStageMin) return hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream);
+hipError_t read_staged(mole_ctx *ctx, void *host, const void *dev, size_t bytes) {
   return stage_read(
       ctx, bytes, kStageChunk,
       [&](char *b, size_t first, size_t n) {
@@ -416,11 +425,19 @@ hipError_t read_back(mole_ctx *ctx, void *host, const void *dev, size_t bytes) {
       [&](const char *b, size_t first, size_t n) { std::memcpy((char *)host + first, b, n); });
 }
 
+// bytes of device memory to the host, there once the stream is idle: the caller
+// waits, once for all its arrays (a wait each made mole_eval of one Li
+// configuration 182 us instead of 151).
+hipError_t read_back(mole_ctx *ctx, void *host, const void *dev, size_t bytes) {
+  return staged(ctx, bytes) ? read_staged(ctx, host, dev, bytes)
+                            : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream);
+}
+
 // cfg [W][D] from columns [D][W] on the device; returns with the stream idle.
 hipError_t read_rows(mole_ctx *ctx, double *cfg, const double *cols, size_t D, size_t W) {
-  if (sizeof(double) * D * W < kStageMin) {
+  if (!staged(ctx, sizeof(double) * D * W)) {
     std::vector<double> soa(D * W);
-    hipError_t e = read_back(ctx, soa.data(), cols, soa.size() * sizeof(double));
+    hipError_t e = hipMemcpyAsync(soa.data(), cols, soa.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
     const hipError_t es = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) e = es;
     for (size_t w = 0; w < W; ++w)
@@ -437,7 +454,7 @@ hipError_t read_rows(mole_ctx *ctx, double *cfg, const double *cols, size_t D, s
 
 // columns [D][W] on the device from cfg [W][D]; returns with the stream idle.
 hipError_t write_rows(mole_ctx *ctx, const double *cfg, double *cols, size_t D, size_t W) {
-  if (sizeof(double) * D * W < kStageMin) {
+  if (!staged(ctx, sizeof(double) * D * W)) {
     std::vector<double> soa(D * W);
     for (size_t w = 0; w < W; ++w)
       for (size_t k = 0; k < D; ++k) soa[k * W + w] = cfg[w * D + k];
@@ -2552,7 +2569,7 @@ mole_status mole_dmc_read_walkers(mole_ctx *ctx, uint32_t sys, double *weights, 
   HIP_TRY(hipStreamSynchronize(ctx->stream));
   const size_t bytes = sizeof(double) * (size_t)s.W;
   auto read = [&](double *host, const double *dev) {
-    return bytes < kStageMin ? hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost) : read_back(ctx, host, dev, bytes);
+    return staged(ctx, bytes) ? read_staged(ctx, host, dev, bytes) : hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost);
   };
   if (weights) HIP_TRY(read(weights, s.dmc.dmc));
   if (e_local) HIP_TRY(read(e_local, s.dmc.dmc + s.W));

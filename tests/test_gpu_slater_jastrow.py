@@ -757,15 +757,49 @@ def test_default_lanes_take_the_shorter_rounds(N, W, precision, proposal):
             assert rounds(c) > default, (L, default)
 
 
-@pytest.mark.parametrize("N,W", [(1, 5461), (1, 5462), (2, 21846), (3, 14563), (11, 3973), (40, 200), (40, 2185)])
+@pytest.mark.parametrize("N,W", [(1, 5461), (1, 5462), (1, 21845), (1, 21846), (2, 21846), (3, 14563), (11, 3973),
+                                 (40, 200), (40, 2185)])
 def test_configurations_round_trip_through_staged_transfers(N, W):
-    # both sides of the staging rule (128 KiB), chunks of 1 MiB with a partial
-    # last one, partial 64 x 32 tiles, more than one column tile
+    # both sides of the staging rules (128 KiB: counted; 512 KiB: always), chunks
+    # of 1 MiB with a partial last one, partial 64 x 32 tiles, more than one
+    # column tile
     sj = S.hydrogenic() if N == 1 else S.hydrogen_chain(N, seed=1)
     cfg = np.random.default_rng(N).normal(size=(W, 3 * N))
     with M.Context([M.slater_jastrow(sj, W)], seed=1, step=0.5, block_size=2) as ctx:
         ctx.set_configs(cfg)
         assert np.array_equal(bits(ctx.get_configs()), bits(cfg))
+
+
+@pytest.mark.parametrize("N,W", [(1, 5462), (3, 7281), (11, 1986)])
+def test_transfers_before_and_after_the_staging_buffer(N, W):
+    # between 128 and 512 KiB a context stages from its ninth transfer on: every
+    # round trip is exact on both sides of it
+    sj = S.hydrogenic() if N == 1 else S.hydrogen_chain(N, seed=1)
+    rng = np.random.default_rng(N)
+    with M.Context([M.slater_jastrow(sj, W)], seed=1, step=0.5, block_size=2) as ctx:
+        for k in range(7):
+            cfg = rng.normal(size=(W, 3 * N))
+            ctx.set_configs(cfg)
+            assert np.array_equal(bits(ctx.get_configs()), bits(cfg)), k
+
+
+def test_one_read_does_not_pay_for_the_staging_buffer():
+    # contexts of 127 and 129 KiB of walkers that are read once and closed, on
+    # the two sides of the staging line: making and freeing a pinned buffer for
+    # the one read would take half as long again
+    import time
+    best = {}
+    for _ in range(20):
+        for W in (2709, 2753):
+            c = M.Context([M.helium(W)], seed=1, step=0.5, block_size=10)
+            c.init_walkers()
+            c.synchronize()
+            t = time.perf_counter()
+            c.get_configs()
+            c.close()
+            best[W] = min(best.get(W, 1.0), time.perf_counter() - t)
+    print(f"one read and close: {best}", flush=True)
+    assert best[2753] <= 1.25 * best[2709], best
 
 
 @pytest.mark.parametrize("proposal", [M.PROPOSAL_BOX, M.PROPOSAL_DIFFUSE])
