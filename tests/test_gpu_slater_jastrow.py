@@ -104,34 +104,31 @@ def tile_footprint(system, lanes):
 
 def test_heterogeneous_batch_at_workload_shape():
     # the heterogeneous workload's launches: 256 systems of 2..40 electrons,
-    # 2^20 walkers split in proportion to N, the lanes its autotuning picked,
-    # mixed precision.  The tiles are grouped into LDS footprint classes (4 KiB
-    # steps), one launch per class with blockIdx.x restarting at 0 in each,
-    # longest tiles first within a class.  The system with the fewest
-    # electrons, the one with the largest tile footprint (system 52, 11
-    # electrons) and the largest system of a third footprint class against
-    # their own oracle runs (systems are independent streams)
+    # 2^20 walkers split in proportion to N, mixed precision.  The tiles are
+    # grouped into LDS footprint classes (one up to an eighth of a CU's 160 KiB,
+    # 4 KiB steps above it), one launch per class with blockIdx.x restarting at 0
+    # in each, longest tiles first within a class.  The lanes its autotuning
+    # picked keep every tile in the first class, so the systems from 21 electrons
+    # on take half of those here.  The system with the fewest electrons, the one
+    # with the largest tile footprint and the largest system of a third class
+    # against their own oracle runs (systems are independent streams)
     from mole_amd import autotune
     from mole_amd import workloads as WL
     lanes = {2: 4, 3: 4, 4: 4, 5: 8, 6: 8, 7: 8, 8: 8, 9: 16, 10: 8, 11: 8, 12: 16, 13: 16, 14: 16, 15: 16,
              16: 16, 17: 16, 18: 16, 19: 32, 20: 16}
-    lanes.update({n: 32 for n in range(21, 32)})
-    lanes.update({n: 64 for n in range(32, 41)})
+    lanes.update({n: 16 for n in range(21, 32)})
+    lanes.update({n: 32 for n in range(32, 41)})
     sys_list = WL.hetero_systems(256, 3)
     Ns = np.array([s.n_electrons for s in sys_list])
     W = np.maximum(1, np.floor(Ns / Ns.sum() * (1 << 20))).astype(int)
     W[np.argmax(Ns)] += (1 << 20) - W.sum()
-    order = np.argsort(Ns, kind="stable")
-    cls = lambda k: (tile_footprint(sys_list[k], lanes[int(Ns[k])]) + 4095) // 4096
-    picks = [int(order[0]), 52]
-    # the third: the most electrons among the systems of a third footprint
-    # class, so class boundaries stay covered
-    taken = {cls(k) for k in picks}
-    for k in order[::-1]:
-        if cls(int(k)) not in taken:
-            picks.append(int(k))
-            break
-    assert len(picks) == 3 and len(taken | {cls(picks[2])}) == 3
+    lds = np.array([tile_footprint(s, lanes[int(n)]) for s, n in zip(sys_list, Ns)])
+    cls = (np.maximum(lds, 163840 // 8) + 4095) // 4096
+    assert np.unique(cls).size >= 3
+    first, largest = int(np.argmin(Ns)), int(np.argmax(lds))
+    others = [k for k in np.argsort(Ns, kind="stable") if cls[k] not in (cls[first], cls[largest])]
+    picks = [first, largest, int(others[-1])]
+    assert np.unique(cls[picks]).size == 3
     steps, B = 4, 2
     print(f"heterogeneous batch: {len(sys_list)} systems, {int(W.sum())} walkers, checking {picks}", flush=True)
     dev = [M.slater_jastrow(s, int(w)) for s, w in zip(sys_list, W)]
