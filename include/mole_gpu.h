@@ -543,9 +543,9 @@ mole_status mole_get_walker_lanes(mole_ctx *ctx, uint32_t sys, uint32_t *lanes);
  * largest dynamic LDS bytes per workgroup among them. */
 mole_status mole_get_launch_info(mole_ctx *ctx, uint32_t *workgroups, size_t *lds_bytes);
 /* Slater-Jastrow tile schedule (no counterpart in the reference).  CLASSES:
- * one launch per LDS footprint class (4 KiB steps
- * above an eighth of a CU's LDS, one class below) with that class's dynamic
- * LDS, longest tiles first within a class.  PERSISTENT (box proposal, plain
+ * one launch per LDS footprint class (4 KiB steps above an eighth of a CU's
+ * LDS, one class below) with that class's dynamic LDS, longest tiles first
+ * within a class.  PERSISTENT (box proposal, plain
  * kernel; other launches keep CLASSES): one launch of `workgroups` resident
  * workgroups (0: CUs x the occupancy the largest footprint allows) that take
  * every tile of the context, longest first, from a device ticket -- the

@@ -77,7 +77,6 @@ struct SysState {
   std::vector<double> params;
   int n_nuc = 0, n_basis = 0, n_orb = 0, L = 0;
   bool lanes_set = false;  // L is the caller's
-  size_t lds_walker = 0;
   double *d_tab = nullptr;  // nuclei xyz, charges, zeta, coefficients
   int *d_center = nullptr;
   void *d_B = nullptr;
@@ -562,8 +561,6 @@ mole_status sj_build_tiles(mole_ctx *ctx) {
   size_t lds = 0;
   for (size_t s = 0; s < ctx->sys.size(); ++s) {
     SysState &st = ctx->sys[s];
-    st.lds_walker = sj_lds_per_walker((int)st.N, (int)st.n_up, (int)st.n_down, st.n_nuc, st.n_basis,
-                                      sj_tsize(ctx), (int)st.params.size(), sj_prop(ctx));
     const int wpt = 64 / st.L;
     const size_t fp = sj_footprint(st, st.L, sj_tsize(ctx), sj_prop(ctx));
     lds = std::max(lds, fp);
@@ -657,7 +654,6 @@ SJSysDev sj_sysdev_of(const mole_ctx *ctx, size_t s) {
   d.draw_base = st.draw_base;
   d.move_base = st.move_base;
   d.sys_index = (uint32_t)s;
-  d.lds_per_walker = (uint32_t)st.lds_walker;
   d.dmc = st.dmc.dmc;
   d.dmc_eref = st.dmc.st ? &st.dmc.st->eref : nullptr;
   d.dmc_pos_in = st.dmc.pos_s;

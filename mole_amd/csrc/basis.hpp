@@ -77,14 +77,6 @@ __device__ __forceinline__ void basis_vgl(int kind, double z, double d0, double 
   basis_vgl_sto(kind, z, d0, d1, d2, e, ir, v, g0, g1, g2, l);
 }
 
-// Gradient only (the drift): as basis_vgl's gradient.
-template <bool GTO>
-__device__ __forceinline__ void basis_grad(int kind, double z, double d0, double d1, double d2, double r, double &g0,
-                                           double &g1, double &g2) {
-  double v, l;
-  basis_vgl<GTO>(kind, z, d0, d1, d2, r, v, g0, g1, g2, l);
-}
-
 // A determinant carried as mant 2^ex: the mantissa is renormalised into
 // [1/2, 1) in magnitude by frexp after every product (exact), so products of
 // many ratios neither overflow nor underflow.  log|det| = log|mant| + ex ln 2

@@ -288,7 +288,8 @@ __device__ __forceinline__ double sum4(double v) {
 // elimination with partial pivoting of A y = e_c gives column c of A^-1.  The
 // sample's four lanes (sub = 0..3) take the rows below a pivot and the Jastrow
 // partners in turn and search pivots, substitute back and evaluate the
-// orbitals alike; all four return the results.  All lanes of the wave call it.
+// orbitals alike; all four return the results, each sum over partners being the
+// lanes' four interleaved sums added.  All lanes of the wave call it.
 __device__ __forceinline__ void move_terms(const SJSysDev &S, const double *cfg, int i, const double *xn, double *scr,
                                            int sub, double *lR2, double *gx) {
   const int N = S.N, sp = i < S.n_up ? 0 : 1;
@@ -311,8 +312,8 @@ __device__ __forceinline__ void move_terms(const SJSysDev &S, const double *cfg,
       ys[p] = s / A[p * n + p];
     }
   }
-  // rd = sum_k phi_k(x') y_k and its gradient: each basis function once, with
-  // its weight sum_k c_km y_k
+  // rd = sum_k phi_k(x') y_k and its gradient: the orbitals' sums over the
+  // basis first, each function evaluated once
   double rd = 0.0, gd[3] = {0.0, 0.0, 0.0};
   double phi[kMlpMaxSpin], g0[kMlpMaxSpin], g1[kMlpMaxSpin], g2[kMlpMaxSpin];
 #pragma unroll

@@ -34,7 +34,7 @@ enum SJAccColumn : int {
   kSJSumO = 9,  // then sum O [np], sum O E [np], sum O O^T [np (np + 1) / 2]
 };
 // Column layout of a system with np parameters (5, or 6 with the exponent
-// scale): only the system's own parameters take columns, in HBM and in LDS.
+// scale): only the system's own parameters take columns.
 __host__ __device__ constexpr int sj_sum_oe(int np) { return kSJSumO + np; }
 __host__ __device__ constexpr int sj_sum_oo(int np) { return kSJSumO + 2 * np; }  // upper triangle, row-major
 __host__ __device__ constexpr int sj_columns(int np) { return kSJSumO + 2 * np + np * (np + 1) / 2; }
@@ -76,7 +76,6 @@ struct SJSysDev {
   uint64_t draw_base;   // draw index of the first move after the stream origin
   uint64_t move_base;   // moves made before the stream origin (LU refresh phase)
   uint32_t sys_index;   // mixed into the Philox key
-  uint32_t lds_per_walker;  // bytes
   // diffusion Monte Carlo (null outside DMC): [4][W] = weight, local
   // energy at the current configuration, and the last step's w E_old and
   // w_old; the reference energy is a device scalar

@@ -475,7 +475,7 @@ __device__ __forceinline__ void refresh_walker(const SJSysDev &S, const SJTab &t
 // evaluated every basis function twice, and 18 three times).
 constexpr int kSJLanesNMax = 10;
 
-// The pieces of the local energy the operator terms need (sub-lane 0).
+// The pieces of the local energy the operator terms need (on every lane).
 struct SJParts {
   double kin;  // sum_i lap_i psi / psi
   double vee;  // sum_{i<j} 1/r_ij
@@ -951,8 +951,8 @@ __device__ __forceinline__ void sj_tile(const SJArgs &a, const SJTile tile, unsi
   // A partial tile's empty slots start from its first walker: with every
   // electron at the origin their local energy would never be in the fast roots'
   // range, and the wave would evaluate it twice (two electrons in 64 functions,
-  // one walker: a sampled sweep at 16 lanes took 39 us instead of 34).  Nothing of theirs is
-  // written back.
+  // one walker: a sampled sweep at 16 lanes took 39 us instead of 34).  Nothing
+  // of theirs is written back.
   const double *pin = dmc_step ? S.dmc_pos_in : S.pos;
   const T *Bg = (const T *)(dmc_step ? S.dmc_B_in : S.B);
   for (int e = lane; e < 3 * N * nslots; e += 64) {

@@ -7,9 +7,9 @@
 //
 // tau_tile_kernel (series that fit a workgroup's LDS, from 2,048 walkers on): a
 // workgroup takes 16 walkers, their series side by side in LDS; a lane takes
-// one walker and 8 neighbouring lags, whose partners it slides through
-// registers (two LDS reads for 8 products), and the lags are taken in passes
-// of 8 per lane group, ending when every walker's sum has met its first
+// one walker and 4 neighbouring lags, whose partners it slides through
+// registers (two LDS reads for 4 products).  32 such lane groups make a pass of
+// 128 lags, and the passes end when every walker's sum has met its first
 // negative rho.  Every sum is the reference's sequential fold on one lane.
 // tau_corr_kernel (the rest): one 256-thread workgroup per walker, a lag
 // per thread, all lags.  Compiled with -ffp-contract=off, both results equal
@@ -40,37 +40,37 @@ constexpr int kTauTileSamples = 1000;  // 16 of them, and a pass's lags, within 
 // slow walker does not hold many others' lanes, and series up to 1,000 samples
 // fit the LDS.
 constexpr int kTileWalkers = 16, kTileStride = 17, kTilePad = 8;
+constexpr int kGroups = 32, kLags = 4;
 
-__host__ __device__ constexpr size_t tau_tile_lds(int n, int lags_per_pass) {
-  return sizeof(double) * ((size_t)(n + kTilePad) * kTileStride + (size_t)(lags_per_pass + 1) * kTileWalkers);
+constexpr size_t tau_tile_lds(int n) {
+  return sizeof(double) * ((size_t)(n + kTilePad) * kTileStride + (size_t)(kGroups * kLags + 1) * kTileWalkers);
 }
 
-template <int GROUPS, int LAGS>
-__global__ void __launch_bounds__(GROUPS * kTileWalkers) tau_tile_kernel(const double *trace_e, int W, size_t cap,
-                                                                         size_t first, int n, double *tau_out) {
+__global__ void __launch_bounds__(kGroups * kTileWalkers) tau_tile_kernel(const double *trace_e, int W, size_t cap,
+                                                                          size_t first, int n, double *tau_out) {
   extern __shared__ double lds[];
   double *y = lds;                                            // [n + pad][stride]
   double *corr = y + (size_t)(n + kTilePad) * kTileStride;    // [lags of a pass][walker]
-  double *stat = corr + GROUPS * LAGS * kTileWalkers;    // mean, then 0 / 1: the walker's sum is complete
-  constexpr int kThreads = GROUPS * kTileWalkers, kPass = GROUPS * LAGS;
+  double *stat = corr + kGroups * kLags * kTileWalkers;       // the walkers' means, then their variances
+  constexpr int kThreads = kGroups * kTileWalkers, kPass = kGroups * kLags;
   const int tid = threadIdx.x, wl = tid % kTileWalkers, g = tid / kTileWalkers;
   const int w0 = blockIdx.x * kTileWalkers;
   const int nw = min(kTileWalkers, W - w0);
-  // GROUPS consecutive samples of a walker per lane group, eight loads of a
+  // kGroups consecutive samples of a walker per lane group, eight loads of a
   // lane in flight; absent walkers of the last workgroup repeat the first
   {
-    const int r = tid / GROUPS, t0 = tid % GROUPS;
+    const int r = tid / kGroups, t0 = tid % kGroups;
     const double *src = trace_e + (size_t)(w0 + (r < nw ? r : 0)) * cap + first;
     double *o = y + r;
     int t = t0;
-    for (; t + 7 * GROUPS < n; t += 8 * GROUPS) {
+    for (; t + 7 * kGroups < n; t += 8 * kGroups) {
       double v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = src[t + u * GROUPS];
+      for (int u = 0; u < 8; ++u) v[u] = src[t + u * kGroups];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) o[(t + u * GROUPS) * kTileStride] = v[u];
+      for (int u = 0; u < 8; ++u) o[(t + u * kGroups) * kTileStride] = v[u];
     }
-    for (; t < n; t += GROUPS) o[t * kTileStride] = src[t];
+    for (; t < n; t += kGroups) o[t * kTileStride] = src[t];
   }
   for (int e = tid; e < kTilePad * kTileStride; e += kThreads) y[n * kTileStride + e] = 0.0;
   __syncthreads();
@@ -102,7 +102,7 @@ __global__ void __launch_bounds__(GROUPS * kTileWalkers) tau_tile_kernel(const d
   __syncthreads();
   {
     const double mean = stat[wl];
-    for (int t = g; t < n; t += GROUPS) y[t * kTileStride + wl] = y[t * kTileStride + wl] - mean;
+    for (int t = g; t < n; t += kGroups) y[t * kTileStride + wl] = y[t * kTileStride + wl] - mean;
   }
   __syncthreads();
   if (tid < kTileWalkers) stat[tid] = fold([](double d) { return d * d; }) / (double)(n - 1);
@@ -113,44 +113,44 @@ __global__ void __launch_bounds__(GROUPS * kTileWalkers) tau_tile_kernel(const d
   double tau = 1.0;     // threads 0..15: the walker's sum
   bool done = tid >= kTileWalkers;
   for (int i0 = 0; i0 < max_i; i0 += kPass) {
-    // lags b + 1 .. b + LAGS of this lane; rows past n are never used
-    const int b = i0 + g * LAGS;
-    double c[LAGS], v[LAGS];
+    // lags b + 1 .. b + kLags of this lane; rows past n are never used
+    const int b = i0 + g * kLags;
+    double c[kLags], v[kLags];
 #pragma unroll
-    for (int j = 0; j < LAGS; ++j) c[j] = 0.0;
-    const int full = n - (b + LAGS);  // t below it: all LAGS products
+    for (int j = 0; j < kLags; ++j) c[j] = 0.0;
+    const int full = n - (b + kLags);  // t below it: all kLags products
     int t = 0;
     if (full >= 8) {
 #pragma unroll
-      for (int j = 0; j < LAGS; ++j) v[j] = yw[(b + 1 + j) * kTileStride];
+      for (int j = 0; j < kLags; ++j) v[j] = yw[(b + 1 + j) * kTileStride];
       for (; t + 8 <= full; t += 8) {
         double a[8], nv[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
           a[u] = yw[(t + u) * kTileStride];
-          nv[u] = yw[(t + u + b + 1 + LAGS) * kTileStride];
+          nv[u] = yw[(t + u + b + 1 + kLags) * kTileStride];
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
 #pragma unroll
-          for (int j = 0; j < LAGS; ++j) {
-            const double yj = u + j < LAGS ? v[u + j < LAGS ? u + j : 0] : nv[u + j < LAGS ? 0 : u + j - LAGS];
+          for (int j = 0; j < kLags; ++j) {
+            const double yj = u + j < kLags ? v[u + j < kLags ? u + j : 0] : nv[u + j < kLags ? 0 : u + j - kLags];
             c[j] += a[u] * yj;
           }
         }
 #pragma unroll
-        for (int j = 0; j < LAGS; ++j) v[j] = nv[8 - LAGS + j];
+        for (int j = 0; j < kLags; ++j) v[j] = nv[8 - kLags + j];
       }
     }
     for (; t < n - (b + 1); ++t) {
       const double a = yw[t * kTileStride];
 #pragma unroll
-      for (int j = 0; j < LAGS; ++j)
+      for (int j = 0; j < kLags; ++j)
         if (t + b + 1 + j < n) c[j] += a * yw[(t + b + 1 + j) * kTileStride];
     }
 #pragma unroll
-    for (int j = 0; j < LAGS; ++j)
-      if (b + 1 + j <= max_i) corr[(g * LAGS + j) * kTileWalkers + wl] = c[j] / (var * (double)(n - (b + 1 + j)));
+    for (int j = 0; j < kLags; ++j)
+      if (b + 1 + j <= max_i) corr[(g * kLags + j) * kTileWalkers + wl] = c[j] / (var * (double)(n - (b + 1 + j)));
     __syncthreads();
     if (!done) {
       // the terms in lag order up to the first negative one (its factor f
@@ -228,18 +228,17 @@ __global__ void __launch_bounds__(kTauThreads) tau_corr_kernel(const double *tra
   }
 }
 
-template <int GROUPS, int LAGS>
 hipError_t launch_tile(const double *trace_e, int W, size_t cap, size_t first, int n, double *tau_out,
                        hipStream_t stream) {
-  const size_t bytes = tau_tile_lds(n, GROUPS * LAGS);
+  const size_t bytes = tau_tile_lds(n);
   if (bytes > 65536) {
     // more than the default 64 KiB of dynamic LDS needs an opt-in per kernel
-    const hipError_t e = hipFuncSetAttribute((const void *)(tau_tile_kernel<GROUPS, LAGS>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    const hipError_t e = hipFuncSetAttribute((const void *)tau_tile_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)bytes);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((tau_tile_kernel<GROUPS, LAGS>), dim3((unsigned)((W + kTileWalkers - 1) / kTileWalkers)),
-                     dim3(GROUPS * kTileWalkers), bytes, stream, trace_e, W, cap, first, n, tau_out);
+  hipLaunchKernelGGL(tau_tile_kernel, dim3((unsigned)((W + kTileWalkers - 1) / kTileWalkers)),
+                     dim3(kGroups * kTileWalkers), bytes, stream, trace_e, W, cap, first, n, tau_out);
   return hipGetLastError();
 }
 
@@ -252,7 +251,7 @@ hipError_t launch_tau_corr(const double *trace_e, int W, size_t cap, size_t firs
   // lag-parallel fold is the shorter one (500 walkers x 400 samples: 52 against
   // 60 us a call; 4,096: 149 against 89).
   if (W >= kTauTileMinWalkers && n <= kTauTileSamples)
-    return launch_tile<32, 4>(trace_e, W, cap, first, n, tau_out, stream);
+    return launch_tile(trace_e, W, cap, first, n, tau_out, stream);
   if (n <= kTauLdsSamples)
     hipLaunchKernelGGL(tau_corr_kernel<true>, dim3(W), dim3(kTauThreads), sizeof(double) * n, stream, trace_e, cap,
                        first, n, tau_out);

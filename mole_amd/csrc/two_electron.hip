@@ -337,8 +337,9 @@ __device__ __forceinline__ void local2_cached(const Sys2 &sp, const double *x,
 // division where its outcome is beyond rounding: t = a - u b is formed with
 // one rounding, and with |t| > 2^-50 b the quotient differs from u by more
 // than two units in u's last place (u < 1), so its rounding lies on the same
-// side of u.  Close calls, NaN, infinities and b < 2^-900 are not `sure`: the
-// caller then divides (accept_div), so every decision is the division's.
+// side of u.  Close calls, NaN, an infinite b and b < 2^-900 are not `sure`: the
+// caller then divides (accept_div), so every decision is the division's (an
+// infinite a over a finite b accepts either way).
 __device__ __forceinline__ bool accept_fast(double a, double b, double u, bool &sure) {
   const double t = fma(-u, b, a);
   sure = sure && fabs(t) > b * 0x1p-50 && b > 0x1p-900;
@@ -347,8 +348,7 @@ __device__ __forceinline__ bool accept_fast(double a, double b, double u, bool &
 __device__ __forceinline__ bool accept_div(double a, double b, double u) { return min_one(a / b) > u; }
 
 constexpr int kQuadXor1 = 0xB1;  // quad_perm [1, 0, 3, 2]
-constexpr int kQuadXor2 = 0x4E;  // quad_perm [2, 3, 0, 1]
-constexpr int kQuadLane0 = 0x00, kQuadLane1 = 0x55, kQuadLane2 = 0xAA, kQuadLane3 = 0xFF;
+constexpr int kQuadLane0 = 0x00, kQuadLane1 = 0x55, kQuadLane2 = 0xAA;
 
 // v of the lane the quad permutation CTRL names (two 32-bit DPP moves)
 template <int CTRL>
@@ -901,9 +901,9 @@ void launch_ws(const Sweep2Args &a, hipStream_t stream) {
 
 template <int KIND, int NNUC>
 void launch_spec(const Sweep2Args &a, int variant, int bt, int cus, hipStream_t stream) {
-  // us per sweep on 256 CUs, helium / H2 (start: four waves per 64 walkers,
+  // us per sweep on 256 CUs, helium / H2 (single: the pair kernel's predecessor,
   // one lane per walker in the chain wave):
-  //   W         quad, 32/wg   pair, 64/wg   pair, T = 2   wide          start
+  //   W         quad, 32/wg   pair, 64/wg   pair, T = 2   wide          single
   //   8,192     0.60 / 0.70   0.69 / 0.85   0.75 / 0.87   1.37 / 1.87   0.80 / 1.24
   //   16,384    0.89 / 1.11   0.71 / 0.86   0.77 / 0.87   1.38 / 1.90   0.83 / 1.26
   //   32,768    1.43 / 2.02   1.08 / 1.71   1.12 / 1.40   1.39 / 1.90   1.59 / 2.45
