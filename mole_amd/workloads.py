@@ -250,7 +250,7 @@ def learned(Z=10, walkers=65536, n_configs=2_000_000, collect_every=5, equil=100
         obj = mlp.train(ctx, train_steps, batch=batch, lr=lr, seed=seed + 10, objective=objective)
         t_train = time.perf_counter() - t0
     n_data = mlp.data_size()
-    box_lanes = autotune.tune([sj], lambda s: walkers, candidates=(4, 8, 16), sweeps=2, precision=precision,
+    box_lanes = autotune.tune([sj], lambda s: walkers, candidates=(2, 4, 8, 16), sweeps=2, precision=precision,
                               lu_period=lu_period)[0]
 
     def measure(proposal, step):
