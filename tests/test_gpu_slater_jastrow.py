@@ -74,8 +74,8 @@ def test_mixed_precision_parity_with_oracle(Z):
     assert np.max(rel) <= E_TOL
 
 
-@pytest.mark.parametrize("Z,lanes,steps", [(3, 4, 30), (4, 4, 12), (5, 4, 10), (6, 4, 10), (7, 4, 8), (8, 8, 8),
-                                           (9, 8, 8), (10, 8, 10)])
+@pytest.mark.parametrize("Z,lanes,steps", [(3, 2, 30), (4, 2, 12), (5, 2, 10), (6, 4, 10), (7, 4, 8), (8, 4, 8),
+                                           (9, 4, 8), (10, 4, 10)])
 def test_mixed_precision_parity_at_workload_width(Z, lanes, steps):
     # the atoms workload's width (65,536 walkers, LU refresh every 64 moves)
     # with the lanes per walker its autotuning picks: every accept decision,
@@ -104,20 +104,16 @@ def tile_footprint(system, lanes):
 
 def test_heterogeneous_batch_at_workload_shape():
     # the heterogeneous workload's launches: 256 systems of 2..40 electrons,
-    # 2^20 walkers split in proportion to N, mixed precision.  The tiles are
-    # grouped into LDS footprint classes (one up to an eighth of a CU's 160 KiB,
-    # 4 KiB steps above it), one launch per class with blockIdx.x restarting at 0
-    # in each, longest tiles first within a class.  The lanes its autotuning
-    # picked keep every tile in the first class, so the systems from 21 electrons
-    # on take half of those here.  The system with the fewest electrons, the one
-    # with the largest tile footprint and the largest system of a third class
-    # against their own oracle runs (systems are independent streams)
+    # 2^20 walkers split in proportion to N, the lanes its autotuning picked,
+    # mixed precision.  The tiles are grouped into LDS footprint classes (one up
+    # to an eighth of a CU's 160 KiB, 4 KiB steps above it), one launch per class
+    # with blockIdx.x restarting at 0 in each, longest tiles first within a class.
+    # The system with the fewest electrons, the one with the largest tile
+    # footprint and the largest system of a third class against their own oracle
+    # runs (systems are independent streams)
     from mole_amd import autotune
     from mole_amd import workloads as WL
-    lanes = {2: 4, 3: 4, 4: 4, 5: 8, 6: 8, 7: 8, 8: 8, 9: 16, 10: 8, 11: 8, 12: 16, 13: 16, 14: 16, 15: 16,
-             16: 16, 17: 16, 18: 16, 19: 32, 20: 16}
-    lanes.update({n: 16 for n in range(21, 32)})
-    lanes.update({n: 32 for n in range(32, 41)})
+    lanes = {n: 4 if n <= 4 else 8 if n <= 16 else 16 if n <= 27 else 32 for n in range(2, 41)}
     sys_list = WL.hetero_systems(256, 3)
     Ns = np.array([s.n_electrons for s in sys_list])
     W = np.maximum(1, np.floor(Ns / Ns.sum() * (1 << 20))).astype(int)
