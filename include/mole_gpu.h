@@ -535,7 +535,9 @@ mole_status mole_dmc_read_walkers(mole_ctx *ctx, uint32_t sys, double *weights, 
 mole_status mole_set_launch_config(mole_ctx *ctx, uint32_t variant, uint32_t block_threads);
 /* Slater-Jastrow: lanes of a wave that share one walker of system sys
  * (power of two, 1..64; 0 = the library's choice).  Results do not depend
- * on it; it only trades per-move parallelism against walkers per wave. */
+ * on it; it only trades per-move parallelism against walkers per wave.
+ * mole_eval takes lanes set here too; the library's choice for it follows the
+ * number of configurations given. */
 mole_status mole_set_walker_lanes(mole_ctx *ctx, uint32_t sys, uint32_t lanes);
 mole_status mole_get_walker_lanes(mole_ctx *ctx, uint32_t sys, uint32_t *lanes);
 /* Slater-Jastrow launch shape: workgroups of one sweep step over all its
